@@ -510,32 +510,140 @@ template <typename T, int PER> __global__ void __launch_bounds__(256) norm_rows_
     }
 }
 
-// BatchNorm: one thread per column over the batch rows (forward.cu:74-126 with
-// norm == 3), then act + dropout.  Consecutive threads read consecutive columns.
-template <typename T> __global__ void __launch_bounds__(256) norm_cols_kernel(RowNormArgs a) {
-    const uint32_t col = blockIdx.x * 256 + threadIdx.x;
-    if (col >= a.n) return;
+// BatchNorm (forward.cu:74-126 with norm == 3), then act + dropout: a workgroup of
+// 1024 threads per 16 columns, all batch rows.  LPR = 16 / VW lanes share a row (4
+// elements each with VEC, one otherwise), so the workgroup takes RPW = 1024 / LPR
+// rows per step and thread t the rows t / LPR, + RPW, ...  HELD: the thread's (at most
+// PER) rows stay in registers, so prenorm is read once for the mean, the variance about
+// it and the outputs; longer batches read it again for each (from L2).  Each sum runs
+// over a thread's rows, then the wave's lanes of a column (butterfly), then the 16 waves
+// in order.  Bound: address processing of the five output streams (a row is one 32-byte
+// piece of a line per tensor) below ~4K rows, HBM above.  The line segments of 64
+// columns belong to 4 workgroups, which the block order puts on one XCD.
+// 2048 x 1024 fp16: 1565 us with one thread walking a column.
+template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024) norm_cols_kernel(RowNormArgs a) {
+    constexpr uint32_t CT = 16, VW = VEC ? 4 : 1, LPR = CT / VW, RPW = 1024 / LPR;
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    typedef typename std::conditional<sizeof(T) == 2, u32x2_t, u32x4_t>::type G;   // 4 elements
+    constexpr bool HELD = PER > 0;
+    constexpr int UNR = HELD ? PER : 4;   // rows loaded before any is used
+    __shared__ float red[16][CT];
+    // workgroup w runs on XCD w % 8: consecutive tiles go to one XCD
+    uint32_t tile = blockIdx.x;
+    if ((gridDim.x & 7u) == 0) tile = (tile & 7u) * (gridDim.x >> 3) + (tile >> 3);
     const uint32_t n = a.n, m = a.m;
-    float s = 0.0f;
-    for (uint32_t r = 0; r < m; ++r) s += to_f32(ldv<T>(a.prenorm, (uint64_t)r * n + col));
-    const float mean = s / (float)m;
-    float ss = 0.0f;
-    for (uint32_t r = 0; r < m; ++r) {
-        const float v = to_f32(ldv<T>(a.prenorm, (uint64_t)r * n + col)) - mean;
-        ss = fmaf(v, v, ss);
+    const uint32_t lr = threadIdx.x % LPR, r0 = threadIdx.x / LPR;
+    const uint32_t c0 = tile * CT + lr * VW;
+    const bool cin = c0 < n;              // VEC: n % VW == 0, so whole groups
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    T zr[UNR][VW];
+
+    auto load = [&](uint32_t r, T (&v)[VW]) {
+        if constexpr (VEC)
+            *reinterpret_cast<G *>(v) =
+                *reinterpret_cast<const G *>(reinterpret_cast<const T *>(a.prenorm) + (uint64_t)r * n + c0);
+        else
+            v[0] = ldv<T>(a.prenorm, (uint64_t)r * n + c0);
+    };
+    // f(row, its VW elements) over the thread's rows
+    auto rows = [&](bool first, auto f) {
+        if constexpr (HELD) {
+            if (first) {
+#pragma unroll
+                for (int i = 0; i < UNR; ++i)
+                    if (cin && r0 + i * RPW < m) load(r0 + i * RPW, zr[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < UNR; ++i)
+                if (cin && r0 + i * RPW < m) f(r0 + i * RPW, zr[i]);
+        } else {
+            if (!cin) return;
+            for (uint32_t rb = r0; rb < m; rb += UNR * RPW) {
+#pragma unroll
+                for (int i = 0; i < UNR; ++i)
+                    if (rb + i * RPW < m) load(rb + i * RPW, zr[i]);
+#pragma unroll
+                for (int i = 0; i < UNR; ++i)
+                    if (rb + i * RPW < m) f(rb + i * RPW, zr[i]);
+            }
+        }
+    };
+    // sum of s over the column's threads; s becomes it in every one of them
+    auto column_sum = [&](float (&s)[VW]) {
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e)
+#pragma unroll
+            for (uint32_t o = 32; o >= LPR; o >>= 1) s[e] += __shfl_xor(s[e], o, 64);
+        __syncthreads();
+        if (lane < LPR) {
+#pragma unroll
+            for (uint32_t e = 0; e < VW; ++e) red[wave][lr * VW + e] = s[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) {
+            float t = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 16; ++w) t += red[w][lr * VW + e];
+            s[e] = t;
+        }
+    };
+
+    float mean[VW] = {}, rstd[VW] = {};
+    rows(true, [&](uint32_t, const T (&v)[VW]) {
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) mean[e] += to_f32(v[e]);
+    });
+    column_sum(mean);
+#pragma unroll
+    for (uint32_t e = 0; e < VW; ++e) mean[e] /= (float)m;
+    rows(false, [&](uint32_t, const T (&v)[VW]) {
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) {
+            const float d = to_f32(v[e]) - mean[e];
+            rstd[e] = fmaf(d, d, rstd[e]);
+        }
+    });
+    column_sum(rstd);
+    if (!cin) return;
+    float g[VW], bias[VW];
+#pragma unroll
+    for (uint32_t e = 0; e < VW; ++e) {
+        rstd[e] = 1.0f / sqrtf(rstd[e] / (float)m + 1e-6f);
+        if (r0 == 0) stv<T>(a.norm_rstd, c0 + e, from_f32<T>(rstd[e]));
+        g[e] = to_f32(ldv<T>(a.norm_w, c0 + e));
+        bias[e] = to_f32(ldv<T>(a.norm_b, c0 + e));
     }
-    const float var = ss / (float)m + 1e-6f;
-    const float rstd32 = 1.0f / sqrtf(var);
-    stv<T>(a.norm_rstd, col, from_f32<T>(rstd32));
-    const float g = to_f32(ldv<T>(a.norm_w, col)), b = to_f32(ldv<T>(a.norm_b, col));
-    for (uint32_t r = 0; r < m; ++r) {
-        const uint64_t idx = (uint64_t)r * n + col;
-        const float v = to_f32(ldv<T>(a.prenorm, idx)) - mean;
-        stv<T>(a.centered, idx, from_f32<T>(v));
-        const T pre = from_f32<T>(fmaf(v * rstd32, g, b));
-        stv<T>(a.preact, idx, pre);
-        act_dropout<T>(a, idx, r, col, pre);
-    }
+    const float scale = a.use_dropout ? 1.0f / (1.0f - a.p) : 1.0f;
+    rows(false, [&](uint32_t r, const T (&v)[VW]) {
+        T cen[VW], pre[VW], pd[VW], mk[VW], ot[VW];
+        const uint32_t rk = dropout_rowkey(r, a.seed + r * 7u);
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) {
+            const float d = to_f32(v[e]) - mean[e];
+            cen[e] = from_f32<T>(d);
+            pre[e] = from_f32<T>(fmaf(d * rstd[e], g[e], bias[e]));
+            const float act = activation<T>(a.act, to_f32(pre[e]), a.leaky);
+            pd[e] = ot[e] = from_f32<T>(act);
+            if (a.use_dropout) {
+                const bool keep = (uint64_t)dropout_bits((c0 + e) * kDropColMul, rk) >= a.keep_min;
+                mk[e] = keep ? from_f32<T>(scale) : (T)0;
+                ot[e] = keep ? from_f32<T>(act * scale) : (T)0;
+            }
+        }
+        const uint64_t idx = (uint64_t)r * n + c0;
+        auto put = [&](void *p, const T (&x)[VW]) {
+            if constexpr (VEC)
+                *reinterpret_cast<G *>(reinterpret_cast<T *>(p) + idx) = *reinterpret_cast<const G *>(x);
+            else
+                stv<T>(p, idx, x[0]);
+        };
+        put(a.centered, cen);
+        put(a.preact, pre);
+        put(a.predrop, pd);
+        put(a.out, ot);
+        if (a.use_dropout) put(a.mask, mk);
+    });
 }
 
 static bool a16p(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -579,15 +687,38 @@ template <typename T> static void launch_norm_rows(const RowNormArgs &a, hipStre
         hipLaunchKernelGGL(norm_rows_kernel<T>, g, b, 0, s, a);
 }
 
+// BatchNorm: 4-element groups where every row of every tensor starts on one; the batch
+// in registers where it fits.
+template <typename T> static void launch_norm_cols(const RowNormArgs &a, hipStream_t s) {
+    constexpr uint32_t RPW_V = 256, RPW_1 = 64;   // rows per step
+    constexpr uintptr_t GB = 4 * sizeof(T) - 1;
+    auto ga = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & GB) == 0; };
+    const bool vec = a.n % 4 == 0 && ga(a.prenorm) && ga(a.centered) && ga(a.preact) && ga(a.predrop) && ga(a.out) &&
+                     (!a.use_dropout || ga(a.mask));
+    const dim3 g(cdiv(a.n, 16)), b(1024);
+    if (vec && a.m <= 2 * RPW_V)
+        hipLaunchKernelGGL((norm_cols_kernel<T, true, 2>), g, b, 0, s, a);
+    else if (vec && a.m <= 8 * RPW_V)
+        hipLaunchKernelGGL((norm_cols_kernel<T, true, 8>), g, b, 0, s, a);
+    else if (vec)
+        hipLaunchKernelGGL((norm_cols_kernel<T, true, 0>), g, b, 0, s, a);
+    else if (a.m <= 8 * RPW_1)
+        hipLaunchKernelGGL((norm_cols_kernel<T, false, 8>), g, b, 0, s, a);
+    else if (a.m <= 32 * RPW_1)
+        hipLaunchKernelGGL((norm_cols_kernel<T, false, 32>), g, b, 0, s, a);
+    else
+        hipLaunchKernelGGL((norm_cols_kernel<T, false, 0>), g, b, 0, s, a);
+}
+
 hipError_t launch_norm_act(const RowNormArgs &a0, hipStream_t s) {
     if (a0.m == 0 || a0.n == 0) return hipSuccess;
     RowNormArgs a = a0;
     a.keep_min = dropout_keep_min(a.p);
     if (a.norm == 3) {
         if (a.dtype == 1)
-            hipLaunchKernelGGL(norm_cols_kernel<half_t>, dim3(cdiv(a.n, 256)), dim3(256), 0, s, a);
+            launch_norm_cols<half_t>(a, s);
         else
-            hipLaunchKernelGGL(norm_cols_kernel<float>, dim3(cdiv(a.n, 256)), dim3(256), 0, s, a);
+            launch_norm_cols<float>(a, s);
     } else if (a.dtype == 1) {
         launch_norm_rows<half_t>(a, s);
     } else {
