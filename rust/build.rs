@@ -25,7 +25,10 @@ fn main() {
             repo.join("soklyn_amd")
         }
     };
-    for src in ["abi.hip", "gemm.hip", "elementwise.hip", "gemm.h", "gemm_dma.h", "device_math.h"] {
+    for src in [
+        "abi.hip", "gemm.hip", "gemm_wave.hip", "elementwise.hip", "epilogue.h", "gemm.h", "gemm_dma.h", "gemm_wave.h",
+        "device_math.h",
+    ] {
         println!("cargo:rerun-if-changed={}", repo.join("soklyn_amd/csrc").join(src).display());
     }
     println!("cargo:rerun-if-changed={}", repo.join("include/soklyn_hip.h").display());

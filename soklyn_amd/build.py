@@ -24,7 +24,7 @@ HOST_LIB = os.path.join(HOST, "libsoklyn_host.so")
 HOST_TOOL = os.path.join(HOST, "soklyn_tool")
 # the host API restates f32 expressions in the reference's evaluation order: no contraction
 GXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wextra", "-I", INCLUDE, "-I", HOST]
-SOURCES = ["gemm.hip", "elementwise.hip", "abi.hip"]
+SOURCES = ["gemm.hip", "gemm_wave.hip", "elementwise.hip", "abi.hip"]
 ARCH = os.environ.get("SOKLYN_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [

@@ -285,10 +285,14 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //    output wastes at most half of its grid and there are at least 192 tiles,
 //    counting the split-K slices a dW with fewer tiles than CUs is given (their
 //    fp32 partial sums, in the workspace, are reduced by the optimiser kernel).
-//  * the register-staged kernels otherwise (fp32; small or skinny fp16), with
-//    the same split-K for small dW grids.
+//  * the K-splitting kernel on small tiles (gemm_wave.h), for outputs that would leave
+//    those tiles' GPU mostly idle and for at most 16 columns: operands as stored, no
+//    workspace;
+//  * the register-staged kernels otherwise (large fp32; small fp16 with little k to
+//    reduce), with the same split-K for small dW grids.
 struct GemmPlan {
-    bool skinny;               // N <= 16: the streaming kernels (forward, dW partials)
+    bool skinny;               // N <= 16: the streaming kernels of dW partials
+    uint32_t wave;             // K-splitting kernel: its tile edge (0: another kernel)
     bool dma;
     bool pad_a, pad_b;
     uint32_t tile;             // direct-to-LDS output tile edge (128 or 256); 128: fp32 dW on 128x128 tiles
@@ -387,7 +391,26 @@ uint32_t dma_tile(Op op, uint32_t Mp, uint32_t Np, uint32_t splits, uint32_t *ba
     return 256u;
 }
 
-GemmPlan plan_gemm(const GemmLaunch &g) {
+// Estimated time (us) of the register-staged kernels, from the measurements behind
+// gemm_wave_tile: a 128x128 fp16 tile takes ~1 us per 64 k whatever the grid, 4 us when
+// its rows are not 16-byte aligned (gathered element by element), and a second tile per
+// CU hides part of it (4096 x 1024, K 1024: 25 us; 512 x 2048, K 2048: 36; 2000 x 1531,
+// K 777: 66).  fp32 grids of at least 192 tiles of 128x128 (160 for a dW) run them at the
+// rate of the K-splitting kernel or above (4096 x 1024, K 1024: dX 70 against 73 us);
+// smaller ones never do.
+double staged_us(const GemmLaunch &g) {
+    const double tiles = (double)((g.M + 127) / 128) * ((g.N + 127) / 128);
+    if (g.dtype == SKL_F32) return tiles >= (g.op == Op::DwOpt ? 160 : 192) ? 0.0 : 1e30;
+    const uint32_t a_ext = g.a_kcontig ? g.K : g.M, b_ext = g.b_kcontig ? g.K : g.N;
+    const bool vec = g.lda % 8 == 0 && g.ldb % 8 == 0 && a_ext % 8 == 0 && b_ext % 8 == 0 && aligned16(g.A) &&
+                     aligned16(g.B);
+    const double kt = (double)((g.K + 63) / 64), u = tiles / 256.0;
+    return vec ? 10.0 + kt * (u > 1.25 ? 0.8 * u : 1.0) : 15.0 + kt * (u > 1.0 ? 4.0 * u : 4.0);
+}
+
+// in_place: the output overlaps an operand (a caller's dx over d_prenorm).  The K-splitting
+// kernel's many small tiles would overwrite rows that others have yet to read.
+GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
     GemmPlan p{};
     p.tile = 256;
     p.splits = 1;
@@ -395,14 +418,22 @@ GemmPlan plan_gemm(const GemmLaunch &g) {
     p.Np = g.N;
     p.Kp = g.K;
     const bool dw = g.op == Op::DwOpt;
-    // skinny outputs: a stream over X beats any MFMA tile that is >90% padding
-    if (g.N <= 16 && g.M && g.K && ((g.op == Op::Fwd && skinny_fwd_ok(g)) || (dw && g.b32 && !g.a_kcontig))) {
-        p.skinny = true;
-        if (dw) {
+    double wave_us = 0.0;
+    const uint32_t wave = !in_place && gemm_wave_ok(g) ? gemm_wave_tile(g, &wave_us) : 0;
+    // skinny outputs: any larger tile is >90% padding.  The dW of a long batch streams X
+    // in batch slices instead (2048 x 10 fp16: 10 against 20 us at 4096 rows, 40 against
+    // 27 us at 16384).
+    if (g.N <= 16 && g.M && g.K) {
+        if (dw && g.b32 && !g.a_kcontig && (!wave || g.K > 8192)) {
+            p.skinny = true;
             p.splits = skinny_dw_slices(g.K, g.M);
             p.part_bytes = (size_t)p.splits * g.M * 16 * sizeof(float);
+            return p;
         }
-        return p;
+        if (wave) {
+            p.wave = wave;
+            return p;
+        }
     }
     if (g.dtype == SKL_F16 && gemm_dma_enabled() && g.M && g.N && g.K) {
         const uint32_t Mp = round_up(g.M, 256), Np = round_up(g.N, 256), Kp = round_up(g.K, 128);
@@ -439,6 +470,11 @@ GemmPlan plan_gemm(const GemmLaunch &g) {
             return p;
         }
     }
+    // grids that leave those tiles' GPU mostly idle: the K-splitting kernel
+    if (wave && wave_us < staged_us(g)) {
+        p.wave = wave;
+        return p;
+    }
     // register-staged kernels; split-K for small dW grids
     if (dw) {
         uint32_t tiles = gemm_tiles(g.dtype, g.M, g.N);
@@ -465,7 +501,7 @@ GemmPlan plan_gemm(const GemmLaunch &g) {
     return p;
 }
 
-enum class GemmKind { Dma, Staged, SkinnyFwd, SkinnyDw };
+enum class GemmKind { Dma, Staged, Wave, SkinnyDw };
 
 // One GEMM launch; when skl_ctx_time_next_gemm armed a pair of events, the GEMM
 // kernel's own dispatch records them (no marker packets in the stream).
@@ -478,7 +514,7 @@ hipError_t timed_gemm(skl_ctx *ctx, const GemmLaunch &g0, GemmKind kind, float *
     switch (kind) {
     case GemmKind::Dma: return launch_gemm_dma(g, ctx->stream);
     case GemmKind::Staged: return launch_gemm(g, ctx->stream);
-    case GemmKind::SkinnyFwd: return launch_skinny_fwd(g, ctx->stream);
+    case GemmKind::Wave: return launch_gemm_wave(g, ctx->stream);
     case GemmKind::SkinnyDw: return launch_skinny_dw(g, partials, slices, ctx->stream);
     }
     return hipSuccess;
@@ -498,8 +534,19 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
     char *wa = ws, *wb = ws + p.a_bytes, *wpart = ws + p.a_bytes + p.b_bytes;
     const OptEpi oe = g.opt;
     const uint32_t M = g.M, N = g.N;
+    if (p.wave) {
+        g.tile = p.wave;
+        if (vec && g.op == Op::DwOpt) {
+            // the bias / norm-parameter update rides in the launch (columns per workgroup
+            // for 256 threads; the launcher scales them to its own)
+            g.opt.vec = *vec;
+            g.opt.vec.cpb = vec_opt_cpb(vec->splits);
+            g.opt.vec_blocks = 1;
+            if (vec_done) *vec_done = true;
+        }
+        return hip_status(timed_gemm(ctx, g, GemmKind::Wave));
+    }
     if (p.skinny) {
-        if (g.op == Op::Fwd) return hip_status(timed_gemm(ctx, g, GemmKind::SkinnyFwd));
         SKL_TRY(timed_gemm(ctx, g, GemmKind::SkinnyDw, reinterpret_cast<float *>(wpart), p.splits));
         DwReduceArgs d{};
         d.dtype = g.dtype;
@@ -1399,7 +1446,10 @@ int32_t skl_dense_input_grad(skl_ctx *ctx, const skl_dense_desc *b, uint32_t bat
     g.st.out = dx;
     g.st.split_stride = 0;
     g.st.ldc = b->inputs;
-    const GemmPlan plan = plan_gemm(g);
+    const size_t esz = f16 ? 2 : 4, dx_sz = (size_t)batch * b->inputs * sizeof(float);
+    const bool in_place = overlaps(dx, dx_sz, g.A, (size_t)batch * b->outputs * esz) ||
+                          overlaps(dx, dx_sz, g.B, (size_t)b->inputs * b->outputs * esz);
+    const GemmPlan plan = plan_gemm(g, in_place);
     if ((r = ensure_ws(ctx, plan.bytes()))) return r;
     if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws), false, nullptr, nullptr, f16 ? KEEP_A : 0)))
         return r;
@@ -1409,11 +1459,10 @@ int32_t skl_dense_input_grad(skl_ctx *ctx, const skl_dense_desc *b, uint32_t bat
     // overlaps a buffer they were summed from
     ColSums &c = ctx->cs;
     if (c.valid && c.call + 1 >= ctx->calls) {
-        const size_t dx_bytes = (size_t)batch * b->inputs * sizeof(float);
         const size_t buf_bytes = (size_t)c.rows * c.n * sizeof(float);
-        const bool hit = overlaps(dx, dx_bytes, c.dp, buf_bytes) ||
+        const bool hit = overlaps(dx, dx_sz, c.dp, buf_bytes) ||
                          (c.norm != SKL_NORM_DISABLED &&
-                          (overlaps(dx, dx_bytes, c.dnw, buf_bytes) || overlaps(dx, dx_bytes, c.dnb, buf_bytes)));
+                          (overlaps(dx, dx_sz, c.dnw, buf_bytes) || overlaps(dx, dx_sz, c.dnb, buf_bytes)));
         if (hit)
             c.valid = false;
         else

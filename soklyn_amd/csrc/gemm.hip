@@ -289,252 +289,9 @@ uint32_t gemm_dma_splits(uint32_t K, uint32_t splits) {
 
 // ---- skinny outputs (N <= 16) ---------------------------------------------------------
 // The output layers of the MLP configurations have 10 and 13 columns: a 256x256
-// (or 128x128) MFMA tile would be >90% padding, and the work is a stream over X.
+// (or 128x128) MFMA tile would be >90% padding, and the dW of a long batch is a stream
+// over X.
 constexpr uint32_t SKINNY_N = 16;
-constexpr uint32_t SKINNY_LDS = 96 * 1024;
-
-// Sum of v[0..15] over the wave by recursive halving: each xor-shuffle step sends
-// half of the values a lane still holds and keeps the other half, so lane l ends
-// with column (l >> 2) & 15 summed over its 4 lanes after 8+4+2+1 shuffles, then 2
-// more finish it (17 in all, fixed order).  Returns the column sum lane l holds.
-__device__ __forceinline__ float wave_sum16(float (&v)[SKINNY_N], uint32_t lane) {
-#pragma unroll
-    for (int h = 8, m = 32; h >= 1; h >>= 1, m >>= 1) {
-        const bool up = (lane & (uint32_t)m) != 0;
-#pragma unroll
-        for (int i = 0; i < h; ++i) {
-            const float send = up ? v[i] : v[i + h];
-            const float keep = up ? v[i + h] : v[i];
-            v[i] = keep + __shfl_xor(send, m, 64);
-        }
-    }
-    float t = v[0];
-    t += __shfl_xor(t, 2, 64);
-    t += __shfl_xor(t, 1, 64);
-    return t;
-}
-
-// Forward, one wave per row: lane l takes the 8-element k chunks l, l + 64, ... of
-// the row (one 16-byte load per chunk on 16-byte aligned rows, 8 element loads
-// otherwise: a wave still covers 512 consecutive elements), and for each of the 16
-// columns one 16-byte LDS read of W^T (staged n-major, rows of Kp = K rounded up to
-// 8, zero past K and past N) feeds 8 FMAs into the lane's partial column sums.  The
-// sums are reduced over the wave, and the lane holding column n < N runs the forward
-// epilogue for it (bias, act, dropout, the three cache stores).  One workgroup per CU
-// stages W once for all of its rows.
-template <typename T, bool VECX>
-__global__ void __launch_bounds__(1024) skinny_fwd_kernel(GemmShape sh, const T *__restrict__ A,
-                                                          const T *__restrict__ B, FwdEpi ep) {
-    constexpr int CH = 8;   // k per chunk
-    __shared__ __attribute__((aligned(16))) T ws[SKINNY_LDS / sizeof(T)];
-    const uint32_t K = sh.K, N = sh.N, Kp = (K + CH - 1) / CH * CH;
-    for (uint32_t i = threadIdx.x; i < SKINNY_N * Kp; i += blockDim.x) {
-        const uint32_t n = i / Kp, k = i - n * Kp;
-        ws[i] = (n < N && k < K) ? B[(uint64_t)k * sh.ldb + n] : (T)0;
-    }
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    for (uint32_t m = blockIdx.x * waves + wave; m < sh.M; m += gridDim.x * waves) {
-        float acc[SKINNY_N];
-#pragma unroll
-        for (int n = 0; n < (int)SKINNY_N; ++n) acc[n] = 0.0f;
-        const T *x = A + (uint64_t)m * sh.lda;
-#pragma unroll 2
-        for (uint32_t k0 = lane * CH; k0 < K; k0 += 64 * CH) {
-            T xv[CH];
-            if (VECX && k0 + CH <= K) {
-                static_assert(sizeof(xv) % 16 == 0, "chunk of whole 16-byte words");
-#pragma unroll
-                for (int q = 0; q < (int)(sizeof(xv) / 16); ++q)
-                    reinterpret_cast<u32x4 *>(xv)[q] = reinterpret_cast<const u32x4 *>(x + k0)[q];
-            } else {
-#pragma unroll
-                for (int e = 0; e < CH; ++e) xv[e] = k0 + e < K ? x[k0 + e] : (T)0;
-            }
-#pragma unroll
-            for (int n = 0; n < (int)SKINNY_N; ++n) {
-                T w8[CH];
-#pragma unroll
-                for (int q = 0; q < (int)(sizeof(w8) / 16); ++q)
-                    reinterpret_cast<u32x4 *>(w8)[q] = reinterpret_cast<const u32x4 *>(ws + n * Kp + k0)[q];
-#pragma unroll
-                for (int e = 0; e < CH; ++e) acc[n] = fmaf(to_f32(xv[e]), to_f32(w8[e]), acc[n]);
-            }
-        }
-        const float z = wave_sum16(acc, lane);
-        const uint32_t n = (lane >> 2) & 15u;
-        if ((lane & 3u) == 0 && n < N) {
-            GemmShape one = sh;   // column n alone
-            one.N = n + 1;
-            EpiFwdK<T>::apply(ep, one, m, n, floatx4{z, 0.0f, 0.0f, 0.0f}, 0);
-        }
-    }
-}
-
-// The same on MFMA (fp16): a quad of 4 waves takes a block of 16 rows (one 16 x 16
-// output block, columns past N zero), wave w of the quad the k-chunks w, w + 4, ...
-// of 32 k, each a v_mfma_f32_16x16x32_f16 with lane l feeding X[row l % 16][k + 8
-// (l / 16) .. + 7] and W^T[column l % 16][same k] (LDS rows of P halves, P = 8
-// mod 128: the 16 rows of a read sit in distinct banks).  Rows that are not 16-byte
-// aligned are cut out of the two aligned 16-byte chunks covering them (funnel
-// shifts; the second chunk only when it holds a row element), k past K reads as
-// zero.  The quad's 4 partial blocks are added in wave order in LDS, and the
-// forward epilogue runs per element (lane l: rows 4 (l / 16) .. + 3 of column
-// l % 16, whose bias is loaded once).  One workgroup of 16 waves per CU stages W^T
-// once; every quad runs the same number of row-block rounds (barriers).
-constexpr uint32_t SKINNY_MFMA_P_MAX = 4104;   // LDS row pitch bound (K <= 4096): 16 rows + the sums fit 160 KB
-__device__ __forceinline__ halfx8 skinny_x8(const half_t *__restrict__ A, uint64_t rb, uint32_t k, uint32_t K,
-                                           uint64_t in_elems, bool vecx) {
-    typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
-    const uint64_t e = rb + k;
-    u32x4v v = {0, 0, 0, 0};
-    if (vecx) {
-        v = *reinterpret_cast<const u32x4v *>(A + e);
-    } else {
-        const uint64_t a0 = e & ~7ull;
-        const uint32_t sh = (uint32_t)(e - a0);   // halves past the aligned chunk
-        const u32x4v lo = *reinterpret_cast<const u32x4v *>(A + a0);
-        const u32x4v hi = (sh && a0 + 8 < in_elems) ? *reinterpret_cast<const u32x4v *>(A + a0 + 8) : u32x4v{0, 0, 0, 0};
-        const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        const uint32_t wd = sh >> 1, bits = (sh & 1u) * 16u;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const uint32_t x0 = wd == 0 ? w[d] : wd == 1 ? w[d + 1] : wd == 2 ? w[d + 2] : w[d + 3];
-            const uint32_t x1 = wd == 0 ? w[d + 1] : wd == 1 ? w[d + 2] : wd == 2 ? w[d + 3] : w[d + 4];
-            v[d] = __builtin_amdgcn_alignbit(x1, x0, bits);   // (x1:x0) >> bits
-        }
-    }
-    halfx8 h = __builtin_bit_cast(halfx8, v);
-    if (k + 8 > K) {
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i)
-            if (k + i >= K) h[i] = (_Float16)0.0f;
-    }
-    return h;
-}
-
-template <bool VECX>
-__global__ void __launch_bounds__(1024) skinny_fwd_mfma_kernel(GemmShape sh, const half_t *__restrict__ A,
-                                                               const half_t *__restrict__ B, FwdEpi ep, uint32_t P) {
-    __shared__ __attribute__((aligned(16))) half_t ws[SKINNY_N * SKINNY_MFMA_P_MAX];
-    __shared__ __attribute__((aligned(16))) float red[16][256];
-    const uint32_t K = sh.K, N = sh.N, M = sh.M;
-    const uint32_t Kc = (K + 31) / 32 * 32;
-    // W^T staging: 8 element loads in flight per thread (W is read as stored,
-    // row k of N halves)
-    for (uint32_t i0 = threadIdx.x; i0 < SKINNY_N * Kc; i0 += 8 * blockDim.x) {
-        half_t v[8];
-#pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) {
-            const uint32_t i = i0 + u * blockDim.x, k = i / SKINNY_N, n = i % SKINNY_N;
-            v[u] = (i < SKINNY_N * Kc && n < N && k < K) ? B[(uint64_t)k * sh.ldb + n] : (half_t)0;
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) {
-            const uint32_t i = i0 + u * blockDim.x, k = i / SKINNY_N, n = i % SKINNY_N;
-            if (i < SKINNY_N * Kc) ws[n * P + k] = v[u];
-        }
-    }
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, quad = wave >> 2, wq = wave & 3u;
-    const uint32_t r16 = lane & 15u, kg = lane >> 4;
-    const uint32_t nblk = (M + 15) / 16, nck = Kc / 32;
-    const typename EpiFwdK<half_t>::Col1 c1 =
-        r16 < N ? EpiFwdK<half_t>::column1(ep, r16) : typename EpiFwdK<half_t>::Col1{};
-    const uint64_t in_elems = (uint64_t)(M - 1) * sh.lda + K;   // readable elements of X
-    const half_t *wrow = ws + r16 * P + kg * 8;
-    for (uint32_t base = blockIdx.x * 4; base < nblk; base += gridDim.x * 4) {
-        const uint32_t blk = base + quad;
-        floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (blk < nblk) {   // uniform in the wave: the MFMAs below run with every lane
-            const uint32_t m = blk * 16 + r16;
-            const bool mrow = m < M;   // rows past M feed zero fragments
-            const uint64_t rb = (uint64_t)(mrow ? m : 0u) * sh.lda;
-            // 4 of the wave's k-chunks per round: their loads first, then the MFMAs
-            for (uint32_t ck0 = wq; ck0 < nck; ck0 += 16) {
-                halfx8 xa[4], wb[4];
-#pragma unroll
-                for (uint32_t u = 0; u < 4; ++u) {
-                    const uint32_t ck = ck0 + 4 * u;   // same in every lane
-                    if (ck < nck) {
-                        const uint32_t k = ck * 32 + kg * 8;
-                        xa[u] = (mrow && k < K) ? skinny_x8(A, rb, k, K, in_elems, VECX && k + 8 <= K) : halfx8{};
-                        wb[u] = *reinterpret_cast<const halfx8 *>(wrow + ck * 32);
-                    } else {
-                        xa[u] = halfx8{};
-                        wb[u] = halfx8{};
-                    }
-                }
-#pragma unroll
-                for (uint32_t u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[u], wb[u], acc, 0, 0, 0);
-            }
-        }
-        *reinterpret_cast<floatx4 *>(&red[wave][lane * 4]) = acc;
-        __syncthreads();
-        if (blk < nblk && wq == 0) {
-            const floatx4 p0 = *reinterpret_cast<const floatx4 *>(&red[quad * 4 + 0][lane * 4]);
-            const floatx4 p1 = *reinterpret_cast<const floatx4 *>(&red[quad * 4 + 1][lane * 4]);
-            const floatx4 p2 = *reinterpret_cast<const floatx4 *>(&red[quad * 4 + 2][lane * 4]);
-            const floatx4 p3 = *reinterpret_cast<const floatx4 *>(&red[quad * 4 + 3][lane * 4]);
-            const floatx4 sum = ((p0 + p1) + p2) + p3;
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) {
-                const uint32_t mo = blk * 16 + 4 * kg + i;
-                if (mo < M && r16 < N) EpiFwdK<half_t>::apply1(ep, mo, r16, sum[i], c1, 0);
-            }
-        }
-        __syncthreads();   // red is rewritten by the next round
-    }
-}
-
-static uint32_t skinny_mfma_pitch(uint32_t K) { return (K + 127) / 128 * 128 + 8; }
-
-bool skinny_fwd_ok(const GemmLaunch &g) {
-    const size_t esz = g.dtype == 1 ? 2 : 4;
-    const size_t kp = (g.K + 7) / 8 * 8;
-    return g.op == Op::Fwd && g.N <= SKINNY_N && g.a_kcontig && !g.b_kcontig && g.K > 0 &&
-           (size_t)SKINNY_N * kp * esz <= SKINNY_LDS;
-}
-
-template <typename T> static void launch_skinny_fwd_t(const GemmShape &sh, const GemmLaunch &g, hipStream_t s) {
-    const bool vecx = sh.lda % 8 == 0 && (reinterpret_cast<uintptr_t>(g.A) & 15u) == 0;
-    if constexpr (sizeof(T) == 2) {
-        const uint32_t P = skinny_mfma_pitch(sh.K);
-        // the MFMA kernel reads 16-byte chunks of X: a 16-byte aligned base
-        if (P <= SKINNY_MFMA_P_MAX && (reinterpret_cast<uintptr_t>(g.A) & 15u) == 0 && sh.M > 0) {
-            uint32_t grid = (sh.M + 63) / 64;   // 4 blocks of 16 rows per workgroup and round
-            if (grid > 256) grid = 256;
-            const half_t *A = reinterpret_cast<const half_t *>(g.A), *B = reinterpret_cast<const half_t *>(g.B);
-            if (vecx)
-                launch_timed(g, skinny_fwd_mfma_kernel<true>, dim3(grid), dim3(1024), s, sh, A, B, g.fwd, P);
-            else
-                launch_timed(g, skinny_fwd_mfma_kernel<false>, dim3(grid), dim3(1024), s, sh, A, B, g.fwd, P);
-            return;
-        }
-    }
-    uint32_t grid = (sh.M + 15) / 16;   // 16 waves per workgroup, a row per wave at a time
-    if (grid > 256) grid = 256;
-    const T *A = reinterpret_cast<const T *>(g.A), *B = reinterpret_cast<const T *>(g.B);
-    if (vecx)
-        launch_timed(g, skinny_fwd_kernel<T, true>, dim3(grid), dim3(1024), s, sh, A, B, g.fwd);
-    else
-        launch_timed(g, skinny_fwd_kernel<T, false>, dim3(grid), dim3(1024), s, sh, A, B, g.fwd);
-}
-
-hipError_t launch_skinny_fwd(const GemmLaunch &g, hipStream_t s) {
-    if (!skinny_fwd_ok(g)) return hipErrorInvalidValue;
-    GemmShape sh{};
-    sh.M = g.M;
-    sh.N = g.N;
-    sh.K = g.K;
-    sh.lda = g.lda;
-    sh.ldb = g.ldb;
-    if (g.dtype == 1)
-        launch_skinny_fwd_t<half_t>(sh, g, s);
-    else
-        launch_skinny_fwd_t<float>(sh, g, s);
-    return hipGetLastError();
-}
 
 // dW partial sums, thread per W row: thread k of workgroup (x, y) walks the batch rows
 // of slice y in order, acc[n] += X[b][k] * dP[b][n], with 64 rows of dP (fp32) at a

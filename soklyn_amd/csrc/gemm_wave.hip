@@ -1,0 +1,135 @@
+// gemm_wave.hip — launcher and tile choice of the K-splitting GEMM kernel (gemm_wave.h).
+#include "epilogue.h"
+#include "gemm_wave.h"
+#include "launch.h"
+
+namespace skl {
+
+// Output rows of every tensor start on a 4-element boundary.
+template <typename T> static bool epi_rows4(const GemmLaunch &g) {
+    auto ok = [](const void *p, size_t esz) { return (reinterpret_cast<uintptr_t>(p) & (4 * esz - 1)) == 0; };
+    switch (g.op) {
+    case Op::Fwd:
+        return g.fwd.ldc % 4 == 0 && ok(g.fwd.bias, sizeof(T)) && ok(g.fwd.z_out, sizeof(T)) &&
+               (!g.fwd.fuse_act || (ok(g.fwd.predrop, sizeof(T)) && ok(g.fwd.out, sizeof(T)) &&
+                                    (!g.fwd.use_dropout || ok(g.fwd.mask, sizeof(T)))));
+    case Op::InputGrad: return g.st.ldc % 4 == 0 && ok(g.st.out, 4);
+    case Op::DwOpt:
+        return g.opt.ldc % 4 == 0 && ok(g.opt.master, 4) && ok(g.opt.dv, 4) && ok(g.opt.dm, 4) &&
+               ok(g.opt.param, sizeof(T));
+    default: return false;
+    }
+}
+
+// Tiles: rows = columns = 16, 32 or 64, with the waves that share a workgroup's K.
+// 16 waves of 16x16 and 4 or 8 of 32x32 or 64x64 put 64-128 KB of loads in flight per CU.
+template <typename T, class Epi, bool AK, bool BK, bool REG, int MB, int W, int S, int WPE>
+static hipError_t run_wave_t(const GemmLaunch &g, const typename Epi::Params &p0, hipStream_t s) {
+    typename Epi::Params p = p0;
+    if constexpr (std::is_same<typename Epi::Params, OptEpi>::value) {
+        // the parameter update's columns per workgroup, given for 256 threads
+        p.vec.cpb *= 64 * W / 256;
+        if (p.vec_blocks) p.vec_blocks = (p.vec.n + p.vec.cpb - 1) / p.vec.cpb;
+    }
+    GemmShape sh{};
+    sh.M = g.M;
+    sh.N = g.N;
+    sh.K = g.K;
+    sh.lda = g.lda;
+    sh.ldb = g.ldb;
+    sh.tiles_m = (g.M + 16 * MB - 1) / (16 * MB);
+    sh.tiles_n = (g.N + 16 * MB - 1) / (16 * MB);
+    sh.k_per_split = (g.K + 63u) / 64u * 64u;
+    sh.nv = epi_rows4<T>(g) ? 1u : 0u;
+    launch_timed(g, gemm_wave_kernel<T, Epi, AK, BK, REG, MB, MB, W, S, WPE>, dim3(sh.tiles_m * sh.tiles_n),
+                 dim3(64 * W), s, sh, reinterpret_cast<const T *>(g.A), reinterpret_cast<const T *>(g.B), p);
+    return hipGetLastError();
+}
+
+template <typename T, class Epi, bool AK, bool BK>
+static hipError_t run_wave(const GemmLaunch &g, const typename Epi::Params &p, hipStream_t s) {
+    if constexpr (sizeof(T) == 2) {
+        if (!wave_dword_rows(g)) {
+            switch (g.tile) {
+            case 16: return run_wave_t<T, Epi, AK, BK, true, 1, 16, 1, 4>(g, p, s);
+            case 32: return run_wave_t<T, Epi, AK, BK, true, 2, 8, 1, 4>(g, p, s);
+            case 64: return run_wave_t<T, Epi, AK, BK, true, 4, 4, 1, 2>(g, p, s);
+            }
+            return hipErrorInvalidValue;
+        }
+        switch (g.tile) {
+        case 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
+        case 32: return run_wave_t<T, Epi, AK, BK, false, 2, 4, 2, 2>(g, p, s);
+        case 64: return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
+        }
+    } else {
+        switch (g.tile) {
+        case 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
+        case 32: return run_wave_t<T, Epi, AK, BK, false, 2, 8, 1, 4>(g, p, s);
+        case 64: return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
+        }
+    }
+    return hipErrorInvalidValue;
+}
+
+template <typename T> static hipError_t run_wave_op(const GemmLaunch &g, hipStream_t s) {
+    switch (g.op) {
+    case Op::Fwd: return run_wave<T, EpiFwdK<T>, true, false>(g, g.fwd, s);
+    case Op::InputGrad: return run_wave<T, EpiStoreK, true, true>(g, g.st, s);
+    case Op::DwOpt: return run_wave<T, EpiOptK<T>, false, false>(g, g.opt, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+// Every row of both operands starts on a 4-byte boundary: direct-to-LDS loads.
+bool wave_dword_rows(const GemmLaunch &g) {
+    if (g.dtype == 0) return true;
+    auto ok = [](const void *p, uint32_t ld) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && ld % 2 == 0; };
+    return ok(g.A, g.lda) && ok(g.B, g.ldb);
+}
+
+// The layouts the kernel is instantiated for, and 32-bit byte offsets below 2 GiB within a
+// tile's rows (k-contiguous) or within the operand (m/n-contiguous).
+bool gemm_wave_ok(const GemmLaunch &g) {
+    const uint64_t esz = g.dtype == 1 ? 2 : 4;
+    if (!g.M || !g.N || !g.K) return false;
+    const bool layout = g.op == Op::Fwd ? g.a_kcontig && !g.b_kcontig
+                        : g.op == Op::InputGrad ? g.a_kcontig && g.b_kcontig
+                        : g.op == Op::DwOpt ? !g.a_kcontig && !g.b_kcontig : false;
+    auto span = [&](bool kc, uint32_t ld) { return ((kc ? 64ull : g.K + 64ull) * ld + g.K) * esz; };
+    return layout && span(g.a_kcontig, g.lda) < (1ull << 31) && span(g.b_kcontig, g.ldb) < (1ull << 31);
+}
+
+// Estimated time (us) of the three tiles, the larger of two lines fitted to measurements of
+// 100 shapes between 16 x 16 x 64 and 16384 x 4096 x 4096 (each within ~20%): what one
+// workgroup takes (the latency of its k-tiles, kt of 128 bytes), and the GPU's rate over
+// units of 256 tiles (one per CU).
+//   f16: 16x16 is ahead below ~256 of its tiles, 64x64 from ~128 of its own on, 32x32
+//        between (512 x 2048, K 2048: 74 / 19 / 12 us; 128 x 2048: 21 / 7.4 / 12)
+//   f32: 64x64 is bound by its MFMAs (0.5 us per k-tile and unit)
+uint32_t gemm_wave_tile(const GemmLaunch &g, double *us) {
+    struct Line { double l0, l1, r0, c, d; };
+    static const Line f16[3] = {{2.6, 0.14, 1.0, 0.085, 1.9}, {2.2, 0.155, 3.0, 0.108, 0.4}, {5.5, 0.17, 2.0, 0.195, 1.9}};
+    static const Line reg[3] = {{2.6, 0.15, 1.0, 0.090, 1.9}, {3.0, 0.18, 3.0, 0.130, 0.6}, {6.0, 0.36, 2.0, 0.230, 2.8}};
+    static const Line f32[3] = {{2.2, 0.11, 1.0, 0.060, 2.0}, {3.6, 0.14, 2.0, 0.122, 1.7}, {5.0, 0.51, 4.0, 0.497, 2.7}};
+    const Line *l = g.dtype == 0 ? f32 : wave_dword_rows(g) ? f16 : reg;
+    const double kt = (double)((g.K + (g.dtype == 0 ? 31u : 63u)) / (g.dtype == 0 ? 32u : 64u));
+    uint32_t best = 0;
+    for (uint32_t i = 0, t = 16; i < 3; ++i, t *= 2) {
+        const double units = (double)((g.M + t - 1) / t) * ((g.N + t - 1) / t) / 256.0;
+        const double lat = l[i].l0 + l[i].l1 * kt, rate = l[i].r0 + units * (l[i].c * kt + l[i].d);
+        const double e = lat > rate ? lat : rate;
+        if (!best || e < *us) {
+            best = t;
+            *us = e;
+        }
+    }
+    return best;
+}
+
+hipError_t launch_gemm_wave(const GemmLaunch &g, hipStream_t s) {
+    if (!gemm_wave_ok(g)) return hipErrorInvalidValue;
+    return g.dtype == 1 ? run_wave_op<half_t>(g, s) : run_wave_op<float>(g, s);
+}
+
+}  // namespace skl

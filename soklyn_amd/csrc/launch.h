@@ -113,11 +113,8 @@ struct GemmLaunch {
 };
 
 hipError_t launch_gemm(const GemmLaunch &g, hipStream_t stream);
-// Skinny outputs (N <= 16).  Forward: a streaming kernel, W staged in LDS
-// (fits when skinny_fwd_ok).  dW: batch-sliced partial sums of X^T . d_prenorm
+// Skinny outputs (N <= 16) of a long batch: batch-sliced partial sums of X^T . d_prenorm
 // (fp32) into partials [slices x K x 16]; skinny_dw_slices gives the slice count.
-bool skinny_fwd_ok(const GemmLaunch &g);
-hipError_t launch_skinny_fwd(const GemmLaunch &g, hipStream_t stream);
 uint32_t skinny_dw_slices(uint32_t rows, uint32_t K);
 hipError_t launch_skinny_dw(const GemmLaunch &g, float *partials, uint32_t slices, hipStream_t stream);
 // The 256x256 direct-to-LDS kernel on operands that fit it (gemm_dma_shape_ok):
@@ -125,6 +122,12 @@ hipError_t launch_skinny_dw(const GemmLaunch &g, float *partials, uint32_t slice
 // K a multiple of 128; DwPartial may split K into g.splits slices.
 hipError_t launch_gemm_dma(const GemmLaunch &g, hipStream_t stream);
 bool gemm_dma_shape_ok(const GemmLaunch &g);
+// The K-splitting kernel (gemm_wave.h) on output tiles of edge g.tile (16, 32 or 64): any
+// M, N, K >= 1, operands as stored.  gemm_wave_tile picks the tile and estimates its time.
+hipError_t launch_gemm_wave(const GemmLaunch &g, hipStream_t stream);
+bool gemm_wave_ok(const GemmLaunch &g);
+bool wave_dword_rows(const GemmLaunch &g);
+uint32_t gemm_wave_tile(const GemmLaunch &g, double *us);
 bool gemm_dma_enabled();
 // Output tile edge of the direct-to-LDS kernel forced by SOKLYN_GEMM_TILE (128 or
 // 256), or 0: the planner picks per GEMM.

@@ -1,0 +1,78 @@
+"""The K-splitting GEMM (16x16, 32x32 and 64x64 tiles, each wave its own k-tiles) through a
+layer's step, against the oracle: sizes around the edges of its tiles and k-tiles, fewer
+k-tiles than waves, widths that are odd (fp16 rows through registers), even but not whole
+16-byte chunks (the last chunk of a row masked), and large enough for each tile; outputs and
+inputs off a 16-byte boundary.  Gates as everywhere (tests/helpers.py)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from soklyn_amd import abi
+from tests.helpers import FP16_TOL, FP32_TOL, check_adam_update, f16, rng
+from tests.test_gpu_parity import check, dev, inputs, make_pair
+from tests.test_gpu_unaligned import misalign
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # batch, inputs, outputs
+    (1, 1, 1), (2, 3, 5), (16, 64, 16), (17, 65, 33), (15, 63, 31), (64, 128, 64), (33, 130, 66), (5, 1000, 24),
+    (70, 77, 200), (130, 36, 12), (20, 4100, 10), (257, 520, 136),
+    (700, 72, 900), (515, 330, 902), (701, 129, 835),      # 64x64 tiles
+]
+
+
+def step(ctx, half, M, K, N, off=0, x_off=0):
+    ob, db = make_pair(ctx, K, N, M, seed=M + K + N, half=half, act=abi.ACT_SILU)
+    if off:
+        misalign(db, off)
+    w0 = (db.get("master_w") if half else db.get("w")).copy()
+    x = inputs(81, M, K, half)
+    xd = dev(x, half)
+    if x_off:
+        buf = torch.zeros(xd.numel() + 8, device="cuda", dtype=xd.dtype)
+        view = buf[x_off:x_off + xd.numel()].view(xd.shape)
+        view.copy_(xd)
+        xd = view
+    s = (rng(82).standard_normal((M, N)) * 512).astype(np.float32)
+    print(f"step {M}x{K}->{N} half={half} off={off},{x_off}", flush=True)
+    ob.forward(x, M)
+    db.forward(xd, M)
+    ob.error_from_sum(s, M)
+    db.error_from_sum(torch.from_numpy(s).cuda(), M)
+    dx = db.input_grad(M).cpu().numpy()
+    opt = abi.sgd(0.5) if not half else abi.adam()
+    db.backward(xd, abi.train_ctx(opt, opt, M, 1e-3), 1)
+    torch.cuda.synchronize()
+    ref_dx = ob.input_grad(M)
+    oopt = O.Optimiser.adam() if half else O.Optimiser.sgd(0.5)
+    ob.backward(x, oopt, oopt, M, 1e-3, 3.4e38, 1)
+    tol = FP16_TOL if half else FP32_TOL
+    for name in ("preact", "predrop", "out"):
+        check(name, db.get(name), getattr(ob, name), tol)
+    check("dx", dx, ref_dx, tol)
+    m = "dm" if half else "dv"
+    for name in (f"{m}_w", f"{m}_b"):
+        check(name, db.get(name), getattr(ob, name), tol)
+    if half:
+        # Adam's first step is lr sign(g) whatever |g| is: where g is rounding noise the
+        # sign is, too, so the update is checked against the device's own moments
+        check_adam_update("w", w0, db.get("master_w"), db.get("dm_w"), db.get("dv_w"), 1e-3, 1,
+                          np.asarray(ob.master_w).reshape(K, N) - w0, np.asarray(ob.dm_w).reshape(K, N))
+        assert (db.get("w") == f16(db.get("master_w"))).all()
+    else:
+        check("w", db.get("w"), ob.w, tol)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_step(ctx, half, M, K, N):
+    step(ctx, half, M, K, N)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("off,x_off", [(1, 0), (2, 1), (0, 1), (0, 2), (0, 3)])
+def test_step_misaligned(ctx, half, off, x_off):
+    step(ctx, half, 50, 96, 72, off, x_off)
