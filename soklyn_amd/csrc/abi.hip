@@ -54,6 +54,16 @@ struct PadCopy {
     bool valid;
 };
 
+// Scratch of kernels that hand partial results to the launch after them (a BatchNorm's
+// column statistics), one piece per stream the context has run on: forwards on two
+// streams of one context share nothing else, so they may overlap.
+constexpr int kStreamSlots = 8;
+constexpr size_t STREAM_SCRATCH_BYTES = size_t(4) << 20;
+struct StreamScratch {
+    hipStream_t stream;
+    void *buf;
+};
+
 struct skl_ctx {
     int device;
     uint32_t tile_dim;
@@ -70,6 +80,7 @@ struct skl_ctx {
     bool keep_pads;      // SOKLYN_PAD_KEEP=0 at skl_ctx_create: GEMMs pad d_prenorm_h into the workspace every time
     hipEvent_t gemm_start, gemm_stop;   // skl_ctx_time_next_gemm
     void *scratch;       // device address of this device's copy of `scratch` (below)
+    StreamScratch streams[kStreamSlots];
 };
 
 // Scratch of the allocation-free entry point (skl_dense_error_from_sum_noalloc):
@@ -129,6 +140,28 @@ int32_t ensure_buf(skl_ctx *ctx, void **buf, size_t *have, size_t bytes) {
 }
 
 int32_t ensure_ws(skl_ctx *ctx, size_t bytes) { return ensure_buf(ctx, &ctx->ws, &ctx->ws_bytes, bytes); }
+
+// The stream's scratch, or null where the caller has to do without: more bytes than a
+// piece holds, a ninth stream, no memory, or a stream under capture (a replayed graph may
+// overlap eager calls on its stream's context, so captured kernels use none).
+void *stream_scratch(skl_ctx *ctx, size_t bytes) {
+    if (bytes == 0 || bytes > STREAM_SCRATCH_BYTES) return nullptr;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
+    for (StreamScratch &s : ctx->streams) {
+        if (s.buf && s.stream == ctx->stream) return s.buf;
+        if (!s.buf) {
+            if (hipMalloc(&s.buf, STREAM_SCRATCH_BYTES) != hipSuccess) {
+                (void)hipGetLastError();   // the caller goes on without
+                s.buf = nullptr;
+                return nullptr;
+            }
+            s.stream = ctx->stream;
+            return s.buf;
+        }
+    }
+    return nullptr;
+}
 
 // Device address of `scratch` on device `dev` (current), looked up once per device.
 constexpr int MAX_DEVICES = 64;
@@ -835,6 +868,8 @@ int32_t skl_ctx_destroy(skl_ctx *ctx) {
     if (ctx->cols) note(hipFree(ctx->cols));
     for (PadCopy &c : ctx->pads)
         if (c.buf) note(hipFree(c.buf));
+    for (StreamScratch &s : ctx->streams)
+        if (s.buf) note(hipFree(s.buf));
     note(hipStreamDestroy(ctx->own_stream));
     delete ctx;
     return first == hipSuccess ? SKL_OK : hip_status(first);
@@ -995,7 +1030,10 @@ int32_t skl_dense_forward(skl_ctx *ctx, const skl_dense_desc *b, const void *in,
         a.out = b->out;
         a.mask = b->mask;
         a.norm_rstd = b->norm_rstd;
-        SKL_TRY(launch_norm_act(a, ctx->stream));
+        float *stats = nullptr;
+        if (a.norm == SKL_NORM_BATCH)
+            stats = reinterpret_cast<float *>(stream_scratch(ctx, norm_cols_scratch(a.m, a.n)));
+        SKL_TRY(launch_norm_act(a, stats, ctx->stream));
     }
     return finish(ctx);
 }

@@ -510,17 +510,17 @@ template <typename T, int PER> __global__ void __launch_bounds__(256) norm_rows_
     }
 }
 
-// BatchNorm (forward.cu:74-126 with norm == 3), then act + dropout: a workgroup of
-// 1024 threads per 16 columns, all batch rows.  LPR = 16 / VW lanes share a row (4
-// elements each with VEC, one otherwise), so the workgroup takes RPW = 1024 / LPR
+// BatchNorm (forward.cu:74-126 with norm == 3), then act + dropout, in one launch: a
+// workgroup of 1024 threads per 16 columns, all batch rows.  LPR = 16 / VW lanes share a
+// row (4 elements each with VEC, one otherwise), so the workgroup takes RPW = 1024 / LPR
 // rows per step and thread t the rows t / LPR, + RPW, ...  HELD: the thread's (at most
 // PER) rows stay in registers, so prenorm is read once for the mean, the variance about
 // it and the outputs; longer batches read it again for each (from L2).  Each sum runs
 // over a thread's rows, then the wave's lanes of a column (butterfly), then the 16 waves
-// in order.  Bound: address processing of the five output streams (a row is one 32-byte
-// piece of a line per tensor) below ~4K rows, HBM above.  The line segments of 64
-// columns belong to 4 workgroups, which the block order puts on one XCD.
-// 2048 x 1024 fp16: 1565 us with one thread walking a column.
+// in order.  Bound: a row is one piece of a line in each of five tensors, ~4 clocks apiece
+// in the CU's address path whatever the piece's width (2048 x 1024 fp16: 20 us with 4, 8
+// or 16 columns per workgroup; 1565 us with one thread walking a column).  Taken for
+// short batches and where the two-launch form below has no scratch.
 template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024) norm_cols_kernel(RowNormArgs a) {
     constexpr uint32_t CT = 16, VW = VEC ? 4 : 1, LPR = CT / VW, RPW = 1024 / LPR;
     typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
@@ -646,6 +646,185 @@ template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024)
     });
 }
 
+// BatchNorm in two launches, for batches of more than a few hundred rows: rows are split
+// over workgroups as well as columns (64 per workgroup: whole lines).
+//  * norm_cols_stats_kernel: slice y of R = PER RPS rows, held in registers, leaves each
+//    column's mean and sum of squares about it in stats[2 y][n], stats[2 y + 1][n].
+//  * norm_cols_apply_kernel: every workgroup merges the slices of its 64 columns (the
+//    parallel form of the variance: M2 = sum M2_s + n_s (mean_s - mean)^2), then writes
+//    64 rows.
+// 256 threads: LPR = 64 / VW lanes per row, RPS = 256 / LPR rows per step.
+// 2048 x 1024 fp16: 4.0 + 8.0 us, against 20 us in one launch.
+template <typename T, bool VEC> struct ColRows {
+    static constexpr uint32_t VW = VEC ? 4 : 1, LPR = 64 / VW, RPS = 256 / LPR;
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    typedef typename std::conditional<sizeof(T) == 2, u32x2_t, u32x4_t>::type G;   // 4 elements
+    __device__ __forceinline__ static void load(const void *p, uint64_t i, T (&v)[VW]) {
+        if constexpr (VEC)
+            *reinterpret_cast<G *>(v) = *reinterpret_cast<const G *>(reinterpret_cast<const T *>(p) + i);
+        else
+            v[0] = ldv<T>(p, i);
+    }
+    __device__ __forceinline__ static void put(void *p, uint64_t i, const T (&v)[VW]) {
+        if constexpr (VEC)
+            __builtin_nontemporal_store(*reinterpret_cast<const G *>(v),
+                                        reinterpret_cast<G *>(reinterpret_cast<T *>(p) + i));
+        else
+            stv<T>(p, i, v[0]);
+    }
+};
+
+template <typename T, bool VEC, int PER>
+__global__ void __launch_bounds__(256) norm_cols_stats_kernel(RowNormArgs a, float *__restrict__ stats) {
+    typedef ColRows<T, VEC> C;
+    constexpr uint32_t VW = C::VW, LPR = C::LPR, RPS = C::RPS;
+    __shared__ float red[RPS][64];
+    const uint32_t n = a.n, lr = threadIdx.x % LPR, rr = threadIdx.x / LPR;
+    const uint32_t c0 = blockIdx.x * 64 + lr * VW;
+    const uint32_t r0 = blockIdx.y * (PER * RPS), cnt = min(a.m - r0, PER * RPS);
+    const bool cin = c0 < n;
+    T z[PER][VW];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (cin && rr + i * RPS < cnt) C::load(a.prenorm, (uint64_t)(r0 + rr + i * RPS) * n + c0, z[i]);
+    auto column_sum = [&](float (&s)[VW]) {
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) red[rr][lr * VW + e] = s[e];
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) {
+            float t = 0.0f;
+#pragma unroll
+            for (uint32_t w = 0; w < RPS; ++w) t += red[w][lr * VW + e];
+            s[e] = t;
+        }
+    };
+    float mean[VW] = {}, m2[VW] = {};
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (cin && rr + i * RPS < cnt) {
+#pragma unroll
+            for (uint32_t e = 0; e < VW; ++e) mean[e] += to_f32(z[i][e]);
+        }
+    column_sum(mean);
+#pragma unroll
+    for (uint32_t e = 0; e < VW; ++e) mean[e] /= (float)cnt;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (cin && rr + i * RPS < cnt) {
+#pragma unroll
+            for (uint32_t e = 0; e < VW; ++e) {
+                const float d = to_f32(z[i][e]) - mean[e];
+                m2[e] = fmaf(d, d, m2[e]);
+            }
+        }
+    column_sum(m2);
+    if (rr != 0 || !cin) return;
+    float *p = stats + (uint64_t)blockIdx.y * 2 * n + c0;
+#pragma unroll
+    for (uint32_t e = 0; e < VW; ++e) {
+        p[e] = mean[e];
+        p[n + e] = m2[e];
+    }
+}
+
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256) norm_cols_apply_kernel(RowNormArgs a, const float *__restrict__ stats,
+                                                              uint32_t slices, uint32_t per) {
+    typedef ColRows<T, VEC> C;
+    constexpr uint32_t VW = C::VW, LPR = C::LPR, RPS = C::RPS;
+    __shared__ float red[4][64], fin[2][64];
+    const uint32_t n = a.n, m = a.m, lr = threadIdx.x % LPR, rr = threadIdx.x / LPR;
+    const uint32_t c0 = blockIdx.x * 64 + lr * VW, r0 = blockIdx.y * 64;
+    const bool cin = c0 < n;
+    constexpr int PER = 64 / RPS;
+    T z[PER][VW];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (cin && r0 + rr + i * RPS < m) C::load(a.prenorm, (uint64_t)(r0 + rr + i * RPS) * n + c0, z[i]);
+    {
+        // column t % 64 of the tile, slices t / 64, + 4, ...: 16 of them in registers, both
+        // rows loaded before either is used; more in loops
+        const uint32_t t = threadIdx.x % 64, q = threadIdx.x / 64, c = blockIdx.x * 64 + t;
+        const bool in = c < n;
+        auto rows_of = [&](uint32_t s) { return (float)min(per, m - s * per); };
+        constexpr int NS = 16;
+        float sm[NS], sv[NS];
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const uint32_t s = q + 4 * i;
+            const bool ok = in && s < slices;
+            sm[i] = ok ? stats[(uint64_t)s * 2 * n + c] : 0.0f;
+            sv[i] = ok ? stats[(uint64_t)s * 2 * n + n + c] : 0.0f;
+        }
+        float s1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) s1 = q + 4 * i < slices ? fmaf(rows_of(q + 4 * i), sm[i], s1) : s1;
+        for (uint32_t s = q + 4 * NS; in && s < slices; s += 4) s1 = fmaf(rows_of(s), stats[(uint64_t)s * 2 * n + c], s1);
+        red[q][t] = s1;
+        __syncthreads();
+        const float mean = ((red[0][t] + red[1][t]) + (red[2][t] + red[3][t])) / (float)m;
+        float s2 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const float d = sm[i] - mean;
+            s2 = q + 4 * i < slices ? s2 + fmaf(rows_of(q + 4 * i) * d, d, sv[i]) : s2;
+        }
+        for (uint32_t s = q + 4 * NS; in && s < slices; s += 4) {
+            const float *p = stats + (uint64_t)s * 2 * n + c;
+            const float d = p[0] - mean;
+            s2 += fmaf(rows_of(s) * d, d, p[n]);
+        }
+        __syncthreads();
+        red[q][t] = s2;
+        __syncthreads();
+        if (q == 0) {
+            const float var = ((red[0][t] + red[1][t]) + (red[2][t] + red[3][t])) / (float)m + 1e-6f;
+            fin[0][t] = mean;
+            fin[1][t] = 1.0f / sqrtf(var);
+            if (in && blockIdx.y == 0) stv<T>(a.norm_rstd, c, from_f32<T>(fin[1][t]));
+        }
+        __syncthreads();
+    }
+    if (!cin) return;
+    float mean[VW], rstd[VW], g[VW], bias[VW];
+#pragma unroll
+    for (uint32_t e = 0; e < VW; ++e) {
+        mean[e] = fin[0][lr * VW + e];
+        rstd[e] = fin[1][lr * VW + e];
+        g[e] = to_f32(ldv<T>(a.norm_w, c0 + e));
+        bias[e] = to_f32(ldv<T>(a.norm_b, c0 + e));
+    }
+    const float scale = a.use_dropout ? 1.0f / (1.0f - a.p) : 1.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const uint32_t r = r0 + rr + i * RPS;
+        if (r >= m) break;
+        T cen[VW], pre[VW], pd[VW], mk[VW], ot[VW];
+        const uint32_t rk = dropout_rowkey(r, a.seed + r * 7u);
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) {
+            const float d = to_f32(z[i][e]) - mean[e];
+            cen[e] = from_f32<T>(d);
+            pre[e] = from_f32<T>(fmaf(d * rstd[e], g[e], bias[e]));
+            const float act = activation<T>(a.act, to_f32(pre[e]), a.leaky);
+            pd[e] = ot[e] = from_f32<T>(act);
+            if (a.use_dropout) {
+                const bool keep = (uint64_t)dropout_bits((c0 + e) * kDropColMul, rk) >= a.keep_min;
+                mk[e] = keep ? from_f32<T>(scale) : (T)0;
+                ot[e] = keep ? from_f32<T>(act * scale) : (T)0;
+            }
+        }
+        const uint64_t idx = (uint64_t)r * n + c0;
+        C::put(a.centered, idx, cen);
+        C::put(a.preact, idx, pre);
+        C::put(a.predrop, idx, pd);
+        C::put(a.out, idx, ot);
+        if (a.use_dropout) C::put(a.mask, idx, mk);
+    }
+}
+
 static bool a16p(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Rows up to 256 x 16 elements run with the row in registers (16-byte chunks when
@@ -687,14 +866,43 @@ template <typename T> static void launch_norm_rows(const RowNormArgs &a, hipStre
         hipLaunchKernelGGL(norm_rows_kernel<T>, g, b, 0, s, a);
 }
 
-// BatchNorm: 4-element groups where every row of every tensor starts on one; the batch
-// in registers where it fits.
-template <typename T> static void launch_norm_cols(const RowNormArgs &a, hipStream_t s) {
+// BatchNorm.  4-element groups where every row of every tensor starts on one.  Batches
+// of more than 384 rows in two launches when there is scratch for their slices (the one
+// launch takes ~4 us + 8 ns per row, the two ~7 us and the bytes); otherwise in one, the
+// batch in registers where it fits.
+constexpr uint32_t COLS_TWO_MIN = 384;
+// Rows per slice: 64, or 256 where that would be more than 64 slices.
+static uint32_t norm_cols_per(uint32_t m) { return m <= 64 * 64 ? 64 : 256; }
+
+size_t norm_cols_scratch(uint32_t m, uint32_t n) {
+    if (m <= COLS_TWO_MIN) return 0;
+    return (size_t)cdiv(m, norm_cols_per(m)) * 2 * n * sizeof(float);
+}
+
+template <typename T> static void launch_norm_cols(const RowNormArgs &a, float *stats, hipStream_t s) {
     constexpr uint32_t RPW_V = 256, RPW_1 = 64;   // rows per step
     constexpr uintptr_t GB = 4 * sizeof(T) - 1;
     auto ga = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & GB) == 0; };
     const bool vec = a.n % 4 == 0 && ga(a.prenorm) && ga(a.centered) && ga(a.preact) && ga(a.predrop) && ga(a.out) &&
                      (!a.use_dropout || ga(a.mask));
+    if (stats && a.m > COLS_TWO_MIN) {
+        const uint32_t per = norm_cols_per(a.m), slices = cdiv(a.m, per);
+        const dim3 gs(cdiv(a.n, 64), slices), ga2(cdiv(a.n, 64), cdiv(a.m, 64)), b(256);
+        if (vec) {
+            if (per == 64)
+                hipLaunchKernelGGL((norm_cols_stats_kernel<T, true, 4>), gs, b, 0, s, a, stats);
+            else
+                hipLaunchKernelGGL((norm_cols_stats_kernel<T, true, 16>), gs, b, 0, s, a, stats);
+            hipLaunchKernelGGL((norm_cols_apply_kernel<T, true>), ga2, b, 0, s, a, stats, slices, per);
+        } else {
+            if (per == 64)
+                hipLaunchKernelGGL((norm_cols_stats_kernel<T, false, 16>), gs, b, 0, s, a, stats);
+            else
+                hipLaunchKernelGGL((norm_cols_stats_kernel<T, false, 64>), gs, b, 0, s, a, stats);
+            hipLaunchKernelGGL((norm_cols_apply_kernel<T, false>), ga2, b, 0, s, a, stats, slices, per);
+        }
+        return;
+    }
     const dim3 g(cdiv(a.n, 16)), b(1024);
     if (vec && a.m <= 2 * RPW_V)
         hipLaunchKernelGGL((norm_cols_kernel<T, true, 2>), g, b, 0, s, a);
@@ -704,21 +912,19 @@ template <typename T> static void launch_norm_cols(const RowNormArgs &a, hipStre
         hipLaunchKernelGGL((norm_cols_kernel<T, true, 0>), g, b, 0, s, a);
     else if (a.m <= 8 * RPW_1)
         hipLaunchKernelGGL((norm_cols_kernel<T, false, 8>), g, b, 0, s, a);
-    else if (a.m <= 32 * RPW_1)
-        hipLaunchKernelGGL((norm_cols_kernel<T, false, 32>), g, b, 0, s, a);
     else
         hipLaunchKernelGGL((norm_cols_kernel<T, false, 0>), g, b, 0, s, a);
 }
 
-hipError_t launch_norm_act(const RowNormArgs &a0, hipStream_t s) {
+hipError_t launch_norm_act(const RowNormArgs &a0, float *stats, hipStream_t s) {
     if (a0.m == 0 || a0.n == 0) return hipSuccess;
     RowNormArgs a = a0;
     a.keep_min = dropout_keep_min(a.p);
     if (a.norm == 3) {
         if (a.dtype == 1)
-            launch_norm_cols<half_t>(a, s);
+            launch_norm_cols<half_t>(a, stats, s);
         else
-            launch_norm_cols<float>(a, s);
+            launch_norm_cols<float>(a, stats, s);
     } else if (a.dtype == 1) {
         launch_norm_rows<half_t>(a, s);
     } else {
