@@ -1460,7 +1460,9 @@ static bool err_aligned(const ErrArgs &a, bool from_sum, const float *partials) 
 static uint32_t err_band(uint32_t n) { return (n & 3u) == 0 ? 1u : (n & 1u) ? 4u : 2u; }
 
 // Partial-sum rows of the error kernels: S row slices x err_band(n).  ~1024
-// workgroups of >= 16 rows when a band has >= 256 chunks; narrower outputs
+// workgroups of >= 16 rows when a band has >= 256 chunks, down to 4 rows (one batch of
+// loads) where that leaves fewer than one per CU (512 x 2048 fp16 with RMSNorm: 32
+// slices 22.3 us, 128 slices 9.3; 2048 x 1024: 128 slices 20.8, 256 17.8); narrower outputs
 // leave most of a workgroup's lanes idle, so they get ~256K active lanes in
 // all, in slices of >= 4 rows (at most 4096 slices).  resident (when not 0):
 // the kernel's workgroups the GPU holds at once; a grid that would exceed it
@@ -1475,6 +1477,8 @@ uint32_t err_col_splits(uint32_t rows, uint32_t n, uint32_t resident) {
     if (chunks >= 256) {
         sp = cdiv(1024, gx);
         cap = cdiv(rows, 16);
+        const uint32_t fill = cdiv(256, gx);
+        if (cap < fill) cap = std::min(fill, cdiv(rows, 4));
     } else {
         sp = cdiv(262144u, chunks ? chunks : 1);
         cap = cdiv(rows, 4);
