@@ -25,12 +25,6 @@ template <typename T> static bool epi_rows4(const GemmLaunch &g) {
 // 16 waves of 16x16 and 4 or 8 of 32x32 or 64x64 put 64-128 KB of loads in flight per CU.
 template <typename T, class Epi, bool AK, bool BK, bool REG, int MB, int W, int S, int WPE>
 static hipError_t run_wave_t(const GemmLaunch &g, const typename Epi::Params &p0, hipStream_t s) {
-    typename Epi::Params p = p0;
-    if constexpr (std::is_same<typename Epi::Params, OptEpi>::value) {
-        // the parameter update's columns per workgroup, given for 256 threads
-        p.vec.cpb *= 64 * W / 256;
-        if (p.vec_blocks) p.vec_blocks = (p.vec.n + p.vec.cpb - 1) / p.vec.cpb;
-    }
     GemmShape sh{};
     sh.M = g.M;
     sh.N = g.N;
@@ -41,7 +35,23 @@ static hipError_t run_wave_t(const GemmLaunch &g, const typename Epi::Params &p0
     sh.tiles_n = (g.N + 16 * MB - 1) / (16 * MB);
     sh.k_per_split = (g.K + 63u) / 64u * 64u;
     sh.nv = epi_rows4<T>(g) ? 1u : 0u;
-    launch_timed(g, gemm_wave_kernel<T, Epi, AK, BK, REG, MB, MB, W, S, WPE>, dim3(sh.tiles_m * sh.tiles_n),
+    const uint32_t tiles = sh.tiles_m * sh.tiles_n;
+    typename Epi::Params p = p0;
+    uint32_t more = 0;
+    if constexpr (std::is_same<typename Epi::Params, OptEpi>::value) {
+        if (p.vec_blocks) {
+            // The parameter update: columns per workgroup as given for 256 threads, in
+            // workgroups of its own where the last round of tiles leaves room for them
+            // (1024 x 1024 dW over 2048 rows: 22 -> 19 us), else behind the tiles (2048 x
+            // 1000, 512 tiles in one full round: 48 us a step in a second round, 45 so).
+            constexpr uint32_t slots = MB == 1 ? 256 : 512;   // workgroups resident at once
+            p.vec.cpb *= 64 * W / 256;
+            const uint32_t blocks = (p.vec.n + p.vec.cpb - 1) / p.vec.cpb, last = tiles % slots;
+            if (last && last + blocks <= slots) more = blocks;
+            p.vec_blocks = more ? 0 : blocks;
+        }
+    }
+    launch_timed(g, gemm_wave_kernel<T, Epi, AK, BK, REG, MB, MB, W, S, WPE>, dim3(tiles + more),
                  dim3(64 * W), s, sh, reinterpret_cast<const T *>(g.A), reinterpret_cast<const T *>(g.B), p);
     return hipGetLastError();
 }
