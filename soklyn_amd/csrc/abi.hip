@@ -425,20 +425,32 @@ uint32_t dma_tile(Op op, uint32_t Mp, uint32_t Np, uint32_t splits, uint32_t *ba
 }
 
 // Estimated time (us) of the register-staged kernels, from the measurements behind
-// gemm_wave_tile: a 128x128 fp16 tile takes ~1 us per 64 k whatever the grid, 4 us when
+// gemm_wave_tile.  fp16: a 128x128 tile takes ~1 us per 64 k whatever the grid, 4 us when
 // its rows are not 16-byte aligned (gathered element by element), and a second tile per
 // CU hides part of it (4096 x 1024, K 1024: 25 us; 512 x 2048, K 2048: 36; 2000 x 1531,
-// K 777: 66).  fp32 grids of at least 192 tiles of 128x128 (160 for a dW) run them at the
-// rate of the K-splitting kernel or above (4096 x 1024, K 1024: dX 70 against 73 us);
-// smaller ones never do.
+// K 777: 66).  fp32: grids of at least 192 tiles of 128x128 (160 for a dW) run them in
+// rounds of 256 (4096 x 1024, K 1024: dX 70 us, forward 82; 8192 rows 133 and 147);
+// smaller ones are behind the K-splitting kernel throughout.
 double staged_us(const GemmLaunch &g) {
     const double tiles = (double)((g.M + 127) / 128) * ((g.N + 127) / 128);
-    if (g.dtype == SKL_F32) return tiles >= (g.op == Op::DwOpt ? 160 : 192) ? 0.0 : 1e30;
+    if (g.dtype == SKL_F32) {
+        if (tiles < (g.op == Op::DwOpt ? 160 : 192)) return 1e30;
+        return std::ceil(tiles / 256.0) * (6.0 + (g.op == Op::InputGrad ? 1.95 : 2.1) * (double)((g.K + 31) / 32));
+    }
     const uint32_t a_ext = g.a_kcontig ? g.K : g.M, b_ext = g.b_kcontig ? g.K : g.N;
     const bool vec = g.lda % 8 == 0 && g.ldb % 8 == 0 && a_ext % 8 == 0 && b_ext % 8 == 0 && aligned16(g.A) &&
                      aligned16(g.B);
     const double kt = (double)((g.K + 63) / 64), u = tiles / 256.0;
     return vec ? 10.0 + kt * (u > 1.25 ? 0.8 * u : 1.0) : 15.0 + kt * (u > 1.0 ? 4.0 * u : 4.0);
+}
+
+// The same for 128x128 direct-to-LDS tiles on a grid short of the 256x256 kernel's, whose
+// operands it reads in place (2048 x 2048, K 2048: 29.4 us, 33 on the K-splitting kernel;
+// 4096 x 2048: 42, 56; dX of 4096 x 1024, K 1024: 14.6, 16.5).  Not the dW, whose fused
+// optimiser is faster on small tiles (2048 x 2048 over 512 rows: 31, 25).
+double dma128_us(const GemmLaunch &g) {
+    const double u = (double)(g.M / 128) * (g.N / 128) / 256.0, kt = g.K / 64.0;
+    return (g.op == Op::InputGrad ? 4.5 : 8.5) + kt * (0.33 + 0.32 * (u > 1.0 ? u : 1.0));
 }
 
 // in_place: the output overlaps an operand (a caller's dx over d_prenorm).  The K-splitting
@@ -500,6 +512,15 @@ GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
             p.a_bytes = p.pad_a ? ((size_t)Mp * Kp * 2 + 255) & ~(size_t)255 : 0;
             p.b_bytes = p.pad_b ? ((size_t)Np * Kp * 2 + 255) & ~(size_t)255 : 0;
             p.part_bytes = splits > 1 ? (size_t)splits * Mp * Np * sizeof(float) : 0;
+            return p;
+        }
+    }
+    if (g.dtype == SKL_F16 && !dw && !in_place && (g.M % 256) == 0 && (g.N % 256) == 0 && gemm_dma_shape_ok(g) &&
+        !gemm_dma_tile_forced()) {
+        const double us = dma128_us(g);
+        if ((!wave || us < wave_us) && us < staged_us(g)) {
+            p.dma = true;
+            p.tile = 128;
             return p;
         }
     }

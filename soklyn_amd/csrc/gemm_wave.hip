@@ -23,6 +23,22 @@ template <typename T> static bool epi_rows4(const GemmLaunch &g) {
 
 // Tiles: rows = columns = 16, 32 or 64, with the waves that share a workgroup's K.
 // 16 waves of 16x16 and 4 or 8 of 32x32 or 64x64 put 64-128 KB of loads in flight per CU.
+// 64x64 tiles keep two waves per SIMD resident, so the fewer waves share a tile, the more
+// tiles one round holds: 4 waves and 512 tiles, or where that makes the grid one round at
+// least three quarters full, 2 waves and 1024 (4096 x 1024, K 1024: f16 21.5 -> 19.9 us, f32
+// 79 -> 73; a grid of 512 so: 43 -> 68, a pair of waves per CU sits on two of its SIMDs) and
+// in fp32 1 wave and 2048 (8192 x 1024, K 1024: 154 -> 143).  Up to 256 tiles fp32 takes 8
+// waves (1024 x 1024 dW over 4096 rows: 76 -> 70).
+static uint32_t wave_share(uint32_t dtype, uint64_t tiles64) {
+    if (tiles64 > 768 && tiles64 <= 1024) return 2;
+    if (dtype == 0 && tiles64 > 1536 && tiles64 <= 2048) return 1;
+    if (dtype == 0 && tiles64 <= 256) return 8;
+    return 4;
+}
+static uint64_t tiles_of(const GemmLaunch &g, uint32_t t) {
+    return (uint64_t)((g.M + t - 1) / t) * ((g.N + t - 1) / t);
+}
+
 template <typename T, class Epi, bool AK, bool BK, bool REG, int MB, int W, int S, int WPE>
 static hipError_t run_wave_t(const GemmLaunch &g, const typename Epi::Params &p0, hipStream_t s) {
     GemmShape sh{};
@@ -44,8 +60,9 @@ static hipError_t run_wave_t(const GemmLaunch &g, const typename Epi::Params &p0
             // workgroups of its own where the last round of tiles leaves room for them
             // (1024 x 1024 dW over 2048 rows: 22 -> 19 us), else behind the tiles (2048 x
             // 1000, 512 tiles in one full round: 48 us a step in a second round, 45 so).
-            constexpr uint32_t slots = MB == 1 ? 256 : 512;   // workgroups resident at once
-            p.vec.cpb *= 64 * W / 256;
+            constexpr uint32_t slots = MB == 1 ? 256 : MB == 2 ? 512 : 2048 / W;   // workgroups resident at once
+            static_assert(W >= 2, "the update's workgroup");
+            p.vec.cpb = p.vec.cpb * W >= 4 ? p.vec.cpb * W / 4 : 1;
             const uint32_t blocks = (p.vec.n + p.vec.cpb - 1) / p.vec.cpb, last = tiles % slots;
             if (last && last + blocks <= slots) more = blocks;
             p.vec_blocks = more ? 0 : blocks;
@@ -70,13 +87,23 @@ static hipError_t run_wave(const GemmLaunch &g, const typename Epi::Params &p, h
         switch (g.tile) {
         case 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
         case 32: return run_wave_t<T, Epi, AK, BK, false, 2, 4, 2, 2>(g, p, s);
-        case 64: return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
+        case 64:
+            return wave_share(1, tiles_of(g, 64)) == 2 ? run_wave_t<T, Epi, AK, BK, false, 4, 2, 1, 2>(g, p, s)
+                                                       : run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
         }
     } else {
         switch (g.tile) {
         case 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
         case 32: return run_wave_t<T, Epi, AK, BK, false, 2, 8, 1, 4>(g, p, s);
-        case 64: return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
+        case 64:
+            switch (wave_share(0, tiles_of(g, 64))) {
+            case 8: return run_wave_t<T, Epi, AK, BK, false, 4, 8, 1, 2>(g, p, s);
+            case 2: return run_wave_t<T, Epi, AK, BK, false, 4, 2, 1, 2>(g, p, s);
+            case 1:
+                if constexpr (!std::is_same<typename Epi::Params, OptEpi>::value)
+                    return run_wave_t<T, Epi, AK, BK, false, 4, 1, 1, 2>(g, p, s);
+            }
+            return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
         }
     }
     return hipErrorInvalidValue;
@@ -117,18 +144,27 @@ bool gemm_wave_ok(const GemmLaunch &g) {
 //   f16: 16x16 is ahead below ~256 of its tiles, 64x64 from ~128 of its own on, 32x32
 //        between (512 x 2048, K 2048: 74 / 19 / 12 us; 128 x 2048: 21 / 7.4 / 12)
 //   f32: 64x64 is bound by its MFMAs (0.5 us per k-tile and unit)
+// 64x64 grids that fill one round with fewer waves per tile (wave_share) have a line of
+// their own.
 uint32_t gemm_wave_tile(const GemmLaunch &g, double *us) {
     struct Line { double l0, l1, r0, c, d; };
     static const Line f16[3] = {{2.6, 0.14, 1.0, 0.085, 1.9}, {2.2, 0.155, 3.0, 0.108, 0.4}, {5.5, 0.17, 2.0, 0.195, 1.9}};
     static const Line reg[3] = {{2.6, 0.15, 1.0, 0.090, 1.9}, {3.0, 0.18, 3.0, 0.130, 0.6}, {6.0, 0.36, 2.0, 0.230, 2.8}};
     static const Line f32[3] = {{2.2, 0.11, 1.0, 0.060, 2.0}, {3.6, 0.14, 2.0, 0.122, 1.7}, {5.0, 0.51, 4.0, 0.497, 2.7}};
-    const Line *l = g.dtype == 0 ? f32 : wave_dword_rows(g) ? f16 : reg;
+    const bool dword = wave_dword_rows(g);
+    const Line *l = g.dtype == 0 ? f32 : dword ? f16 : reg;
     const double kt = (double)((g.K + (g.dtype == 0 ? 31u : 63u)) / (g.dtype == 0 ? 32u : 64u));
     uint32_t best = 0;
     for (uint32_t i = 0, t = 16; i < 3; ++i, t *= 2) {
-        const double units = (double)((g.M + t - 1) / t) * ((g.N + t - 1) / t) / 256.0;
+        const uint64_t tiles = tiles_of(g, t);
+        const double units = (double)tiles / 256.0;
         const double lat = l[i].l0 + l[i].l1 * kt, rate = l[i].r0 + units * (l[i].c * kt + l[i].d);
-        const double e = lat > rate ? lat : rate;
+        double e = lat > rate ? lat : rate;
+        if (t == 64 && dword) {
+            const uint32_t w = wave_share(g.dtype, tiles);
+            if (w == 2) e = g.dtype == 0 ? 8.0 + 1.98 * kt : 6.5 + 0.83 * kt;
+            if (w == 1 && g.op != Op::DwOpt) e = 12.0 + 3.9 * kt;
+        }
         if (!best || e < *us) {
             best = t;
             *us = e;

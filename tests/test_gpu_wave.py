@@ -12,6 +12,7 @@ import torch
 from oracle import oracle as O
 from soklyn_amd import abi
 from tests.helpers import FP16_TOL, FP32_TOL, check_adam_update, f16, rng
+from tests.test_gpu_fused_error import test_fused_hidden_error_and_backward as fused_error
 from tests.test_gpu_parity import check, dev, inputs, make_pair
 from tests.test_gpu_unaligned import misalign
 
@@ -21,6 +22,7 @@ SHAPES = [  # batch, inputs, outputs
     (1, 1, 1), (2, 3, 5), (16, 64, 16), (17, 65, 33), (15, 63, 31), (64, 128, 64), (33, 130, 66), (5, 1000, 24),
     (70, 77, 200), (130, 36, 12), (20, 4100, 10), (257, 520, 136),
     (700, 72, 900), (515, 330, 902), (701, 129, 835),      # 64x64 tiles
+    (1700, 40, 2000), (2500, 33, 2560), (2000, 1700, 40),  # fewer waves per tile
 ]
 
 
@@ -76,3 +78,16 @@ def test_step(ctx, half, M, K, N):
 @pytest.mark.parametrize("off,x_off", [(1, 0), (2, 1), (0, 1), (0, 2), (0, 3)])
 def test_step_misaligned(ctx, half, off, x_off):
     step(ctx, half, 50, 96, 72, off, x_off)
+
+
+# fp16 grids on 128x128 direct-to-LDS tiles short of the 256x256 kernel's: the forward, the
+# input gradient and, in the hidden error, the fused epilogue
+
+
+def test_step_128(ctx):
+    step(ctx, True, 2048, 1024, 2048)
+
+
+@pytest.mark.parametrize("norm,act,p", [(abi.NORM_RMS, abi.ACT_MISH, 0.1), (abi.NORM_BATCH, abi.ACT_TANH, 0.0)])
+def test_hidden_error_128(ctx, norm, act, p):
+    fused_error(ctx, 2048, 64, 2048, 1024, norm, act, p, 0)
