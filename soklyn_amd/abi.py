@@ -114,7 +114,7 @@ def load(path: str = LIB_PATH):
 
 
 def call(name: str, *args) -> int:
-    rc = getattr(load(), name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != SKL_OK:
         raise SklError(name, rc)
     return rc

@@ -5,6 +5,8 @@
 #include "launch.h"
 #include "vec_opt.h"
 
+#include <algorithm>
+#include <atomic>
 #include <type_traits>
 #include <utility>
 
@@ -1515,9 +1517,13 @@ template <typename T> static uint32_t err_flat_per_cu_s(uint32_t src, uint32_t b
 
 uint32_t err_resident(uint32_t dtype, uint32_t src, uint32_t n, bool norm) {
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        return 0;
+    static std::atomic<int> known[64];   // CUs of each device, asked for once
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
+    if (dev < 64) cus = known[dev].load(std::memory_order_relaxed);
+    if (cus == 0) {
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 0;
+        if (dev < 64) known[dev].store(cus, std::memory_order_relaxed);
+    }
     const uint32_t band = err_band(n);
     const uint32_t per_cu = dtype == 1 ? err_flat_per_cu_s<half_t>(src, band, norm)
                                        : err_flat_per_cu_s<float>(src, band, norm);

@@ -9,6 +9,7 @@ blocks fp32 masters.  Every hot-path step is one C-ABI call.
 from __future__ import annotations
 
 import ctypes as C
+import threading
 
 import numpy as np
 import torch
@@ -19,6 +20,27 @@ T_FIELDS = ("w", "b", "norm_w", "norm_b", "out", "predrop", "preact", "centered"
 F32_FIELDS = ("master_w", "master_b", "master_norm_w", "master_norm_b",
               "dv_w", "dv_b", "dm_w", "dm_b", "dv_norm_w", "dv_norm_b", "dm_norm_w", "dm_norm_b",
               "grad", "d_prenorm", "d_norm_w", "d_norm_b")
+
+
+# The descriptor pointers each call reads (src/io/device/ffn_device.rs), without a norm and
+# those that come with one.  A descriptor of 28 tensors costs more to fill than the launch it
+# describes (3.4 us; 9.2 us for a whole forward call), so each call fills its own few.
+_NORM_CACHES = ("norm_w", "norm_b", "centered", "prenorm", "norm_rstd")
+_ERROR = ("w", "preact", "grad", "d_prenorm", "d_prenorm_h")
+_ERROR_NORM = _NORM_CACHES + ("d_norm_w", "d_norm_b", "master_norm_w")
+_UPDATE = ("w", "b", "master_w", "master_b", "dv_w", "dm_w", "dv_b", "dm_b", "grad", "d_prenorm", "d_prenorm_h")
+_UPDATE_NORM = _ERROR_NORM + ("master_norm_b", "dv_norm_w", "dm_norm_w", "dv_norm_b", "dm_norm_b")
+_READS = {
+    "forward": (("w", "b", "out", "predrop", "preact", "mask"), _NORM_CACHES),
+    "output_error": (_ERROR + ("out",), _ERROR_NORM),
+    "error": (_ERROR + ("predrop", "mask"), _ERROR_NORM),
+    "input_grad": (("w", "d_prenorm", "d_prenorm_h"), ()),
+    "above": (("w", "d_prenorm", "d_prenorm_h"), ()),
+    "update": (_UPDATE, _UPDATE_NORM),
+    "hidden": (_UPDATE + ("predrop", "preact", "mask"), _UPDATE_NORM),
+}
+_SCALARS = tuple(n for n, _ in abi.SklDenseDesc._fields_[:11])
+_PTR_AT = {n: getattr(abi.SklDenseDesc, n).offset // 8 for n in abi.DESC_POINTERS}
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -72,6 +94,7 @@ class DeviceBlock:
             setattr(self, n, zeros((M, N), torch.float32) if is_training else None)
         self.d_prenorm_h = zeros((M, N), torch.float16) if (half and is_training) else None
         self._desc = None
+        self._local = threading.local()   # _fill's descriptors, one set per thread
 
     # -- descriptor -----------------------------------------------------------------
     def desc(self) -> abi.SklDenseDesc:
@@ -86,40 +109,63 @@ class DeviceBlock:
         self._desc = d
         return d
 
+    def _fill(self, call: str):
+        """Reference to this call's own descriptor with its pointers read from the tensors as
+        they are now; the pointers it does not read stay null."""
+        key = (self.half, self.inputs, self.outputs, self.max_batch, self.norm, self.act, self.leaky, self.mask_coeff,
+               self.regularisation, self.regu_coeff, self.is_training)
+        descs = self._local.__dict__
+        kept = descs.get(call)
+        if kept is None or kept[0] != key:
+            d = abi.SklDenseDesc()
+            for n, v in zip(_SCALARS, (abi.F16 if self.half else abi.F32,) + key[1:10] + (int(self.is_training),)):
+                setattr(d, n, v)
+            names, with_norm = _READS[call]
+            at = tuple((n, _PTR_AT[n]) for n in (names + with_norm if self.norm else names))
+            kept = descs[call] = (key, C.byref(d), memoryview(d).cast("B").cast("Q"), at)
+        _, ref, words, at = kept
+        tensors = self.__dict__
+        for n, i in at:
+            t = tensors[n]
+            words[i] = 0 if t is None else t.data_ptr()
+        return ref
+
     # -- hot-path steps ------------------------------------------------------------------
     def forward(self, x: torch.Tensor, batch: int, use_dropout: bool = False, seed: int = 0):
-        abi.call("skl_dense_forward", self.ctx.h, C.byref(self.desc()), C.c_void_p(x.data_ptr()),
-                 x.shape[0], x.shape[1], batch, int(use_dropout), seed & 0xFFFFFFFF)
+        rows, cols = x.shape
+        abi.call("skl_dense_forward", self.ctx.h, self._fill("forward"), x.data_ptr(), rows, cols, batch,
+                 int(use_dropout), seed & 0xFFFFFFFF)
         return self.out
 
     def output_error(self, target: torch.Tensor, loss: int, act: int, leaky: float = 0.0):
-        abi.call("skl_dense_output_error", self.ctx.h, C.byref(self.desc()), C.c_void_p(target.data_ptr()),
-                 target.shape[0], target.shape[1], loss, act, leaky)
+        rows, cols = target.shape
+        abi.call("skl_dense_output_error", self.ctx.h, self._fill("output_error"), target.data_ptr(), rows, cols, loss,
+                 act, leaky)
 
     def hidden_error(self, nxt: "DeviceBlock", batch: int):
-        abi.call("skl_dense_hidden_error", self.ctx.h, C.byref(self.desc()), C.byref(nxt.desc()), batch)
+        abi.call("skl_dense_hidden_error", self.ctx.h, self._fill("hidden"), nxt._fill("above"), batch)
 
     def backward(self, x: torch.Tensor, tc: abi.SklTrainCtx, step: int):
-        abi.call("skl_dense_backward", self.ctx.h, C.byref(self.desc()), C.c_void_p(x.data_ptr()),
-                 x.shape[0], x.shape[1], C.byref(tc), step)
+        rows, cols = x.shape
+        abi.call("skl_dense_backward", self.ctx.h, self._fill("update"), x.data_ptr(), rows, cols, C.byref(tc), step)
 
     def backward_hidden(self, nxt: "DeviceBlock", x: torch.Tensor, tc: abi.SklTrainCtx, step: int):
-        abi.call("skl_dense_backward_hidden", self.ctx.h, C.byref(self.desc()), C.byref(nxt.desc()),
-                 C.c_void_p(x.data_ptr()), x.shape[0], x.shape[1], C.byref(tc), step)
+        rows, cols = x.shape
+        abi.call("skl_dense_backward_hidden", self.ctx.h, self._fill("hidden"), nxt._fill("above"), x.data_ptr(), rows,
+                 cols, C.byref(tc), step)
 
     def error_from_sum(self, s: torch.Tensor, batch: int):
         assert s.dtype == torch.float32 and s.is_contiguous()
-        abi.call("skl_dense_error_from_sum", self.ctx.h, C.byref(self.desc()), C.c_void_p(s.data_ptr()), batch)
+        abi.call("skl_dense_error_from_sum", self.ctx.h, self._fill("error"), s.data_ptr(), batch)
 
     def error_from_sum_noalloc(self, s: torch.Tensor, batch: int):
         assert s.dtype == torch.float32 and s.is_contiguous()
-        abi.call("skl_dense_error_from_sum_noalloc", self.ctx.h, C.byref(self.desc()), C.c_void_p(s.data_ptr()),
-                 batch)
+        abi.call("skl_dense_error_from_sum_noalloc", self.ctx.h, self._fill("error"), s.data_ptr(), batch)
 
     def input_grad(self, batch: int, out: torch.Tensor | None = None) -> torch.Tensor:
         if out is None:
             out = torch.empty((batch, self.inputs), device=self.w.device, dtype=torch.float32)
-        abi.call("skl_dense_input_grad", self.ctx.h, C.byref(self.desc()), batch, C.c_void_p(out.data_ptr()))
+        abi.call("skl_dense_input_grad", self.ctx.h, self._fill("input_grad"), batch, out.data_ptr())
         return out
 
     # -- host views ----------------------------------------------------------------------
