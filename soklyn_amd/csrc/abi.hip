@@ -320,11 +320,10 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //    fp32 partial sums, in the workspace, are reduced by the optimiser kernel).
 //  * the K-splitting kernel on small tiles (gemm_wave.h), for outputs that would leave
 //    those tiles' GPU mostly idle and for at most 16 columns: operands as stored, no
-//    workspace;
+//    workspace but the partial planes of a dW over a long batch;
 //  * the register-staged kernels otherwise (large fp32; small fp16 with little k to
 //    reduce), with the same split-K for small dW grids.
 struct GemmPlan {
-    bool skinny;               // N <= 16: the streaming kernels of dW partials
     uint32_t wave;             // K-splitting kernel: its tile edge (0: another kernel)
     bool dma;
     bool pad_a, pad_b;
@@ -356,7 +355,7 @@ bool dma_operand_ok(const void *p, uint32_t rows, uint32_t cols, uint32_t ld, ui
 // when that is faster: C5's 1024 x 1536 dW (24 tiles) on 128x128 tiles in 5
 // slices, 17 us faster than 256x256 in 10; C4's 2048 x 2048 dW stays on
 // 256x256 in 4 slices (128x128 in 2: +26 us a layer).
-uint32_t dw_dma_splits(uint32_t tiles, uint32_t Kp, uint64_t out_elems, uint32_t *tile) {
+uint32_t dw_dma_splits(uint32_t tiles, uint32_t Kp, uint64_t out_elems, uint32_t *tile, double *us) {
     constexpr uint32_t kCus = 256;
     uint32_t best = 1;
     double best_us = 0.0;
@@ -378,6 +377,7 @@ uint32_t dw_dma_splits(uint32_t tiles, uint32_t Kp, uint64_t out_elems, uint32_t
             }
         }
     }
+    *us = best_us;
     return best;
 }
 
@@ -430,13 +430,17 @@ uint32_t dma_tile(Op op, uint32_t Mp, uint32_t Np, uint32_t splits, uint32_t *ba
 // CU hides part of it (4096 x 1024, K 1024: 25 us; 512 x 2048, K 2048: 36; 2000 x 1531,
 // K 777: 66).  fp32: grids of at least 192 tiles of 128x128 (160 for a dW) run them in
 // rounds of 256 (4096 x 1024, K 1024: dX 70 us, forward 82; 8192 rows 133 and 147);
-// smaller ones are behind the K-splitting kernel throughout.
+// smaller ones, and any fp16 dW (2048 x 2048 over 512 rows: 31 us, 25), are behind the
+// K-splitting kernel throughout.
 double staged_us(const GemmLaunch &g) {
     const double tiles = (double)((g.M + 127) / 128) * ((g.N + 127) / 128);
+    const bool dw = g.op == Op::DwOpt;
     if (g.dtype == SKL_F32) {
-        if (tiles < (g.op == Op::DwOpt ? 160 : 192)) return 1e30;
-        return std::ceil(tiles / 256.0) * (6.0 + (g.op == Op::InputGrad ? 1.95 : 2.1) * (double)((g.K + 31) / 32));
+        if (tiles < (dw ? 160 : 192)) return 1e30;
+        return std::ceil(tiles / 256.0) * (6.0 + (g.op == Op::InputGrad ? 1.95 : 2.1) * (double)((g.K + 31) / 32)) +
+               (dw ? (double)g.M * g.N * 16.0 / 7.0e6 : 0.0);
     }
+    if (dw) return 1e30;
     const uint32_t a_ext = g.a_kcontig ? g.K : g.M, b_ext = g.b_kcontig ? g.K : g.N;
     const bool vec = g.lda % 8 == 0 && g.ldb % 8 == 0 && a_ext % 8 == 0 && b_ext % 8 == 0 && aligned16(g.A) &&
                      aligned16(g.B);
@@ -463,29 +467,33 @@ GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
     p.Np = g.N;
     p.Kp = g.K;
     const bool dw = g.op == Op::DwOpt;
+    // a dW may go in batch slices (partial planes in the workspace) where the register-
+    // staged kernels would split it too: below 160 tiles of 128x128 and from 8 k-tiles on
+    const uint32_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128);
     double wave_us = 0.0;
-    const uint32_t wave = !in_place && gemm_wave_ok(g) ? gemm_wave_tile(g, &wave_us) : 0;
-    // skinny outputs: any larger tile is >90% padding.  The dW of a long batch streams X
-    // in batch slices instead (2048 x 10 fp16: 10 against 20 us at 4096 rows, 40 against
-    // 27 us at 16384).
-    if (g.N <= 16 && g.M && g.K) {
-        if (dw && g.b32 && !g.a_kcontig && (!wave || g.K > 8192)) {
-            p.skinny = true;
-            p.splits = skinny_dw_slices(g.K, g.M);
-            p.part_bytes = (size_t)p.splits * g.M * 16 * sizeof(float);
-            return p;
+    uint32_t wave_splits = dw && t128 < 160 && g.K >= 8 * gemm_bk(g.dtype) ? 16 : 1;
+    const uint32_t wave = in_place ? 0 : gemm_wave_tile(g, &wave_splits, &wave_us);
+    auto take_wave = [&] {
+        p.wave = wave;
+        if (wave_splits > 1) {
+            const uint32_t slice = gemm_wave_slice(g.K, wave_splits);
+            p.splits = (g.K + slice - 1) / slice;
+            // planes on 16-byte boundaries, rows without padding
+            if (p.splits > 1) p.part_bytes = (size_t)p.splits * (((uint64_t)g.M * g.N + 3) & ~3ull) * sizeof(float);
         }
-        if (wave) {
-            p.wave = wave;
-            return p;
-        }
+    };
+    // outputs of at most 16 columns: any larger tile is >90% padding
+    if (g.N <= 16 && wave) {
+        take_wave();
+        return p;
     }
     if (g.dtype == SKL_F16 && gemm_dma_enabled() && g.M && g.N && g.K) {
         const uint32_t Mp = round_up(g.M, 256), Np = round_up(g.N, 256), Kp = round_up(g.K, 128);
         // in units of 256x256 tiles whatever the kernel's tile edge
         const uint32_t tiles = (Mp / 256) * (Np / 256);
         uint32_t dw_tile = 256;
-        const uint32_t splits = dw && tiles < 160 ? dw_dma_splits(tiles, Kp, (uint64_t)Mp * Np, &dw_tile) : 1;
+        double dma_us = (tiles + 255) / 256 * (Kp / 128) * 3.4;
+        const uint32_t splits = dw && tiles < 160 ? dw_dma_splits(tiles, Kp, (uint64_t)Mp * Np, &dw_tile, &dma_us) : 1;
         const bool waste_ok = (uint64_t)Mp * Np <= (uint64_t)g.M * g.N * 3 / 2;
         // the kernel's operand offsets are 32-bit
         const uint64_t a_span = g.a_kcontig ? (uint64_t)Mp * (g.lda > Kp ? g.lda : Kp)
@@ -512,6 +520,25 @@ GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
             p.a_bytes = p.pad_a ? ((size_t)Mp * Kp * 2 + 255) & ~(size_t)255 : 0;
             p.b_bytes = p.pad_b ? ((size_t)Np * Kp * 2 + 255) & ~(size_t)255 : 0;
             p.part_bytes = splits > 1 ? (size_t)splits * Mp * Np * sizeof(float) : 0;
+            // A dW of few tiles against the K-splitting kernel, with the copies of padded
+            // operands and the optimiser's bytes: 832 x 2368 over 1640 rows takes two
+            // copies, the GEMM and a reduction, 41 us, against 25 in one launch; 2048 x 2048
+            // over 16384 rows 163 against 220.
+            if (dw && wave && !gemm_dma_tile_forced()) {
+                const double elems = (double)g.M * g.N;
+                dma_us += elems * 26.0 / 7.0e6 + (splits > 1 ? 3.0 + elems * 4.0 * splits / 4.5e6 : 0.0);
+                if (p.pad_a) dma_us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
+                if (p.pad_b) dma_us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
+                if (wave_us < 0.9 * dma_us) {
+                    p = GemmPlan{};
+                    p.tile = 256;
+                    p.splits = 1;
+                    p.Mp = g.M;
+                    p.Np = g.N;
+                    p.Kp = g.K;
+                    take_wave();
+                }
+            }
             return p;
         }
     }
@@ -526,7 +553,7 @@ GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
     }
     // grids that leave those tiles' GPU mostly idle: the K-splitting kernel
     if (wave && wave_us < staged_us(g)) {
-        p.wave = wave;
+        take_wave();
         return p;
     }
     // register-staged kernels; split-K for small dW grids
@@ -536,7 +563,6 @@ GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
         // fp32: 128x128 tiles split over the batch rather than the 64x64 tiles a
         // small grid would otherwise get (C2's 1024 x 1024 dW over 4096 rows: 4
         // slices of 64 tiles, 103 -> 77 us, against 256 whole 64x64 tiles)
-        const uint32_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128);
         if (g.dtype == SKL_F32 && t128 < 160 && g.K >= 8 * 4 * bk) {
             tiles = t128;
             p.tile = 128;
@@ -555,12 +581,11 @@ GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
     return p;
 }
 
-enum class GemmKind { Dma, Staged, Wave, SkinnyDw };
+enum class GemmKind { Dma, Staged, Wave };
 
 // One GEMM launch; when skl_ctx_time_next_gemm armed a pair of events, the GEMM
 // kernel's own dispatch records them (no marker packets in the stream).
-hipError_t timed_gemm(skl_ctx *ctx, const GemmLaunch &g0, GemmKind kind, float *partials = nullptr,
-                      uint32_t slices = 0) {
+hipError_t timed_gemm(skl_ctx *ctx, const GemmLaunch &g0, GemmKind kind) {
     GemmLaunch g = g0;
     g.time_start = ctx->gemm_start;
     g.time_stop = ctx->gemm_stop;
@@ -569,7 +594,6 @@ hipError_t timed_gemm(skl_ctx *ctx, const GemmLaunch &g0, GemmKind kind, float *
     case GemmKind::Dma: return launch_gemm_dma(g, ctx->stream);
     case GemmKind::Staged: return launch_gemm(g, ctx->stream);
     case GemmKind::Wave: return launch_gemm_wave(g, ctx->stream);
-    case GemmKind::SkinnyDw: return launch_skinny_dw(g, partials, slices, ctx->stream);
     }
     return hipSuccess;
 }
@@ -590,7 +614,13 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
     const uint32_t M = g.M, N = g.N;
     if (p.wave) {
         g.tile = p.wave;
-        if (vec && g.op == Op::DwOpt) {
+        if (p.splits > 1) {
+            g.op = Op::DwPartial;
+            g.splits = p.splits;
+            g.st.out = reinterpret_cast<float *>(wpart);
+            g.st.split_stride = ((uint64_t)M * N + 3) & ~3ull;
+            g.st.ldc = N;
+        } else if (vec && g.op == Op::DwOpt) {
             // the bias / norm-parameter update rides in the launch (columns per workgroup
             // for 256 threads; the launcher scales them to its own)
             g.opt.vec = *vec;
@@ -598,28 +628,8 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
             g.opt.vec_blocks = 1;
             if (vec_done) *vec_done = true;
         }
-        return hip_status(timed_gemm(ctx, g, GemmKind::Wave));
-    }
-    if (p.skinny) {
-        SKL_TRY(timed_gemm(ctx, g, GemmKind::SkinnyDw, reinterpret_cast<float *>(wpart), p.splits));
-        DwReduceArgs d{};
-        d.dtype = g.dtype;
-        d.rows = M;
-        d.n = N;
-        d.splits = p.splits;
-        d.partials = reinterpret_cast<const float *>(wpart);
-        d.plane = (uint64_t)M * 16;
-        d.pld = 16;
-        d.e = oe;
-        if (vec) {
-            d.with_vec = 1;
-            d.vec = *vec;
-        }
-        SKL_TRY(launch_dw_reduce_opt(d, ctx->stream));
-        if (vec_done) *vec_done = vec != nullptr;
-        return SKL_OK;
-    }
-    if (p.dma) {
+        SKL_TRY(timed_gemm(ctx, g, GemmKind::Wave));
+    } else     if (p.dma) {
         // a d_prenorm_h padded by the GEMM before (or padded now into a kept slot),
         // else a padded copy in the workspace
         if (p.pad_a) {
@@ -722,7 +732,7 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
         d.n = N;
         d.splits = p.splits;
         d.partials = reinterpret_cast<const float *>(wpart);
-        d.plane = p.dma ? (uint64_t)p.Mp * p.Np : (uint64_t)M * N;
+        d.plane = p.dma ? (uint64_t)p.Mp * p.Np : p.wave ? g.st.split_stride : (uint64_t)M * N;
         d.pld = p.dma ? p.Np : N;
         d.e = oe;
         if (vec) {
@@ -1334,7 +1344,6 @@ static int32_t backward_impl(skl_ctx *ctx, const skl_dense_desc *b, const void *
     g.b_kcontig = false;
     g.A = in;
     g.B = f16 ? b->d_prenorm_h : b->d_prenorm;
-    g.b32 = b->d_prenorm;
     g.splits = 1;
     g.op = Op::DwOpt;
     g.opt = oe;

@@ -1744,6 +1744,18 @@ hipError_t launch_vec_opt(const VecOptArgs &a0, hipStream_t s) {
 // Grid: 1-D, blocks [0, a.vec_blocks) run the bias / norm-parameter update of
 // a.vec (vec_opt_block; independent of W), the next blocks the reduction: block
 // gx * y + x, or for narrow outputs (gx = 0) one thread per element of the gy.
+// FLAT (launcher): planes without row padding whose rows are not 4-element groups go as one
+// row of all elements, so that every access is 16 bytes whatever n is (777 x 1531, 5 planes:
+// an element per thread took 27 us).
+template <typename T> __device__ __forceinline__ float reduced(const DwReduceArgs &a, uint32_t r, uint32_t c, float v) {
+    if constexpr (sizeof(T) == 2) {
+        if (__builtin_expect(!__builtin_isfinite(v), 0) && a.flat_n) {
+            r = c / a.flat_n;
+            c -= r * a.flat_n;
+        }
+    }
+    return dw_checked<T>(a.e, r, c, v);
+}
 template <typename T, int VW> __global__ void __launch_bounds__(256) dw_reduce_opt_kernel(DwReduceArgs a, uint32_t gx,
                                                                                          uint32_t gy) {
     if (blockIdx.x < a.vec_blocks) {
@@ -1797,7 +1809,7 @@ template <typename T, int VW> __global__ void __launch_bounds__(256) dw_reduce_o
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 float pj = p[j], vj = dv[j], mj = dm[j];
-                const float gj = dw_checked<T>(e, r, c + j, sum[j]);
+                const float gj = reduced<T>(a, r, c + j, sum[j]);
                 optimiser_step<sizeof(T) == 2>(pj, vj, mj, gj * kLossScaleInv, e.inv_m, e.lr, e.clamp, e.opt,
                                                e.regularisation, e.regu_coeff, true);
                 p[j] = pj;
@@ -1806,7 +1818,7 @@ template <typename T, int VW> __global__ void __launch_bounds__(256) dw_reduce_o
             }
             if (e.param) store4<T>(e.param, idx, p);
         } else {
-            const float g = dw_checked<T>(e, r, c, sum);
+            const float g = reduced<T>(a, r, c, sum);
             optimiser_step<sizeof(T) == 2>(p, dv, dm, g * kLossScaleInv, e.inv_m, e.lr, e.clamp, e.opt,
                                            e.regularisation, e.regu_coeff, true);
             if (e.param) stv<T>(e.param, idx, from_f32<T>(p));
@@ -1819,7 +1831,14 @@ template <typename T, int VW> __global__ void __launch_bounds__(256) dw_reduce_o
 
 static bool aligned_to(const void *p, uintptr_t b) { return (reinterpret_cast<uintptr_t>(p) & (b - 1)) == 0; }
 
-template <typename T> static void launch_dw_reduce_t(const DwReduceArgs &a, hipStream_t s) {
+template <typename T> static void launch_dw_reduce_t(const DwReduceArgs &a0, hipStream_t s) {
+    DwReduceArgs a = a0;
+    const uint64_t all = (uint64_t)a.rows * a.n;
+    if (a.n % 4 != 0 && a.pld == a.n && all % 4 == 0 && all < (1ull << 31)) {
+        a.flat_n = a.n;
+        a.rows = 1;
+        a.n = a.pld = (uint32_t)all;
+    }
     const bool vec = a.n % 4 == 0 && a.pld % 4 == 0 && a.plane % 4 == 0 && aligned_to(a.partials, 16) &&
                      aligned_to(a.e.master, 16) && aligned_to(a.e.dv, 16) && aligned_to(a.e.dm, 16) &&
                      (!a.e.param || aligned_to(a.e.param, 4 * sizeof(T)));

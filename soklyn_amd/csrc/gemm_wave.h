@@ -467,13 +467,14 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WPE
     const uint32_t m0 = tm * BM, n0 = tn * BN;
     const uint32_t kbeg = blockIdx.y * sh.k_per_split;
     const uint32_t kend = min(sh.K, kbeg + sh.k_per_split);
-    const uint32_t kt0 = kbeg / BKE + wave, kt1 = (kend + BKE - 1) / BKE;
+    const uint32_t kt0 = wave, kt1 = (kend - kbeg + BKE - 1) / BKE;   // k-tiles of the slice
 
     const uint32_t lds0 = (uint32_t)(uintptr_t)lsm + wave * (S * STAGE);
     OA oa;
     OB ob;
-    oa.init(A, sh.lda, sh.M, sh.K, m0, lane, lds0);
-    ob.init(B, sh.ldb, sh.N, sh.K, n0, lane, lds0 + BM * 128);
+    // m/n-contiguous operands start at the slice's first k-row (only dW, with both, is split)
+    oa.init(A_KC ? A : A + (uint64_t)kbeg * sh.lda, sh.lda, sh.M, A_KC ? sh.K : kend - kbeg, m0, lane, lds0);
+    ob.init(B_KC ? B : B + (uint64_t)kbeg * sh.ldb, sh.ldb, sh.N, B_KC ? sh.K : kend - kbeg, n0, lane, lds0 + BM * 128);
 
     floatx4 acc[MB][NB];
 #pragma unroll

@@ -106,28 +106,26 @@ struct GemmLaunch {
     OptEpi opt;
     StoreEpi st;
     ErrEpi err;
-    const float *b32;     // dW: fp32 d_prenorm (ld N), read by the skinny kernel instead of B
     // When set, the GEMM kernel's own dispatch records these events at its start
     // and end (hipExtLaunchKernelGGL: no marker packets between kernels).
     hipEvent_t time_start, time_stop;
 };
 
 hipError_t launch_gemm(const GemmLaunch &g, hipStream_t stream);
-// Skinny outputs (N <= 16) of a long batch: batch-sliced partial sums of X^T . d_prenorm
-// (fp32) into partials [slices x K x 16]; skinny_dw_slices gives the slice count.
-uint32_t skinny_dw_slices(uint32_t rows, uint32_t K);
-hipError_t launch_skinny_dw(const GemmLaunch &g, float *partials, uint32_t slices, hipStream_t stream);
 // The 256x256 direct-to-LDS kernel on operands that fit it (gemm_dma_shape_ok):
 // M, N whole 256 tiles (zero-padded copies allowed: the epilogue stops at mv, nv),
 // K a multiple of 128; DwPartial may split K into g.splits slices.
 hipError_t launch_gemm_dma(const GemmLaunch &g, hipStream_t stream);
 bool gemm_dma_shape_ok(const GemmLaunch &g);
 // The K-splitting kernel (gemm_wave.h) on output tiles of edge g.tile (16, 32 or 64): any
-// M, N, K >= 1, operands as stored.  gemm_wave_tile picks the tile and estimates its time.
+// M, N, K >= 1, operands as stored; DwPartial in g.splits slices of gemm_wave_slice k.
+// gemm_wave_tile picks the tile, and for a dW up to *splits slices, and estimates its time
+// (0: the kernel does not take the operands).
 hipError_t launch_gemm_wave(const GemmLaunch &g, hipStream_t stream);
-bool gemm_wave_ok(const GemmLaunch &g);
+bool gemm_wave_ok(const GemmLaunch &g, uint32_t splits);
 bool wave_dword_rows(const GemmLaunch &g);
-uint32_t gemm_wave_tile(const GemmLaunch &g, double *us);
+uint32_t gemm_wave_slice(uint32_t K, uint32_t splits);
+uint32_t gemm_wave_tile(const GemmLaunch &g, uint32_t *splits, double *us);
 bool gemm_dma_enabled();
 // Output tile edge of the direct-to-LDS kernel forced by SOKLYN_GEMM_TILE (128 or
 // 256), or 0: the planner picks per GEMM.
@@ -212,7 +210,8 @@ struct DwReduceArgs {
     uint32_t dtype, rows, n, splits;
     const float *partials;         // split sp, element (r, c) at sp * plane + r * pld + c
     uint64_t plane;
-    uint32_t pld, pad;
+    uint32_t pld;
+    uint32_t flat_n;               // set by the launcher: rows = 1, n all elements of rows of flat_n
     OptEpi e;
     // with_vec: the same launch also runs launch_vec_opt(vec) (the bias / norm-
     // parameter update, independent of W) in its first workgroups

@@ -23,6 +23,7 @@ SHAPES = [  # batch, inputs, outputs
     (70, 77, 200), (130, 36, 12), (20, 4100, 10), (257, 520, 136),
     (700, 72, 900), (515, 330, 902), (701, 129, 835),      # 64x64 tiles
     (1700, 40, 2000), (2500, 33, 2560), (2000, 1700, 40),  # fewer waves per tile
+    (3001, 200, 96), (4100, 61, 35), (5000, 130, 10), (2053, 40, 3),   # dW in batch slices
 ]
 
 
