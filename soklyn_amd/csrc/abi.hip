@@ -326,6 +326,7 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 struct GemmPlan {
     uint32_t wave;             // K-splitting kernel: its tile edge (0: another kernel)
     bool dma;
+    bool rag;                  // direct-to-LDS on operands as stored, 128x128 tiles
     bool pad_a, pad_b;
     uint32_t tile;             // direct-to-LDS output tile edge (128 or 256); 128: fp32 dW on 128x128 tiles
     uint32_t band;             // > 0: rows [0, band) on 256x256 tiles, the rest on 128x128 (two launches)
@@ -448,13 +449,13 @@ double staged_us(const GemmLaunch &g) {
     return vec ? 10.0 + kt * (u > 1.25 ? 0.8 * u : 1.0) : 15.0 + kt * (u > 1.0 ? 4.0 * u : 4.0);
 }
 
-// The same for 128x128 direct-to-LDS tiles on a grid short of the 256x256 kernel's, whose
-// operands it reads in place (2048 x 2048, K 2048: 29.4 us, 33 on the K-splitting kernel;
-// 4096 x 2048: 42, 56; dX of 4096 x 1024, K 1024: 14.6, 16.5).  Not the dW, whose fused
-// optimiser is faster on small tiles (2048 x 2048 over 512 rows: 31, 25).
+// The same for 128x128 direct-to-LDS tiles, whose operands are read in place (2048 x 2048,
+// K 2048: 29.4 us, 33 on the K-splitting kernel; 4096 x 2048: 42, 56; dX of 4096 x 1024,
+// K 1024: 14.6, 16.5).  Not the dW, whose fused optimiser is faster on small tiles (2048 x
+// 2048 over 512 rows: 31, 25).
 double dma128_us(const GemmLaunch &g) {
-    const double u = (double)(g.M / 128) * (g.N / 128) / 256.0, kt = g.K / 64.0;
-    return (g.op == Op::InputGrad ? 4.5 : 8.5) + kt * (0.33 + 0.32 * (u > 1.0 ? u : 1.0));
+    const double u = (double)((g.M + 127) / 128) * ((g.N + 127) / 128) / 256.0, kt = (double)((g.K + 63) / 64);
+    return (g.op == Op::InputGrad ? 4.5 : 8.5) + kt * (0.5 * u > 0.65 ? 0.5 * u : 0.65);
 }
 
 // in_place: the output overlaps an operand (a caller's dx over d_prenorm).  The K-splitting
@@ -539,14 +540,30 @@ GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
                     take_wave();
                 }
             }
+            // padded copies against the operands as stored on 128x128 tiles
+            if (!dw && !in_place && (p.pad_a || p.pad_b) && gemm_dma_rag_ok(g) && !gemm_dma_tile_forced()) {
+                double us = 8.0 + std::ceil(tiles / 256.0) * (Kp / 128) * 3.2;
+                if (p.pad_a) us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
+                if (p.pad_b) us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
+                if (1.1 * dma128_us(g) < us) {
+                    p = GemmPlan{};
+                    p.dma = p.rag = true;
+                    p.tile = 128;
+                    p.splits = 1;
+                    p.Mp = g.M;
+                    p.Np = g.N;
+                    p.Kp = g.K;
+                }
+            }
             return p;
         }
     }
-    if (g.dtype == SKL_F16 && !dw && !in_place && (g.M % 256) == 0 && (g.N % 256) == 0 && gemm_dma_shape_ok(g) &&
-        !gemm_dma_tile_forced()) {
-        const double us = dma128_us(g);
-        if ((!wave || us < wave_us) && us < staged_us(g)) {
+    if (g.dtype == SKL_F16 && !dw && !in_place && !gemm_dma_tile_forced()) {
+        const bool whole = g.M % 256 == 0 && g.N % 256 == 0 && gemm_dma_shape_ok(g);
+        const double us = whole ? dma128_us(g) : 1.1 * dma128_us(g);
+        if ((whole || gemm_dma_rag_ok(g)) && (!wave || us < wave_us) && us < staged_us(g)) {
             p.dma = true;
+            p.rag = !whole;
             p.tile = 128;
             return p;
         }
@@ -673,6 +690,7 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
         g.mv = full_out ? p.Mp : M;
         g.nv = full_out ? p.Np : N;
         g.tile = p.tile;
+        g.rag = p.rag;
         if (vec && g.op == Op::DwOpt && p.splits == 1) {
             // the bias / norm-parameter update rides in the fused kernel's launch;
             // its 64 NW threads take cpb columns each with the lanes per column of a
@@ -1233,7 +1251,7 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     e.leaky = cur->act == SKL_ACT_LEAKY_RELU ? cur->leaky : 0.0f;
     e.inv_n = 1.0f / (float)cur->outputs;
     e.inv_m = 1.0f / (float)batch;
-    if (plan.dma && hidden_err_fusable(e, batch, cur->outputs)) {
+    if (plan.dma && !plan.rag && hidden_err_fusable(e, batch, cur->outputs)) {
         // One kernel, as the reference has it (backward.cu:59-102): the 256x256
         // GEMM's epilogue computes the error from the sum in its accumulators
         // and leaves the column sums of each 256-row tile for cur's backward.

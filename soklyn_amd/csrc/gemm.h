@@ -53,6 +53,7 @@ struct GemmShape {
     uint32_t tiles_m, tiles_n;
     uint32_t mv, nv;         // 256x256 kernel on zero-padded operands: the real output extent
     uint32_t m_base;         // direct-to-LDS kernel: first output row of the launch's tiles
+    uint32_t whole;          // its bounded form: output rows allow the vector epilogue
 };
 
 // Workgroup barrier that orders LDS only: wait for this wave's LDS accesses,

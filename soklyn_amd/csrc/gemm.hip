@@ -249,7 +249,51 @@ static hipError_t run_dma(const GemmLaunch &g, const typename Epi::Params &p, ui
     return run_dma_t<Epi, AK, BK_, 8, AK ? 16 : 32, 256>(g, p, splits, kps, s);
 }
 
+// The 128x128 kernel on operands as stored: fp16 forward and input gradient, K whole
+// 16-byte chunks (it is contiguous in A), rows and bases on 4-byte boundaries, byte offsets
+// below 2 GiB with the tiles and k-tiles past the ends.
+bool gemm_dma_rag_ok(const GemmLaunch &g) {
+    if (!gemm_dma_enabled() || g.dtype != 1 || (g.op != Op::Fwd && g.op != Op::InputGrad) || !dma_layout_ok(g))
+        return false;
+    auto dword = [](const void *p, uint32_t ld) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0 && ld % 2 == 0; };
+    const uint64_t a_rows = g.M + 256ull, b_rows = g.b_kcontig ? g.N + 256ull : g.K + 512ull;
+    return g.M && g.N && g.K && g.K % 8 == 0 && dword(g.A, g.lda) && dword(g.B, g.ldb) &&
+           a_rows * g.lda * 2 < (1ull << 31) && b_rows * g.ldb * 2 < (1ull << 31);
+}
+
+template <class Epi, bool B_KC> static hipError_t run_dma_rag(const GemmLaunch &g, const typename Epi::Params &p,
+                                                             bool whole, hipStream_t s) {
+    GemmShape sh{};
+    sh.M = g.M;
+    sh.N = g.N;
+    sh.K = g.K;
+    sh.lda = g.lda;
+    sh.ldb = g.ldb;
+    sh.k_per_split = (g.K + 127) / 128 * 128;
+    sh.tiles_m = (g.M + 127) / 128;
+    sh.tiles_n = (g.N + 127) / 128;
+    sh.mv = g.M;
+    sh.nv = g.N;
+    sh.whole = whole;
+    launch_timed(g, gemm_dma_kernel<Epi, true, B_KC, 4, true, 16, 128, true>, dim3(sh.tiles_m * sh.tiles_n), dim3(256), s,
+                 sh, reinterpret_cast<const half_t *>(g.A), reinterpret_cast<const half_t *>(g.B), p);
+    return hipGetLastError();
+}
+
+static hipError_t launch_dma_rag(const GemmLaunch &g, hipStream_t s) {
+    if (!gemm_dma_rag_ok(g)) return hipErrorInvalidValue;
+    if (g.op == Op::Fwd) {
+        // 8-column, 16-byte stores of the caches
+        const FwdEpi &e = g.fwd;
+        const bool whole = e.ldc % 8 == 0 && aligned16(e.bias) && aligned16(e.z_out) &&
+                           (!e.fuse_act || (aligned16(e.predrop) && aligned16(e.out) && (!e.use_dropout || aligned16(e.mask))));
+        return g.b_kcontig ? hipErrorInvalidValue : run_dma_rag<EpiFwdK<half_t>, false>(g, e, whole, s);
+    }
+    return run_dma_rag<EpiStoreK, true>(g, g.st, g.st.ldc % 4 == 0 && aligned16(g.st.out), s);
+}
+
 hipError_t launch_gemm_dma(const GemmLaunch &g, hipStream_t s) {
+    if (g.rag) return launch_dma_rag(g, s);
     if (!gemm_dma_shape_ok(g)) return hipErrorInvalidValue;
     // split-K: slices of k_per_split (a multiple of 128), the last one possibly shorter
     const uint32_t splits_req = g.splits ? g.splits : 1;

@@ -129,6 +129,12 @@ struct DmaSrc {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, reinterpret_cast<__attribute__((address_space(3))) void *>(dst),
                                                  16, (int)voff, (int)add, 0, 0);
     }
+    // at the lane's own byte offset `off`, all of it range-checked (the scalar offset of
+    // load() is not): dwords past the resource's end read as zero
+    __device__ __forceinline__ void load_at(uint32_t off, lds_char *dst) const {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, reinterpret_cast<__attribute__((address_space(3))) void *>(dst),
+                                                 16, (int)off, 0, 0, 0);
+    }
 };
 
 // s_waitcnt with only one counter constrained (gfx9 encoding: vmcnt[3:0] +
@@ -164,7 +170,7 @@ __device__ __forceinline__ void pin(u32x2 &v) { asm volatile("" : "+v"(v)); }
 // chunks of 8 halves, chunk c of row r stored at slot c ^ ((r >> 1) & 7): any
 // 16 consecutive rows of one chunk column hit 16 distinct 16-byte bank groups.
 // A fragment is one ds_read_b128.
-template <int NW, int NF, int MI = 32, int ROWS = 256> struct OpK {
+template <int NW, int NF, int MI = 32, int ROWS = 256, bool RAG = false> struct OpK {
     static constexpr int IPO = ROWS / 8 / NW;   // DMA instructions per tile and wave
     static constexpr uint32_t CPK = 512 / MI / 8;   // 16-byte chunks of a row per k-step
     struct Frag { u32x4 v[NF]; };
@@ -172,14 +178,20 @@ template <int NW, int NF, int MI = 32, int ROWS = 256> struct OpK {
     uint32_t step;                    // bytes between DMA instructions (8 NW rows)
     uint32_t lds;                     // LDS byte address of this lane's fragment row, stage 0
     uint32_t g;                       // swizzle term of the fragment row
+    uint32_t kc, chunks;              // RAG: this lane's chunk of a tile's row, chunks of the operand's rows
 
-    __device__ __forceinline__ void init(const half_t *p, uint32_t ld, uint32_t rows, uint32_t mn0, uint32_t wbase,
-                                         uint32_t wave, uint32_t lane, uint32_t lds_op) {
+    // k: length of a row (RAG)
+    __device__ __forceinline__ void init(const half_t *p, uint32_t ld, uint32_t rows, uint32_t k, uint32_t mn0,
+                                         uint32_t wbase, uint32_t wave, uint32_t lane, uint32_t lds_op) {
         // instruction t fills rows 8 (NW t + wave) .. + 7; lane -> row + lane / 8, slot lane % 8;
         // (row >> 1) & 7 does not depend on t (8 NW t >> 1 is a multiple of 8)
         const uint32_t row0 = 8u * wave + (lane >> 3);
-        const uint32_t kc = (lane & 7u) ^ ((row0 >> 1) & 7u);
-        dma.init(p, rows * ld * 2u, (mn0 + row0) * ld * 2u + kc * 16u);
+        kc = (lane & 7u) ^ ((row0 >> 1) & 7u);
+        chunks = k / 8u;
+        if constexpr (RAG)
+            dma.init(p, ((rows - 1u) * ld + k) * 2u, (mn0 + row0) * ld * 2u);
+        else
+            dma.init(p, rows * ld * 2u, (mn0 + row0) * ld * 2u + kc * 16u);
         step = 8u * NW * ld * 2u;
         // wbase is a multiple of 32: the fragment row's swizzle is that of lane % MI
         const uint32_t frow = lane % MI;
@@ -187,7 +199,12 @@ template <int NW, int NF, int MI = 32, int ROWS = 256> struct OpK {
         lds = lds_op + (wbase + frow) * 128u;
     }
     __device__ __forceinline__ void issue(int kt, int t, lds_char *dst) const {
-        dma.load((uint32_t)kt * 128u + t * step, dst + t * (NW * 1024u));
+        if constexpr (RAG) {
+            const uint32_t c = (uint32_t)kt * 8u + kc;
+            dma.load_at(c < chunks ? dma.voff + t * step + c * 16u : 0x80000000u, dst + t * (NW * 1024u));
+        } else {
+            dma.load((uint32_t)kt * 128u + t * step, dst + t * (NW * 1024u));
+        }
     }
     // fragment i: logical chunk CPK ks + lane / MI of row MI i + lane % MI (the
     // two terms have disjoint bits, so the swizzle XOR applies to them apart)
@@ -223,7 +240,7 @@ template <int NW, int NF, int MI = 32, int ROWS = 256> struct OpK {
 // 4 distinct 64-byte bank windows.  Fragment i of the wave sits 32 rows
 // further on: chunk + 4 i, i.e. the lane's address XOR 64 i (the wave's first
 // row is a multiple of 32 NF, so the chunk bits that i flips start clear).
-template <int NW, int NF, int MI = 32, int COLS = 256> struct OpN {
+template <int NW, int NF, int MI = 32, int COLS = 256, bool RAG = false> struct OpN {
     static constexpr uint32_t P = 2u * COLS;             // bytes per LDS k-row
     static constexpr uint32_t LPR = P / 16u;             // DMA lanes per k-row
     static constexpr uint32_t RPI = 64u / LPR;           // k-rows per DMA instruction
@@ -241,8 +258,9 @@ template <int NW, int NF, int MI = 32, int COLS = 256> struct OpN {
         return (4u * (r & 3u)) ^ (MI == 16 ? 2u * ((r >> 3) & 1u) : 0u);
     }
 
-    __device__ __forceinline__ void init(const half_t *p, uint32_t ld, uint32_t rows, uint32_t mn0, uint32_t wbase,
-                                         uint32_t wave, uint32_t lane, uint32_t lds_op_) {
+    // cols: length of a k-row (RAG)
+    __device__ __forceinline__ void init(const half_t *p, uint32_t ld, uint32_t rows, uint32_t cols, uint32_t mn0,
+                                         uint32_t wbase, uint32_t wave, uint32_t lane, uint32_t lds_op_) {
         // instruction t (q = wave + NW t) fills k-rows RPI q .. RPI q + RPI - 1; lane -> k-row
         // RPI q + lane / LPR, slot lane % LPR; r & 3 does not depend on t (NW is even), (r >> 3) & 1
         // at most on t's parity
@@ -250,7 +268,7 @@ template <int NW, int NF, int MI = 32, int COLS = 256> struct OpN {
         for (uint32_t t = 0; t < 2; ++t) {
             const uint32_t r = RPI * (wave + NW * t) + lane / LPR;
             const uint32_t cl = (lane % LPR) ^ swz(r);
-            dma[t].init(p, rows * ld * 2u, (RPI * wave + lane / LPR) * ld * 2u + mn0 * 2u + cl * 16u);
+            dma[t].init(p, RAG ? (((rows - 1u) * ld + cols) * 2u + 3u) & ~3u : rows * ld * 2u, (RPI * wave + lane / LPR) * ld * 2u + mn0 * 2u + cl * 16u);
         }
         step = RPI * NW * ld * 2u;
         kstep = 64u * ld * 2u;
@@ -267,7 +285,10 @@ template <int NW, int NF, int MI = 32, int COLS = 256> struct OpN {
         lds_op = lds_op_;
     }
     __device__ __forceinline__ void issue(int kt, int t, lds_char *dst) const {
-        dma[t & 1].load((uint32_t)kt * kstep + t * step, dst + t * (NW * 1024u));
+        if constexpr (RAG)
+            dma[t & 1].load_at(dma[t & 1].voff + (uint32_t)kt * kstep + t * step, dst + t * (NW * 1024u));
+        else
+            dma[t & 1].load((uint32_t)kt * kstep + t * step, dst + t * (NW * 1024u));
     }
     // fragment i sits MI rows further on: the lane's offset XOR 2 MI i; k-rows
     // KSTEP ks + 4 h (+ 8 g) at offsets KSB ks + 2048 h keep the swizzle
@@ -346,23 +367,30 @@ template <class E, int NW> struct EpiReadsPerMfma<E, NW, std::void_t<decltype(E:
     static constexpr int value = E::kReadsPerMfma;
 };
 
-template <bool KC, int NW, int NF, int MI, int R> struct DmaOpSel { typedef OpK<NW, NF, MI, R> type; };
-template <int NW, int NF, int MI, int R> struct DmaOpSel<false, NW, NF, MI, R> { typedef OpN<NW, NF, MI, R> type; };
+template <bool KC, int NW, int NF, int MI, int R, bool RAG> struct DmaOpSel { typedef OpK<NW, NF, MI, R, RAG> type; };
+template <int NW, int NF, int MI, int R, bool RAG> struct DmaOpSel<false, NW, NF, MI, R, RAG> {
+    typedef OpN<NW, NF, MI, R, RAG> type;
+};
 
 // Grid: (tiles, splits); each workgroup takes one (tile, split) pair (split-K grids
 // remap the pairs onto the XCDs, below).  Split y reduces k in [y k_per_split,
 // (y + 1) k_per_split) (k_per_split a multiple of 128; the last split may be
 // shorter, also a multiple of 128).  EDGE: the operands are zero-padded copies whose M, N
 // extend past the real output [mv x nv]; the epilogue then goes element by
-// element through Epi::apply with those bounds (any leading dimension).
-template <class Epi, bool A_KC, bool B_KC, int NW, bool EDGE, int MI = 32, int BT = 256>
+// element through Epi::apply1 with those bounds (any leading dimension).  RAG: the operands
+// are read as stored, whatever M, N and K are (K a multiple of 8 where it is contiguous,
+// rows on 4-byte boundaries): rows past an operand's end and k past K read as zero by the
+// resource's range check, columns past a row's end only reach outputs that are not stored;
+// only tiles that reach past the output go element by element.
+template <class Epi, bool A_KC, bool B_KC, int NW, bool EDGE, int MI = 32, int BT = 256, bool RAG = false>
 __global__ void __launch_bounds__(64 * NW)
     __attribute__((amdgpu_waves_per_eu(DmaCfg<NW, MI, BT, BT>::WPE, DmaCfg<NW, MI, BT, BT>::WPE)))
     gemm_dma_kernel(GemmShape sh, const half_t *__restrict__ A, const half_t *__restrict__ B,
                     typename Epi::Params ep) {
     typedef DmaCfg<NW, MI, BT, BT> C;
-    typedef typename DmaOpSel<A_KC, NW, C::MT, MI, C::BM>::type OA;
-    typedef typename DmaOpSel<B_KC, NW, C::NTL, MI, C::BN>::type OB;
+    typedef typename DmaOpSel<A_KC, NW, C::MT, MI, C::BM, RAG>::type OA;
+    typedef typename DmaOpSel<B_KC, NW, C::NTL, MI, C::BN, RAG>::type OB;
+    static_assert(!RAG || (EDGE && BT == 128), "operands as stored: 128x128 tiles with bounds");
     typedef DmaMma<MI> MM;
     static_assert(C::KS % 2 == 0, "k-steps alternate between two fragment sets");
     constexpr int EPITCH = C::BN + 4;
@@ -402,13 +430,13 @@ __global__ void __launch_bounds__(64 * NW)
     const uint32_t m0 = sh.m_base + tm * C::BM, n0 = tn * C::BN;
     const uint32_t kbeg = split * sh.k_per_split;
     const int kb = (int)(kbeg / C::BK);                                  // first k-tile of this split
-    const int nk = (int)((min(sh.K, kbeg + sh.k_per_split) - kbeg) / C::BK);
+    const int nk = (int)((min(sh.K, kbeg + sh.k_per_split) - kbeg + (RAG ? C::BK - 1 : 0)) / C::BK);
 
     const uint32_t lds0 = (uint32_t)(uintptr_t)lsm;   // LDS byte address of smem
     OA oa;
     OB ob;
-    oa.init(A, sh.lda, A_KC ? sh.M : sh.K, m0, wm * C::TWM, wave, lane, lds0);
-    ob.init(B, sh.ldb, B_KC ? sh.N : sh.K, n0, wn * C::TWN, wave, lane, lds0 + C::OPA);
+    oa.init(A, sh.lda, A_KC ? sh.M : sh.K, A_KC ? sh.K : sh.M, m0, wm * C::TWM, wave, lane, lds0);
+    ob.init(B, sh.ldb, B_KC ? sh.N : sh.K, B_KC ? sh.K : sh.N, n0, wn * C::TWN, wave, lane, lds0 + C::OPA);
 
     auto issue = [&](int kt, int stage) {
         lds_char *st = lsm + stage * C::STAGEB + wave * 1024u;
@@ -500,7 +528,9 @@ __global__ void __launch_bounds__(64 * NW)
         }
     };
 
-    const int klast = kb + nk - 1;
+    // the last refills fetch the final k-tile again, never read; RAG: tiles past the end,
+    // zeros (one of them is read when nk is odd)
+    const int klast = RAG ? 0x7fffffff : kb + nk - 1;
     if constexpr (MI == 16 && !AGPR_ASM) {
         // 16x16x32: A fragments single-buffered, B double-buffered.  A fragment i
         // of the next k-step is read in place right after row i's MFMAs (its last
@@ -544,7 +574,7 @@ __global__ void __launch_bounds__(64 * NW)
         issue(kb, 0);
         wait_vmcnt<0>();
         __builtin_amdgcn_s_barrier();
-        issue(kb + (nk > 1 ? 1 : 0), 1);
+        issue(kb + (RAG || nk > 1 ? 1 : 0), 1);
 #pragma unroll
         for (int j = 0; j < C::NTL; ++j) ob.read_frag(fb[0], 0, 0, j);
 #pragma unroll
@@ -583,7 +613,7 @@ __global__ void __launch_bounds__(64 * NW)
     issue(kb, 0);
     wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
-    issue(kb + (nk > 1 ? 1 : 0), 1);
+    issue(kb + (RAG || nk > 1 ? 1 : 0), 1);
     read(0, 0, 0);
 
     for (int kt0 = 0; kt0 < nk; kt0 += 2) {
@@ -684,7 +714,9 @@ __global__ void __launch_bounds__(64 * NW)
     shv.M = sh.mv;
     shv.N = sh.nv;
     const typename Epi::Params eps = Epi::at_split(ep, split);
-    const typename Epi::Col col = EDGE ? typename Epi::Col{} : Epi::column(eps, n0 + c);
+    // RAG: this tile lies inside the output and its rows are whole vectors
+    const bool whole = !EDGE || (RAG && m0 + C::BM <= shv.M && n0 + C::BN <= shv.N && sh.whole);
+    const typename Epi::Col col = whole ? Epi::column(eps, n0 + c) : typename Epi::Col{};
     // EDGE: lane l's columns n0 + l + 64 q, their per-column operands loaded once
     constexpr int EQ = C::BN / 64;
     typename Epi::Col1 col1[EQ];
@@ -719,7 +751,7 @@ __global__ void __launch_bounds__(64 * NW)
             }
         }
         lds_barrier();
-        if constexpr (EDGE) {
+        if constexpr (EDGE) if (!whole) {
             // element by element, lane l taking columns l, l + 64, ... of the
             // row: each store instruction covers 64 consecutive columns
             // whatever the output's alignment; the per-column operands (bias)

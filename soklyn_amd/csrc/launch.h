@@ -101,6 +101,7 @@ struct GemmLaunch {
     // only (0, 0: all M), m_begin a multiple of 256 and m_rows of the tile edge;
     // not for HiddenErr, whose column sums are indexed by the tile row
     uint32_t m_begin, m_rows;
+    bool rag;             // direct-to-LDS kernel on 128x128 tiles: operands as stored, any M, N, K (gemm_dma_rag_ok)
     Op op;
     FwdEpi fwd;
     OptEpi opt;
@@ -117,6 +118,8 @@ hipError_t launch_gemm(const GemmLaunch &g, hipStream_t stream);
 // K a multiple of 128; DwPartial may split K into g.splits slices.
 hipError_t launch_gemm_dma(const GemmLaunch &g, hipStream_t stream);
 bool gemm_dma_shape_ok(const GemmLaunch &g);
+// Its form for operands as stored (128x128 tiles; forward and input gradient).
+bool gemm_dma_rag_ok(const GemmLaunch &g);
 // The K-splitting kernel (gemm_wave.h) on output tiles of edge g.tile (16, 32 or 64): any
 // M, N, K >= 1, operands as stored; DwPartial in g.splits slices of gemm_wave_slice k.
 // gemm_wave_tile picks the tile, and for a dW up to *splits slices, and estimates its time

@@ -89,6 +89,13 @@ def test_step_128(ctx):
     step(ctx, True, 2048, 1024, 2048)
 
 
+# ... and on operands as stored: ragged M and N, an odd number of k-tiles whose last is cut,
+# rows of the output that are whole vectors, 4-element groups, and neither
+@pytest.mark.parametrize("M,K,N", [(2100, 2104, 2056), (2049, 2184, 2052), (2177, 2120, 2050)])
+def test_step_ragged_128(ctx, M, K, N):
+    step(ctx, True, M, K, N)
+
+
 @pytest.mark.parametrize("norm,act,p", [(abi.NORM_RMS, abi.ACT_MISH, 0.1), (abi.NORM_BATCH, abi.ACT_TANH, 0.0)])
 def test_hidden_error_128(ctx, norm, act, p):
     fused_error(ctx, 2048, 64, 2048, 1024, norm, act, p, 0)
