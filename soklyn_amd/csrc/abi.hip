@@ -1107,9 +1107,6 @@ int32_t skl_dense_output_error(skl_ctx *ctx, const skl_dense_desc *b, const void
 
     // The reference zero-fills all dNorm rows, then writes rows [0, m).
     if ((r = zero_dnorm_tail(ctx, b, target_rows))) return r;
-    // Softmax in place on out over all cache rows (ffn_device.rs:167-186).
-    if (act == SKL_ACT_SOFTMAX) SKL_TRY(launch_softmax(b->dtype, b->out, b->max_batch, b->outputs, ctx->stream));
-
     ErrArgs a{};
     a.dtype = b->dtype;
     a.rows = target_rows;   // kernel m = max_batch (Q: ffn_device.rs:152); rows past target_rows are not readable
@@ -1134,6 +1131,16 @@ int32_t skl_dense_output_error(skl_ctx *ctx, const skl_dense_desc *b, const void
     a.d_norm_b = b->d_norm_b;
     a.d_prenorm_h = b->dtype == SKL_F16 ? reinterpret_cast<half_t *>(b->d_prenorm_h) : nullptr;
     uint32_t splits = 0;
+    if (act == SKL_ACT_SOFTMAX && softmax_ce_ok(a)) {   // softmax and cross-entropy, always together
+        splits = softmax_ce_splits(b->max_batch, b->outputs);
+        if ((r = ensure_cols_splits(ctx, splits, b->outputs))) return r;
+        note_rewrite(ctx, b);
+        SKL_TRY(launch_softmax_ce(a, b->out, b->max_batch, ctx->cols, ctx->stream));
+        record_cols(ctx, b, target_rows, splits);
+        return finish(ctx);
+    }
+    // Softmax in place on out over all cache rows (ffn_device.rs:167-186).
+    if (act == SKL_ACT_SOFTMAX) SKL_TRY(launch_softmax(b->dtype, b->out, b->max_batch, b->outputs, ctx->stream));
     if ((r = ensure_cols(ctx, b, target_rows, 0, &splits))) return r;
     note_rewrite(ctx, b);
     SKL_TRY(launch_output_error(a, ctx->cols, splits, ctx->stream));

@@ -182,6 +182,11 @@ struct ErrArgs {
 // over all rows.  splits must come from err_col_splits.
 hipError_t launch_output_error(const ErrArgs &a, float *partials, uint32_t splits, hipStream_t s);
 hipError_t launch_error_from_sum(const ErrArgs &a, float *partials, uint32_t splits, hipStream_t s);
+// The softmax of the `all` rows of out in place and the cross-entropy error of the first
+// a.rows of them in one launch; partials [softmax_ce_splits x 3 x n].
+bool softmax_ce_ok(const ErrArgs &a);
+uint32_t softmax_ce_splits(uint32_t all, uint32_t n);
+hipError_t launch_softmax_ce(const ErrArgs &a, void *out, uint32_t all, float *partials, hipStream_t s);
 // Partial-sum rows the error kernels write for [rows x n].
 uint32_t err_col_splits(uint32_t rows, uint32_t n, uint32_t resident = 0);
 // Workgroups of the flat error kernel for (dtype, src: 0 output error, 1 from
