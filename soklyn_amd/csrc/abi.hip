@@ -1271,6 +1271,16 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
         record_cols(ctx, cur, batch, tiles_m);
         return SKL_OK;
     }
+    if (plan.wave && hidden_err_wave_ok(e, cur->outputs)) {
+        // the same on the K-splitting kernel's tiles
+        const uint32_t tiles_m = (batch + plan.wave - 1) / plan.wave;
+        if ((r = ensure_cols_splits(ctx, tiles_m, cur->outputs))) return r;
+        e.partials = ctx->cols;
+        g.op = Op::HiddenErr;
+        if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws)))) return r;
+        record_cols(ctx, cur, batch, tiles_m);
+        return SKL_OK;
+    }
     // s on the kernel's whole (padded) grid: the full-tile epilogue, 16-byte rows
     const uint32_t s_ld = plan.Np;
     const size_t s_bytes = ((size_t)plan.Mp * s_ld * sizeof(float) + 255) & ~(size_t)255;

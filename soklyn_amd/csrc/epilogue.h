@@ -5,6 +5,8 @@
 
 #include <hip/hip_ext.h>
 
+#include <type_traits>
+
 #include "gemm.h"
 #include "launch.h"
 #include "vec_opt.h"
@@ -333,7 +335,8 @@ template <typename T> struct EpiErrK {
     // per-column operands of 4 columns: the norm weight, and BatchNorm's per-column rstd
     struct Col { f32x4 nw, rstd; };
     // per-element operands of one row's 4 columns, as loaded (T)
-    struct Pre { f16x4 pd, pa, mk, pn; float rstd; };
+    typedef typename std::conditional<sizeof(T) == 2, f16x4, f32x4>::type V4;
+    struct Pre { V4 pd, pa, mk, pn; float rstd; };
     // running sums of the thread's 4 columns
     struct Acc { f32x4 dp, nw, nb; };
     __device__ __forceinline__ static Col column(const ErrEpi &e, uint32_t n) {
@@ -344,15 +347,14 @@ template <typename T> struct EpiErrK {
     }
     // nontemporal: the forward caches are read once here (C4's fused hidden error
     // 0.268 -> 0.262 ms against plain loads)
-    __device__ __forceinline__ static f16x4 ld4h(const void *p, uint64_t idx) {
-        return __builtin_nontemporal_load(reinterpret_cast<const f16x4 *>(reinterpret_cast<const half_t *>(p) + idx));
+    __device__ __forceinline__ static V4 ld4(const void *p, uint64_t idx) {
+        return __builtin_nontemporal_load(reinterpret_cast<const V4 *>(reinterpret_cast<const T *>(p) + idx));
     }
     __device__ __forceinline__ static void load(const ErrEpi &e, uint64_t idx, uint32_t m, Pre &q) {
-        static_assert(sizeof(T) == 2, "the 256x256 kernel is fp16");
-        q.pd = ld4h(e.predrop, idx);
-        q.pa = ld4h(e.preact, idx);
-        q.mk = ld4h(e.mask, idx);
-        q.pn = e.norm ? ld4h(e.norm == 1 ? e.prenorm : e.centered, idx) : f16x4{0, 0, 0, 0};
+        q.pd = ld4(e.predrop, idx);
+        q.pa = ld4(e.preact, idx);
+        q.mk = ld4(e.mask, idx);
+        q.pn = e.norm ? ld4(e.norm == 1 ? e.prenorm : e.centered, idx) : V4{0, 0, 0, 0};
         q.rstd = (e.norm == 1 || e.norm == 2) ? to_f32(reinterpret_cast<const T *>(e.norm_rstd)[m]) : 0.0f;
     }
     __device__ __forceinline__ static void finish(const ErrEpi &e, uint64_t idx, uint32_t, uint32_t, floatx4 v,
@@ -373,8 +375,9 @@ template <typename T> struct EpiErrK {
         }
         __builtin_nontemporal_store(g, reinterpret_cast<f32x4 *>(e.grad + idx));
         *reinterpret_cast<f32x4 *>(e.d_prenorm + idx) = dp;
-        *reinterpret_cast<f16x4 *>(e.d_prenorm_h + idx) = f16x4{(half_t)dp[0], (half_t)dp[1], (half_t)dp[2],
-                                                                (half_t)dp[3]};
+        if constexpr (sizeof(T) == 2)
+            *reinterpret_cast<f16x4 *>(e.d_prenorm_h + idx) = f16x4{(half_t)dp[0], (half_t)dp[1], (half_t)dp[2],
+                                                                    (half_t)dp[3]};
         if (e.norm) {
             __builtin_nontemporal_store(dnw, reinterpret_cast<f32x4 *>(e.d_norm_w + idx));
             __builtin_nontemporal_store(dnb, reinterpret_cast<f32x4 *>(e.d_norm_b + idx));
@@ -383,7 +386,31 @@ template <typename T> struct EpiErrK {
         acc.nw += dnw;
         acc.nb += dnb;
     }
-    struct Col1 {};   // no element-by-element form: whole tiles only
+    struct Col1 {};   // no element-by-element form: whole 4-column groups only
+    // The tile's column sums from SLOTS threads per 4-column group (slot, group), added in slot
+    // order: writes the columns < ncols of partials[tm][k].  Every thread of the NT calls it.
+    template <int SLOTS, int BN, int NT>
+    __device__ __forceinline__ static void flush_slots(const ErrEpi &e, const Acc &acc, float *lds, uint32_t tid,
+                                                       uint32_t slot, uint32_t group, uint32_t tm, uint32_t n0) {
+        if (slot < SLOTS) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t c = 4u * group + j;
+                lds[(slot * 3 + 0) * BN + c] = acc.dp[j];
+                lds[(slot * 3 + 1) * BN + c] = acc.nw[j];
+                lds[(slot * 3 + 2) * BN + c] = acc.nb[j];
+            }
+        }
+        __syncthreads();
+        for (uint32_t t = tid; t < 3 * BN; t += NT) {
+            const uint32_t k = t / BN, c = t % BN;
+            if ((k > 0 && !e.norm) || n0 + c >= e.ncols) continue;
+            float s = 0.0f;
+#pragma unroll
+            for (uint32_t w = 0; w < SLOTS; ++w) s += lds[(w * 3 + k) * BN + c];
+            e.partials[((uint64_t)tm * 3 + k) * e.ncols + n0 + c] = s;
+        }
+    }
     // The tile's column sums: each of the NW waves leaves its 3 x 256 running sums
     // in LDS (column 4 lane + j of the tile), then the block adds the waves in
     // order 0..NW-1 and writes the columns < ncols of partials[tm][k].  lds:

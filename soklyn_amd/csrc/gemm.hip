@@ -182,6 +182,9 @@ bool hidden_err_fusable(const ErrEpi &e, uint32_t M, uint32_t N) {
     return M % 256 == 0 && N % 256 == 0 && e.ldc % 4 == 0 && err_epi_aligned(e);
 }
 
+// ... or into the K-splitting kernel: whole 4-column groups, any number of rows.
+bool hidden_err_wave_ok(const ErrEpi &e, uint32_t N) { return N % 4 == 0 && e.ldc % 4 == 0 && err_epi_aligned(e); }
+
 // Whole output tiles with a 4-aligned leading dimension: the batched epilogue.
 static bool dma_full_epilogue(const GemmLaunch &g) {
     const uint32_t mv = g.mv ? g.mv : g.M, nv = g.nv ? g.nv : g.N;

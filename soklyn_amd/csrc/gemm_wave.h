@@ -553,6 +553,41 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WPE
             *reinterpret_cast<floatx4 *>(E + (wave * BM + 16 * i + (lane & 15u)) * EP + 16 * j + 4 * (lane >> 4)) =
                 acc[i][j];
     lds_barrier();
+    if constexpr (EpiSums<Epi>::value) {
+        // the hidden error: 4 columns per lane (the launcher has checked their alignment), a
+        // thread's group of columns fixed; the operands of up to 4 rows loaded before any use
+        constexpr uint32_t QN = BM * BN / 4, GR = BN / 4, ACT = QN < NT ? QN : NT, ROWS = QN / ACT;
+        constexpr uint32_t UB = ROWS < 4 ? ROWS : 4;
+        static_assert(NT % GR == 0 && ROWS % UB == 0, "one column group per thread");
+        static_assert((ACT / GR) * 3 * BN * 4 <= sizeof(smem), "column sums fit the ring");
+        const uint32_t group = tid % GR, n = n0 + 4 * group;
+        const bool live = tid < ACT && n + 3 < sh.N;
+        typename EpiSums<Epi>::Acc csum{};
+        if (live) {
+            const typename Epi::Col col = Epi::column(ep, n);
+#pragma unroll 1
+            for (uint32_t u0 = 0; u0 < ROWS; u0 += UB) {
+                typename Epi::Pre pre[UB];
+#pragma unroll
+                for (uint32_t u = 0; u < UB; ++u) {
+                    const uint32_t m = m0 + (tid + (u0 + u) * ACT) / GR;
+                    if (m < sh.M) Epi::load(ep, (uint64_t)m * Epi::ldc(ep) + n, m, pre[u]);
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < UB; ++u) {
+                    const uint32_t r = (tid + (u0 + u) * ACT) / GR, m = m0 + r;
+                    if (m >= sh.M) continue;
+                    floatx4 v = *reinterpret_cast<const floatx4 *>(E + r * EP + 4 * group);
+#pragma unroll
+                    for (int w = 1; w < W; ++w)
+                        v += *reinterpret_cast<const floatx4 *>(E + (w * BM + r) * EP + 4 * group);
+                    Epi::finish(ep, (uint64_t)m * Epi::ldc(ep) + n, m, n, v, col, pre[u], csum);
+                }
+            }
+        }
+        lds_barrier();   // every wave is done reading E
+        Epi::template flush_slots<ACT / GR, BN, NT>(ep, csum, E, tid, tid / GR, group, tm, n0);
+    } else {
     if (sh.nv) {   // output rows on 4-element boundaries: 4 columns per lane
         // (the optimiser's state loaded ahead of this sum made a 2048 x 1000 dW 3 us slower)
         for (uint32_t q = tid; q < BM * BN / 4; q += NT) {
@@ -575,6 +610,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WPE
                 Epi::apply1(ep, m0 + r, n, v, col, blockIdx.y);
             }
         }
+    }
     }
     // or it rides behind the tiles (the launcher's choice)
     if constexpr (std::is_same<typename Epi::Params, OptEpi>::value) {

@@ -120,6 +120,8 @@ template <typename T> static hipError_t run_wave_op(const GemmLaunch &g, hipStre
     case Op::InputGrad: return run_wave<T, EpiStoreK, true, true>(g, g.st, s);
     case Op::DwOpt: return run_wave<T, EpiOptK<T>, false, false>(g, g.opt, s);
     case Op::DwPartial: return run_wave<T, EpiStoreK, false, false>(g, g.st, s);
+    case Op::HiddenErr:
+        return hidden_err_wave_ok(g.err, g.N) ? run_wave<T, EpiErrK<T>, true, true>(g, g.err, s) : hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
 }
@@ -142,7 +144,7 @@ bool gemm_wave_ok(const GemmLaunch &g, uint32_t splits) {
     const uint64_t esz = g.dtype == 1 ? 2 : 4;
     if (!g.M || !g.N || !g.K) return false;
     const bool layout = g.op == Op::Fwd ? g.a_kcontig && !g.b_kcontig
-                        : g.op == Op::InputGrad ? g.a_kcontig && g.b_kcontig
+                        : g.op == Op::InputGrad || g.op == Op::HiddenErr ? g.a_kcontig && g.b_kcontig
                         : g.op == Op::DwOpt || g.op == Op::DwPartial ? !g.a_kcontig && !g.b_kcontig : false;
     const uint64_t k = gemm_wave_slice(g.K, splits);
     auto span = [&](bool kc, uint32_t ld) { return ((kc ? 64ull : k + 64ull) * ld + g.K) * esz; };

@@ -85,6 +85,8 @@ enum class Op { Fwd, InputGrad, DwOpt, DwPartial, HiddenErr };
 // The fused hidden error fits the 256x256 kernel's output of M x N (whole tiles,
 // 4-aligned rows, 16-byte aligned buffers).
 bool hidden_err_fusable(const ErrEpi &e, uint32_t M, uint32_t N);
+// ... or the K-splitting kernel's output of N columns.
+bool hidden_err_wave_ok(const ErrEpi &e, uint32_t N);
 
 // One GEMM launch.  dtype selects fp16 (MFMA 32x32x16 f16) or fp32
 // (MFMA 32x32x2 f32).  a_kcontig / b_kcontig as in gemm.h.

@@ -99,3 +99,41 @@ def test_step_ragged_128(ctx, M, K, N):
 @pytest.mark.parametrize("norm,act,p", [(abi.NORM_RMS, abi.ACT_MISH, 0.1), (abi.NORM_BATCH, abi.ACT_TANH, 0.0)])
 def test_hidden_error_128(ctx, norm, act, p):
     fused_error(ctx, 2048, 64, 2048, 1024, norm, act, p, 0)
+
+
+# the hidden error in the K-splitting kernel's epilogue: each tile, rows past the batch, columns
+# past the output, odd k (fp16 rows through registers), every norm; its column sums through the
+# bias and norm-parameter moments.  A width that is not whole 4-column groups takes two kernels.
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N0,N1,norm,act,p", [
+    (3, 4, 17, abi.NORM_RMS, abi.ACT_MISH, 0.0), (40, 36, 33, abi.NORM_LAYER, abi.ACT_SILU, 0.1),
+    (130, 100, 200, abi.NORM_BATCH, abi.ACT_TANH, 0.0), (257, 516, 66, abi.NORM_DISABLED, abi.ACT_SILU, 0.2),
+    (515, 900, 330, abi.NORM_RMS, abi.ACT_MISH, 0.1), (701, 836, 129, abi.NORM_LAYER, abi.ACT_SIGMOID, 0.0),
+    (1700, 2000, 40, abi.NORM_DISABLED, abi.ACT_TANH, 0.0), (66, 50, 72, abi.NORM_RMS, abi.ACT_SILU, 0.0)])
+def test_hidden_error(ctx, half, M, N0, N1, norm, act, p):
+    K0 = 24
+    print(f"hidden error M={M} {N0} <- {N1} norm={norm} half={half}", flush=True)
+    o0, d0 = make_pair(ctx, K0, N0, M, seed=M + N0, half=half, norm=norm, act=act, p=p)
+    o1, d1 = make_pair(ctx, N0, N1, M, seed=N1, half=half)
+    x = inputs(111, M, K0, half)
+    o0.forward(x, M, p > 0, 99)
+    d0.forward(dev(x, half), M, p > 0, 99)
+    o1.forward(o0.out, M)
+    d1.forward(d0.out, M)
+    s = (rng(112).standard_normal((M, N1)) * 64).astype(np.float32)
+    o1.error_from_sum(s, M)
+    d1.error_from_sum(torch.from_numpy(s).cuda(), M)
+    opt = (O.Optimiser.sgd(0.5), abi.sgd(0.5))
+    o0.hidden_error(o1, M)
+    o0.backward(x, opt[0], opt[0], M, 1e-3, 3.4e38, 1)
+    d0.backward_hidden(d1, dev(x, half), abi.train_ctx(opt[1], opt[1], M, 1e-3), 1)
+    torch.cuda.synchronize()
+    tol = FP16_TOL if half else FP32_TOL
+    for name in ["grad", "d_prenorm"] + (["d_norm_w", "d_norm_b"] if norm else []):
+        check(name, d0.get(name), getattr(o0, name), tol)
+    if half:
+        assert np.array_equal(d0.get("d_prenorm_h"), f16(d0.get("d_prenorm")))
+    names = (["dv_b"] if norm != abi.NORM_BATCH else []) + (["dv_norm_w"] if norm else [])
+    names += ["dv_norm_b"] if norm >= abi.NORM_LAYER else []
+    for name in names + ["dv_w"]:
+        check(name, d0.get(name), getattr(o0, name), tol)
