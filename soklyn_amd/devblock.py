@@ -132,13 +132,13 @@ class DeviceBlock:
 
     # -- hot-path steps ------------------------------------------------------------------
     def forward(self, x: torch.Tensor, batch: int, use_dropout: bool = False, seed: int = 0):
-        rows, cols = x.shape
+        rows, cols = x.shape[0], x.shape[1]
         abi.call("skl_dense_forward", self.ctx.h, self._fill("forward"), x.data_ptr(), rows, cols, batch,
                  int(use_dropout), seed & 0xFFFFFFFF)
         return self.out
 
     def output_error(self, target: torch.Tensor, loss: int, act: int, leaky: float = 0.0):
-        rows, cols = target.shape
+        rows, cols = target.shape[0], target.shape[1]
         abi.call("skl_dense_output_error", self.ctx.h, self._fill("output_error"), target.data_ptr(), rows, cols, loss,
                  act, leaky)
 
@@ -146,11 +146,11 @@ class DeviceBlock:
         abi.call("skl_dense_hidden_error", self.ctx.h, self._fill("hidden"), nxt._fill("above"), batch)
 
     def backward(self, x: torch.Tensor, tc: abi.SklTrainCtx, step: int):
-        rows, cols = x.shape
+        rows, cols = x.shape[0], x.shape[1]
         abi.call("skl_dense_backward", self.ctx.h, self._fill("update"), x.data_ptr(), rows, cols, C.byref(tc), step)
 
     def backward_hidden(self, nxt: "DeviceBlock", x: torch.Tensor, tc: abi.SklTrainCtx, step: int):
-        rows, cols = x.shape
+        rows, cols = x.shape[0], x.shape[1]
         abi.call("skl_dense_backward_hidden", self.ctx.h, self._fill("hidden"), nxt._fill("above"), x.data_ptr(), rows,
                  cols, C.byref(tc), step)
 

@@ -47,3 +47,14 @@ def test_descriptors_are_per_thread():
     t.start()
     t.join()
     assert got[0] is not b._fill("forward")._obj
+
+
+def test_leading_dimensions_of_inputs_and_targets(monkeypatch):
+    """Rows and columns are the first two dimensions, whatever follows them."""
+    calls = []
+    monkeypatch.setattr(abi, "call", lambda name, *args: calls.append((name, args)))
+    b = block(False, abi.NORM_DISABLED)
+    b.forward(torch.zeros(8, 24, 1), 8)
+    b.output_error(torch.zeros(8, 16, 1), abi.LOSS_CE, abi.ACT_SOFTMAX)
+    b.backward(torch.zeros(8, 24, 1), abi.train_ctx(abi.sgd(0.5), abi.sgd(0.5), 8, 1e-3), 1)
+    assert [args[3:5] for _, args in calls] == [(8, 24), (8, 16), (8, 24)]
