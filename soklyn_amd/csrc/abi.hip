@@ -458,8 +458,9 @@ double dma128_us(const GemmLaunch &g) {
     return (g.op == Op::InputGrad ? 4.5 : 8.5) + kt * (0.5 * u > 0.65 ? 0.5 * u : 0.65);
 }
 
-// in_place: the output overlaps an operand (a caller's dx over d_prenorm).  The K-splitting
-// kernel's many small tiles would overwrite rows that others have yet to read.
+// in_place: the output overlaps an operand (a caller's dx over d_prenorm, a layer fed its own
+// output).  The K-splitting kernel's many small tiles would overwrite rows that others have
+// yet to read.
 GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
     GemmPlan p{};
     p.tile = 256;
@@ -646,7 +647,7 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
             if (vec_done) *vec_done = true;
         }
         SKL_TRY(timed_gemm(ctx, g, GemmKind::Wave));
-    } else     if (p.dma) {
+    } else if (p.dma) {
         // a d_prenorm_h padded by the GEMM before (or padded now into a kept slot),
         // else a padded copy in the workspace
         if (p.pad_a) {
@@ -1055,7 +1056,15 @@ int32_t skl_dense_forward(skl_ctx *ctx, const skl_dense_desc *b, const void *in,
     g.fwd.leaky = b->act == SKL_ACT_LEAKY_RELU ? b->leaky : 0.0f;       // ffn_device.rs:32-35
     g.fwd.p = b->mask_coeff;
     g.fwd.ldc = b->outputs;
-    const GemmPlan plan = plan_gemm(g);
+    // the layer's own output as its input (up to one tile wide): a tile then reads its rows
+    // whole before it writes them, which the smaller tiles do not
+    const size_t esz = b->dtype == SKL_F16 ? 2 : 4, in_sz = (size_t)batch * in_cols * esz;
+    const size_t o_sz = (size_t)batch * b->outputs * esz;
+    bool in_place = overlaps(in, in_sz, g.fwd.z_out, o_sz);
+    if (g.fwd.fuse_act)
+        in_place = in_place || overlaps(in, in_sz, b->predrop, o_sz) || overlaps(in, in_sz, b->out, o_sz) ||
+                   (use_dropout && overlaps(in, in_sz, b->mask, o_sz));
+    const GemmPlan plan = plan_gemm(g, in_place);
     if ((r = ensure_ws(ctx, plan.bytes()))) return r;
     if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws)))) return r;
 
@@ -1258,7 +1267,18 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     e.leaky = cur->act == SKL_ACT_LEAKY_RELU ? cur->leaky : 0.0f;
     e.inv_n = 1.0f / (float)cur->outputs;
     e.inv_m = 1.0f / (float)batch;
-    if (plan.dma && !plan.rag && hidden_err_fusable(e, batch, cur->outputs)) {
+    // Layers that share their backward buffers: an epilogue that writes cur's error would
+    // overwrite rows of next's that other tiles have yet to read; the sum goes first then.
+    const size_t esz = cur->dtype == SKL_F16 ? 2 : 4, cells = (size_t)batch * cur->outputs;
+    auto over_next = [&](const void *p, size_t sz) {
+        return overlaps(p, cells * sz, next_dp, (size_t)batch * next->outputs * esz) ||
+               overlaps(p, cells * sz, next->w, (size_t)cur->outputs * next->outputs * esz);
+    };
+    const bool shared = over_next(cur->grad, 4) || over_next(cur->d_prenorm, 4) ||
+                        (cur->dtype == SKL_F16 && over_next(cur->d_prenorm_h, 2)) ||
+                        (cur->norm != SKL_NORM_DISABLED &&
+                         (over_next(cur->d_norm_w, 4) || over_next(cur->d_norm_b, 4)));
+    if (!shared && plan.dma && !plan.rag && hidden_err_fusable(e, batch, cur->outputs)) {
         // One kernel, as the reference has it (backward.cu:59-102): the 256x256
         // GEMM's epilogue computes the error from the sum in its accumulators
         // and leaves the column sums of each 256-row tile for cur's backward.
@@ -1271,7 +1291,7 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
         record_cols(ctx, cur, batch, tiles_m);
         return SKL_OK;
     }
-    if (plan.wave && hidden_err_wave_ok(e, cur->outputs)) {
+    if (!shared && plan.wave && hidden_err_wave_ok(e, cur->outputs)) {
         // the same on the K-splitting kernel's tiles
         const uint32_t tiles_m = (batch + plan.wave - 1) / plan.wave;
         if ((r = ensure_cols_splits(ctx, tiles_m, cur->outputs))) return r;

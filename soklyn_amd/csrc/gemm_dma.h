@@ -268,7 +268,8 @@ template <int NW, int NF, int MI = 32, int COLS = 256, bool RAG = false> struct 
         for (uint32_t t = 0; t < 2; ++t) {
             const uint32_t r = RPI * (wave + NW * t) + lane / LPR;
             const uint32_t cl = (lane % LPR) ^ swz(r);
-            dma[t].init(p, RAG ? (((rows - 1u) * ld + cols) * 2u + 3u) & ~3u : rows * ld * 2u, (RPI * wave + lane / LPR) * ld * 2u + mn0 * 2u + cl * 16u);
+            dma[t].init(p, RAG ? (((rows - 1u) * ld + cols) * 2u + 3u) & ~3u : rows * ld * 2u,
+                        (RPI * wave + lane / LPR) * ld * 2u + mn0 * 2u + cl * 16u);
         }
         step = RPI * NW * ld * 2u;
         kstep = 64u * ld * 2u;

@@ -137,3 +137,41 @@ def test_hidden_error(ctx, half, M, N0, N1, norm, act, p):
     names += ["dv_norm_b"] if norm >= abi.NORM_LAYER else []
     for name in names + ["dv_w"]:
         check(name, d0.get(name), getattr(o0, name), tol)
+
+
+# Layers whose backward buffers are one piece of memory, and a narrow layer fed its own output:
+# the calls that read and write it take routes that read it whole first.
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N0,N1", [(512, 512, 256), (300, 260, 72)])
+def test_hidden_error_over_the_layer_above(ctx, half, M, N0, N1):
+    K0 = 24
+    o0, d0 = make_pair(ctx, K0, N0, M, seed=M + N0, half=half, act=abi.ACT_SILU)
+    o1, d1 = make_pair(ctx, N0, N1, M, seed=N1, half=half)
+    # one buffer of the larger size: d0's whole, d1's a leading part of it
+    name = "d_prenorm_h" if half else "d_prenorm"
+    setattr(d1, name, getattr(d0, name).view(-1)[:M * N1].view(M, N1))
+    x = inputs(111, M, K0, half)
+    o0.forward(x, M)
+    d0.forward(dev(x, half), M)
+    o1.forward(o0.out, M)
+    d1.forward(d0.out, M)
+    s = (rng(112).standard_normal((M, N1)) * 64).astype(np.float32)
+    o1.error_from_sum(s, M)
+    d1.error_from_sum(torch.from_numpy(s).cuda(), M)
+    o0.hidden_error(o1, M)
+    d0.hidden_error(d1, M)
+    torch.cuda.synchronize()
+    for field in ("grad", "d_prenorm"):
+        check(field, d0.get(field), getattr(o0, field), FP16_TOL if half else FP32_TOL)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N", [(200, 64), (77, 10)])
+def test_forward_of_its_own_output(ctx, half, M, N):
+    ob, db = make_pair(ctx, N, N, M, seed=N, half=half, act=abi.ACT_SILU)
+    x = inputs(113, M, N, half)
+    db.out.copy_(dev(x, half))
+    ob.forward(x, M)
+    db.forward(db.out, M)
+    torch.cuda.synchronize()
+    check("out", db.get("out"), ob.out, FP16_TOL if half else FP32_TOL)
