@@ -1207,29 +1207,6 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     const uint32_t keep = cur->dtype == SKL_F16 ? KEEP_A : 0;   // next_dp is a d_prenorm_h
     note_rewrite(ctx, cur);
 
-    // A next layer of at most 16 outputs: its GEMM would pad k to 128, so the
-    // error kernel forms s = next.d_prenorm . next.W^T itself, per element, from
-    // copies of the two operands padded to 16 columns (same operands as the
-    // GEMM: f16(d_prenorm) and the working W for fp16 blocks).
-    if (next->outputs <= 16) {
-        uint32_t splits = 0;
-        if ((r = ensure_cols(ctx, cur, batch, 2, &splits))) return r;
-        const size_t esz = cur->dtype == SKL_F16 ? 2 : 4;
-        const size_t a_bytes = ((size_t)batch * 16 * esz + 255) & ~(size_t)255;
-        if ((r = ensure_ws(ctx, a_bytes + (size_t)cur->outputs * 16 * esz))) return r;
-        char *a16 = reinterpret_cast<char *>(ctx->ws), *w16 = a16 + a_bytes;
-        a.sk_a = a16;
-        a.sk_w = w16;
-        if (err_skinny_ok(a, ctx->cols)) {
-            SKL_TRY(launch_skinny_operands(cur->dtype, next_dp, batch, next->w, cur->outputs, next->outputs, a16, w16,
-                                           ctx->stream));
-            SKL_TRY(launch_error_skinny(a, ctx->cols, splits, ctx->stream));
-            record_cols(ctx, cur, batch, splits);
-            return SKL_OK;
-        }
-        a.sk_a = a.sk_w = nullptr;
-    }
-
     // s = next.d_prenorm . next.W^T into the workspace (backward.cu:72-77; fp16:
     // f16(d_prenorm) and the working W, == f16(master) after every update) ...
     GemmLaunch g{};
@@ -1246,6 +1223,34 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     g.splits = 1;
     g.op = Op::InputGrad;
     const GemmPlan plan = plan_gemm(g);
+
+    // A next layer of at most 16 outputs: its GEMM would pad k to 128, so the
+    // error kernel forms s = next.d_prenorm . next.W^T itself, per element, from
+    // copies of the two operands padded to 16 columns (same operands as the
+    // GEMM: f16(d_prenorm) and the working W for fp16 blocks).  Up to 2M elements
+    // the K-splitting kernel's epilogue is ahead, one launch for two: next of 10,
+    // 64 x 128 fp32 8.0 -> 5.4 us, 1024 x 512 fp16 8.4 -> 5.3, 4096 x 512 11.9 -> 9.5;
+    // beyond, its many short tiles are not: 4096 x 2048 27 -> 35, 12345 x 512 23 -> 29.
+    const size_t esz = cur->dtype == SKL_F16 ? 2 : 4, cells = (size_t)batch * cur->outputs;
+    const bool small = plan.wave && cur->outputs % 4 == 0 && cells <= (size_t(1) << 21);
+    if (next->outputs <= 16 && !small) {
+        uint32_t splits = 0;
+        if ((r = ensure_cols(ctx, cur, batch, 2, &splits))) return r;
+        const size_t a_bytes = ((size_t)batch * 16 * esz + 255) & ~(size_t)255;
+        if ((r = ensure_ws(ctx, a_bytes + (size_t)cur->outputs * 16 * esz))) return r;
+        char *a16 = reinterpret_cast<char *>(ctx->ws), *w16 = a16 + a_bytes;
+        a.sk_a = a16;
+        a.sk_w = w16;
+        if (err_skinny_ok(a, ctx->cols)) {
+            SKL_TRY(launch_skinny_operands(cur->dtype, next_dp, batch, next->w, cur->outputs, next->outputs, a16, w16,
+                                           ctx->stream));
+            SKL_TRY(launch_error_skinny(a, ctx->cols, splits, ctx->stream));
+            record_cols(ctx, cur, batch, splits);
+            return SKL_OK;
+        }
+        a.sk_a = a.sk_w = nullptr;
+    }
+
     ErrEpi &e = g.err;
     // an operand act' does not read aliases the mask (loaded anyway: cache hits)
     e.predrop = act_uses_output(cur->act) ? cur->predrop : cur->mask;
@@ -1269,7 +1274,6 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     e.inv_m = 1.0f / (float)batch;
     // Layers that share their backward buffers: an epilogue that writes cur's error would
     // overwrite rows of next's that other tiles have yet to read; the sum goes first then.
-    const size_t esz = cur->dtype == SKL_F16 ? 2 : 4, cells = (size_t)batch * cur->outputs;
     auto over_next = [&](const void *p, size_t sz) {
         return overlaps(p, cells * sz, next_dp, (size_t)batch * next->outputs * esz) ||
                overlaps(p, cells * sz, next->w, (size_t)cur->outputs * next->outputs * esz);

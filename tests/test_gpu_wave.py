@@ -139,6 +139,17 @@ def test_hidden_error(ctx, half, M, N0, N1, norm, act, p):
         check(name, d0.get(name), getattr(o0, name), tol)
 
 
+# the layer above of at most 16 outputs: in the epilogue up to 2M elements, in the error kernel
+# beyond and for widths that are not whole 4-column groups
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N0,N1,norm", [(1, 4, 1, abi.NORM_DISABLED), (64, 128, 10, abi.NORM_DISABLED),
+                                          (300, 260, 3, abi.NORM_RMS), (1024, 512, 16, abi.NORM_LAYER),
+                                          (2048, 1024, 10, abi.NORM_RMS), (2049, 1024, 10, abi.NORM_RMS),
+                                          (130, 51, 7, abi.NORM_BATCH)])
+def test_hidden_error_below_a_narrow_layer(ctx, half, M, N0, N1, norm):
+    test_hidden_error(ctx, half, M, N0, N1, norm, abi.ACT_SILU, 0.1)
+
+
 # Layers whose backward buffers are one piece of memory, and a narrow layer fed its own output:
 # the calls that read and write it take routes that read it whole first.
 @pytest.mark.parametrize("half", [False, True])
