@@ -1831,8 +1831,7 @@ hipError_t launch_vec_opt(const VecOptArgs &a0, hipStream_t s) {
 // a.vec (vec_opt_block; independent of W), the next blocks the reduction: block
 // gx * y + x, or for narrow outputs (gx = 0) one thread per element of the gy.
 // FLAT (launcher): planes without row padding whose rows are not 4-element groups go as one
-// row of all elements, so that every access is 16 bytes whatever n is (777 x 1531, 5 planes:
-// an element per thread took 27 us).
+// row of all elements where their number is a multiple of 4: 16-byte accesses at any such n.
 template <typename T> __device__ __forceinline__ float reduced(const DwReduceArgs &a, uint32_t r, uint32_t c, float v) {
     if constexpr (sizeof(T) == 2) {
         if (__builtin_expect(!__builtin_isfinite(v), 0) && a.flat_n) {
