@@ -6,6 +6,7 @@
 // the MI355X kernels on the context's stream.
 #include <float.h>
 #include <math.h>
+#include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -54,6 +55,16 @@ struct PadCopy {
     bool valid;
 };
 
+// SOKLYN_GEMM_ROUTE at skl_ctx_create names the kernel of the context's GEMMs (tests of one
+// instantiation, A/B comparisons): "staged", "dma", "dma128" (operands as stored), "skinny" or
+// "wave:TILE[:WAVES[:SLICES]]" (0: as planned).  A call whose GEMM that kernel does not take
+// fails, so a test that passes has run it.
+enum class Route : uint32_t { Planned, Staged, Dma, Dma128, Skinny, Wave };
+struct GemmRoute {
+    Route kind;
+    uint32_t tile, waves, splits;
+};
+
 // Scratch of kernels that hand partial results to the launch after them (a BatchNorm's
 // column statistics), one piece per stream the context has run on: forwards on two
 // streams of one context share nothing else, so they may overlap.
@@ -78,6 +89,7 @@ struct skl_ctx {
     ColSums cs;
     PadCopy pads[kPadSlots];
     bool keep_pads;      // SOKLYN_PAD_KEEP=0 at skl_ctx_create: GEMMs pad d_prenorm_h into the workspace every time
+    GemmRoute route;     // SOKLYN_GEMM_ROUTE at skl_ctx_create: the kernel every GEMM must take
     hipEvent_t gemm_start, gemm_stop;   // skl_ctx_time_next_gemm
     void *scratch;       // device address of this device's copy of `scratch` (below)
     StreamScratch streams[kStreamSlots];
@@ -321,10 +333,15 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //  * the K-splitting kernel on small tiles (gemm_wave.h), for outputs that would leave
 //    those tiles' GPU mostly idle and for at most 16 columns: operands as stored, no
 //    workspace but the partial planes of a dW over a long batch;
+//  * the streaming kernel for a dW of at most 16 columns over a large X whose rows the
+//    K-splitting kernel reads slowly or not at all (skinny_us);
 //  * the register-staged kernels otherwise (large fp32; small fp16 with little k to
 //    reduce), with the same split-K for small dW grids.
 struct GemmPlan {
     uint32_t wave;             // K-splitting kernel: its tile edge (0: another kernel)
+    uint32_t waves;            // ... and its waves per tile (0: the launcher's choice)
+    bool skinny;               // dW of at most 16 columns: the streaming kernel's partials, then the reduction
+    bool refused;              // the kernel that SOKLYN_GEMM_ROUTE names does not take the GEMM
     bool dma;
     bool rag;                  // direct-to-LDS on operands as stored, 128x128 tiles
     bool pad_a, pad_b;
@@ -458,152 +475,234 @@ double dma128_us(const GemmLaunch &g) {
     return (g.op == Op::InputGrad ? 4.5 : 8.5) + kt * (0.5 * u > 0.65 ? 0.5 * u : 0.65);
 }
 
-// in_place: the output overlaps an operand (a caller's dx over d_prenorm, a layer fed its own
-// output).  The K-splitting kernel's many small tiles would overwrite rows that others have
-// yet to read.
-GemmPlan plan_gemm(const GemmLaunch &g, bool in_place = false) {
+GemmPlan plan_as_stored(const GemmLaunch &g) {
     GemmPlan p{};
     p.tile = 256;
     p.splits = 1;
     p.Mp = g.M;
     p.Np = g.N;
     p.Kp = g.K;
+    return p;
+}
+
+// The K-splitting kernel on tiles of edge `tile`, a dW in up to `splits` batch slices.
+bool plan_wave(const GemmLaunch &g, uint32_t tile, uint32_t splits, GemmPlan *out) {
+    if (!tile || !gemm_wave_ok(g, splits)) return false;
+    GemmPlan p = plan_as_stored(g);
+    p.wave = tile;
+    if (splits > 1) {
+        const uint32_t slice = gemm_wave_slice(g.K, splits);
+        p.splits = (g.K + slice - 1) / slice;
+        // planes on 16-byte boundaries, rows without padding
+        if (p.splits > 1) p.part_bytes = (size_t)p.splits * (((uint64_t)g.M * g.N + 3) & ~3ull) * sizeof(float);
+    }
+    *out = p;
+    return true;
+}
+
+// The streaming kernel for a dW of at most 16 columns.
+bool plan_skinny(const GemmLaunch &g, GemmPlan *out) {
+    if (g.op != Op::DwOpt || g.N > 16 || !g.M || !g.N || !g.K) return false;
+    GemmPlan p = plan_as_stored(g);
+    p.skinny = true;
+    p.splits = skinny_dw_slices(g.K, g.M);
+    p.part_bytes = (size_t)p.splits * g.M * 16 * sizeof(float);
+    *out = p;
+    return true;
+}
+
+// The direct-to-LDS kernel on operands padded to its tiles where they are not whole, for
+// grids that fill the GPU.  *us: its estimated time, the copies included.
+bool plan_dma(const GemmLaunch &g, GemmPlan *out, double *us) {
+    if (g.dtype != SKL_F16 || !gemm_dma_enabled() || !g.M || !g.N || !g.K) return false;
     const bool dw = g.op == Op::DwOpt;
-    // a dW may go in batch slices (partial planes in the workspace) where the register-
-    // staged kernels would split it too: below 160 tiles of 128x128 and from 8 k-tiles on
-    const uint32_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128);
-    double wave_us = 0.0;
-    uint32_t wave_splits = dw && t128 < 160 && g.K >= 8 * gemm_bk(g.dtype) ? 16 : 1;
-    const uint32_t wave = in_place ? 0 : gemm_wave_tile(g, &wave_splits, &wave_us);
-    auto take_wave = [&] {
-        p.wave = wave;
-        if (wave_splits > 1) {
-            const uint32_t slice = gemm_wave_slice(g.K, wave_splits);
-            p.splits = (g.K + slice - 1) / slice;
-            // planes on 16-byte boundaries, rows without padding
-            if (p.splits > 1) p.part_bytes = (size_t)p.splits * (((uint64_t)g.M * g.N + 3) & ~3ull) * sizeof(float);
-        }
-    };
-    // outputs of at most 16 columns: any larger tile is >90% padding
-    if (g.N <= 16 && wave) {
-        take_wave();
-        return p;
+    const uint32_t Mp = round_up(g.M, 256), Np = round_up(g.N, 256), Kp = round_up(g.K, 128);
+    // in units of 256x256 tiles whatever the kernel's tile edge
+    const uint32_t tiles = (Mp / 256) * (Np / 256);
+    uint32_t dw_tile = 256;
+    *us = (tiles + 255) / 256 * (Kp / 128) * 3.4;
+    const uint32_t splits = dw && tiles < 160 ? dw_dma_splits(tiles, Kp, (uint64_t)Mp * Np, &dw_tile, us) : 1;
+    const bool waste_ok = (uint64_t)Mp * Np <= (uint64_t)g.M * g.N * 3 / 2;
+    // the kernel's operand offsets are 32-bit
+    const uint64_t a_span = g.a_kcontig ? (uint64_t)Mp * (g.lda > Kp ? g.lda : Kp)
+                                        : (uint64_t)Kp * (g.lda > Mp ? g.lda : Mp);
+    const uint64_t b_span = g.b_kcontig ? (uint64_t)Np * (g.ldb > Kp ? g.ldb : Kp)
+                                        : (uint64_t)Kp * (g.ldb > Np ? g.ldb : Np);
+    const bool offsets_ok = a_span * 2 < (1ull << 32) && b_span * 2 < (1ull << 32);
+    // enough workgroups to fill the GPU: 192 of 256x256, or 384 of 128x128 (two per CU)
+    const uint32_t fill = dw_tile == 128 ? 4 * tiles * splits / 2 : tiles * splits;
+    if (!waste_ok || !offsets_ok || fill < 192) return false;
+    GemmPlan p{};
+    p.dma = true;
+    p.Mp = Mp;
+    p.Np = Np;
+    p.Kp = Kp;
+    p.splits = splits;
+    p.tile = dma_tile(g.op, Mp, Np, splits, &p.band);
+    if (dw && dw_tile == 128 && !gemm_dma_tile_forced()) p.tile = 128;
+    // A: k-contiguous [M x K] or m-contiguous [K x M]; B likewise with N
+    p.pad_a = g.a_kcontig ? !dma_operand_ok(g.A, g.M, g.K, g.lda, 256, 128)
+                          : !dma_operand_ok(g.A, g.K, g.M, g.lda, 128, 256);
+    p.pad_b = g.b_kcontig ? !dma_operand_ok(g.B, g.N, g.K, g.ldb, 256, 128)
+                          : !dma_operand_ok(g.B, g.K, g.N, g.ldb, 128, 256);
+    // 256-byte aligned regions
+    p.a_bytes = p.pad_a ? ((size_t)Mp * Kp * 2 + 255) & ~(size_t)255 : 0;
+    p.b_bytes = p.pad_b ? ((size_t)Np * Kp * 2 + 255) & ~(size_t)255 : 0;
+    p.part_bytes = splits > 1 ? (size_t)splits * Mp * Np * sizeof(float) : 0;
+    *out = p;
+    return true;
+}
+
+// 128x128 direct-to-LDS tiles over operands as stored (forward and input gradient).
+bool plan_dma128(const GemmLaunch &g, GemmPlan *out) {
+    if (g.dtype != SKL_F16 || (g.op != Op::Fwd && g.op != Op::InputGrad)) return false;
+    const bool whole = g.M % 256 == 0 && g.N % 256 == 0 && gemm_dma_shape_ok(g);
+    if (!whole && !gemm_dma_rag_ok(g)) return false;
+    GemmPlan p = plan_as_stored(g);
+    p.dma = true;
+    p.rag = !whole;
+    p.tile = 128;
+    *out = p;
+    return true;
+}
+
+// The register-staged kernels, with split-K for small dW grids.
+GemmPlan plan_staged(const GemmLaunch &g) {
+    GemmPlan p = plan_as_stored(g);
+    if (g.op != Op::DwOpt) return p;
+    const uint32_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128), bk = gemm_bk(g.dtype);
+    uint32_t tiles = gemm_tiles(g.dtype, g.M, g.N);
+    // fp32: 128x128 tiles split over the batch rather than the 64x64 tiles a
+    // small grid would otherwise get (C2's 1024 x 1024 dW over 4096 rows: 4
+    // slices of 64 tiles, 103 -> 77 us, against 256 whole 64x64 tiles)
+    if (g.dtype == SKL_F32 && t128 < 160 && g.K >= 8 * 4 * bk) {
+        tiles = t128;
+        p.tile = 128;
     }
-    if (g.dtype == SKL_F16 && gemm_dma_enabled() && g.M && g.N && g.K) {
-        const uint32_t Mp = round_up(g.M, 256), Np = round_up(g.N, 256), Kp = round_up(g.K, 128);
-        // in units of 256x256 tiles whatever the kernel's tile edge
-        const uint32_t tiles = (Mp / 256) * (Np / 256);
-        uint32_t dw_tile = 256;
-        double dma_us = (tiles + 255) / 256 * (Kp / 128) * 3.4;
-        const uint32_t splits = dw && tiles < 160 ? dw_dma_splits(tiles, Kp, (uint64_t)Mp * Np, &dw_tile, &dma_us) : 1;
-        const bool waste_ok = (uint64_t)Mp * Np <= (uint64_t)g.M * g.N * 3 / 2;
-        // the kernel's operand offsets are 32-bit
-        const uint64_t a_span = g.a_kcontig ? (uint64_t)Mp * (g.lda > Kp ? g.lda : Kp)
-                                            : (uint64_t)Kp * (g.lda > Mp ? g.lda : Mp);
-        const uint64_t b_span = g.b_kcontig ? (uint64_t)Np * (g.ldb > Kp ? g.ldb : Kp)
-                                            : (uint64_t)Kp * (g.ldb > Np ? g.ldb : Np);
-        const bool offsets_ok = a_span * 2 < (1ull << 32) && b_span * 2 < (1ull << 32);
-        // enough workgroups to fill the GPU: 192 of 256x256, or 384 of 128x128 (two per CU)
-        const uint32_t fill = dw_tile == 128 ? 4 * tiles * splits / 2 : tiles * splits;
-        if (waste_ok && offsets_ok && fill >= 192) {
-            p.dma = true;
-            p.Mp = Mp;
-            p.Np = Np;
-            p.Kp = Kp;
+    if (tiles < 160 && g.K >= 8 * bk) {
+        uint32_t splits = (256 + tiles - 1) / tiles;
+        const uint32_t max_splits = g.K / (4 * bk);
+        if (splits > max_splits) splits = max_splits;
+        if (splits > 16) splits = 16;
+        if (splits >= 2) {
             p.splits = splits;
-            p.tile = dma_tile(g.op, Mp, Np, splits, &p.band);
-            if (dw && dw_tile == 128 && !gemm_dma_tile_forced()) p.tile = 128;
-            // A: k-contiguous [M x K] or m-contiguous [K x M]; B likewise with N
-            p.pad_a = g.a_kcontig ? !dma_operand_ok(g.A, g.M, g.K, g.lda, 256, 128)
-                                  : !dma_operand_ok(g.A, g.K, g.M, g.lda, 128, 256);
-            p.pad_b = g.b_kcontig ? !dma_operand_ok(g.B, g.N, g.K, g.ldb, 256, 128)
-                                  : !dma_operand_ok(g.B, g.K, g.N, g.ldb, 128, 256);
-            // 256-byte aligned regions
-            p.a_bytes = p.pad_a ? ((size_t)Mp * Kp * 2 + 255) & ~(size_t)255 : 0;
-            p.b_bytes = p.pad_b ? ((size_t)Np * Kp * 2 + 255) & ~(size_t)255 : 0;
-            p.part_bytes = splits > 1 ? (size_t)splits * Mp * Np * sizeof(float) : 0;
-            // A dW of few tiles against the K-splitting kernel, with the copies of padded
-            // operands and the optimiser's bytes: 832 x 2368 over 1640 rows takes two
-            // copies, the GEMM and a reduction, 41 us, against 25 in one launch; 2048 x 2048
-            // over 16384 rows 163 against 220.
-            if (dw && wave && !gemm_dma_tile_forced()) {
-                const double elems = (double)g.M * g.N;
-                dma_us += elems * 26.0 / 7.0e6 + (splits > 1 ? 3.0 + elems * 4.0 * splits / 4.5e6 : 0.0);
-                if (p.pad_a) dma_us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
-                if (p.pad_b) dma_us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
-                if (wave_us < 0.9 * dma_us) {
-                    p = GemmPlan{};
-                    p.tile = 256;
-                    p.splits = 1;
-                    p.Mp = g.M;
-                    p.Np = g.N;
-                    p.Kp = g.K;
-                    take_wave();
-                }
-            }
-            // padded copies against the operands as stored on 128x128 tiles
-            if (!dw && !in_place && (p.pad_a || p.pad_b) && gemm_dma_rag_ok(g) && !gemm_dma_tile_forced()) {
-                double us = 8.0 + std::ceil(tiles / 256.0) * (Kp / 128) * 3.2;
-                if (p.pad_a) us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
-                if (p.pad_b) us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
-                if (1.1 * dma128_us(g) < us) {
-                    p = GemmPlan{};
-                    p.dma = p.rag = true;
-                    p.tile = 128;
-                    p.splits = 1;
-                    p.Mp = g.M;
-                    p.Np = g.N;
-                    p.Kp = g.K;
-                }
-            }
-            return p;
-        }
-    }
-    if (g.dtype == SKL_F16 && !dw && !in_place && !gemm_dma_tile_forced()) {
-        const bool whole = g.M % 256 == 0 && g.N % 256 == 0 && gemm_dma_shape_ok(g);
-        const double us = whole ? dma128_us(g) : 1.1 * dma128_us(g);
-        if ((whole || gemm_dma_rag_ok(g)) && (!wave || us < wave_us) && us < staged_us(g)) {
-            p.dma = true;
-            p.rag = !whole;
-            p.tile = 128;
-            return p;
-        }
-    }
-    // grids that leave those tiles' GPU mostly idle: the K-splitting kernel
-    if (wave && wave_us < staged_us(g)) {
-        take_wave();
-        return p;
-    }
-    // register-staged kernels; split-K for small dW grids
-    if (dw) {
-        uint32_t tiles = gemm_tiles(g.dtype, g.M, g.N);
-        const uint32_t bk = gemm_bk(g.dtype);
-        // fp32: 128x128 tiles split over the batch rather than the 64x64 tiles a
-        // small grid would otherwise get (C2's 1024 x 1024 dW over 4096 rows: 4
-        // slices of 64 tiles, 103 -> 77 us, against 256 whole 64x64 tiles)
-        if (g.dtype == SKL_F32 && t128 < 160 && g.K >= 8 * 4 * bk) {
-            tiles = t128;
-            p.tile = 128;
-        }
-        if (tiles < 160 && g.K >= 8 * bk) {
-            uint32_t splits = (256 + tiles - 1) / tiles;
-            const uint32_t max_splits = g.K / (4 * bk);
-            if (splits > max_splits) splits = max_splits;
-            if (splits > 16) splits = 16;
-            if (splits >= 2) {
-                p.splits = splits;
-                p.part_bytes = (size_t)splits * g.M * g.N * sizeof(float);
-            }
+            p.part_bytes = (size_t)splits * g.M * g.N * sizeof(float);
         }
     }
     return p;
 }
 
-enum class GemmKind { Dma, Staged, Wave };
+// Time (us) of a dW of at most 16 columns, a stream over X, from 64 MB of it on (below, the
+// K-splitting kernel's one launch is ahead).  The streaming kernel: 4.3 TB/s
+// (fp16) and 4.8 (fp32) and the reduction's serial walk over its slices.  The K-splitting
+// kernel cannot be faster than ~5 TB/s, or 2.8 where rows are not 16-byte aligned or, in
+// fp16, the odd pitch of either operand takes it through registers.  Streaming kernel
+// against it: f16 4096 x 4096 -> 10 19 us, 16; 16384 x 2048 -> 10 26, 23; 9406 x 38336 -> 8 180, 144; 18807 x 29256 ->
+// 7 255, 408; f32 42395 x 4032 -> 5 141, 117; 93006 x 5038 -> 11 403, 918.  Above 2 GiB of X
+// only the streaming kernel takes it (the other's 32-bit offsets in a slice).
+double skinny_us(const GemmLaunch &g) {
+    const double bytes = (double)g.M * g.K * (g.dtype == SKL_F16 ? 2.0 : 4.0);
+    return 8.0 + bytes / (g.dtype == SKL_F16 ? 4.3e6 : 4.8e6) + 0.06 * skinny_dw_slices(g.K, g.M);
+}
+double narrow_wave_us(const GemmLaunch &g) {
+    const uint32_t esz = g.dtype == SKL_F16 ? 2 : 4;
+    const bool rows16 = (uint64_t)g.lda * esz % 16 == 0 && aligned16(g.A) && wave_dword_rows(g);
+    return 6.0 + (double)g.M * g.K * esz / (rows16 ? 5.0e6 : 2.8e6);
+}
+
+GemmPlan plan_route(const GemmLaunch &g, const GemmRoute &route, bool in_place) {
+    GemmPlan p{};
+    double us;
+    bool ok = true;
+    switch (route.kind) {
+    case Route::Staged: p = plan_staged(g); break;
+    case Route::Dma: ok = plan_dma(g, &p, &us); break;
+    case Route::Dma128: ok = !in_place && plan_dma128(g, &p); break;
+    case Route::Skinny: ok = plan_skinny(g, &p); break;
+    default: {
+        uint32_t splits = g.op == Op::DwOpt ? 16 : 1, tile = gemm_wave_tile(g, &splits, &us);
+        if (route.tile) {
+            tile = route.tile;
+            splits = g.op == Op::DwOpt && route.splits ? route.splits : 1;
+        }
+        ok = !in_place && plan_wave(g, tile, splits, &p);
+        p.waves = route.waves;
+    }
+    }
+    p.refused = !ok;
+    return p;
+}
+
+// in_place: the output overlaps an operand (a caller's dx over d_prenorm, a layer fed its own
+// output).  The K-splitting kernel's many small tiles would overwrite rows that others have
+// yet to read.
+GemmPlan plan_gemm(const GemmLaunch &g, const GemmRoute &route, bool in_place = false) {
+    if (route.kind != Route::Planned) return plan_route(g, route, in_place);
+    GemmPlan p{}, q{};
+    const bool dw = g.op == Op::DwOpt;
+    // a dW may go in batch slices (partial planes in the workspace) where the register-
+    // staged kernels would split it too: below 160 tiles of 128x128 and from 8 k-tiles on
+    const uint32_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128);
+    double wave_us = 0.0, dma_us = 0.0;
+    uint32_t wave_splits = dw && t128 < 160 && g.K >= 8 * gemm_bk(g.dtype) ? 16 : 1;
+    const uint32_t wave = in_place ? 0 : gemm_wave_tile(g, &wave_splits, &wave_us);
+    // outputs of at most 16 columns: any larger tile is >90% padding
+    if (dw && g.N <= 16) {
+        const bool w = plan_wave(g, wave, wave_splits, &p);
+        const bool large = (uint64_t)g.M * g.K * (g.dtype == SKL_F16 ? 2 : 4) >= (64ull << 20);
+        if (plan_skinny(g, &q) && (!w || (large && std::fmax(wave_us, narrow_wave_us(g)) > 0.9 * skinny_us(g))))
+            return q;
+        if (w) return p;
+    }
+    if (g.N <= 16 && plan_wave(g, wave, wave_splits, &p)) return p;
+    if (plan_dma(g, &p, &dma_us)) {
+        const uint32_t tiles = (p.Mp / 256) * (p.Np / 256);
+        // A dW of few tiles against the K-splitting kernel, with the copies of padded
+        // operands and the optimiser's bytes: 832 x 2368 over 1640 rows takes two
+        // copies, the GEMM and a reduction, 41 us, against 25 in one launch; 2048 x 2048
+        // over 16384 rows 163 against 220.
+        if (dw && wave && !gemm_dma_tile_forced()) {
+            const double elems = (double)g.M * g.N;
+            dma_us += elems * 26.0 / 7.0e6 + (p.splits > 1 ? 3.0 + elems * 4.0 * p.splits / 4.5e6 : 0.0);
+            if (p.pad_a) dma_us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
+            if (p.pad_b) dma_us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
+            if (wave_us < 0.9 * dma_us && plan_wave(g, wave, wave_splits, &q)) return q;
+        }
+        // padded copies against the operands as stored on 128x128 tiles
+        if (!dw && !in_place && (p.pad_a || p.pad_b) && gemm_dma_rag_ok(g) && !gemm_dma_tile_forced()) {
+            double us = 8.0 + std::ceil(tiles / 256.0) * (p.Kp / 128) * 3.2;
+            if (p.pad_a) us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
+            if (p.pad_b) us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
+            if (1.1 * dma128_us(g) < us && plan_dma128(g, &q)) return q;
+        }
+        return p;
+    }
+    if (!in_place && !gemm_dma_tile_forced() && plan_dma128(g, &p)) {
+        const double us = p.rag ? 1.1 * dma128_us(g) : dma128_us(g);
+        if ((!wave || us < wave_us) && us < staged_us(g)) return p;
+    }
+    // grids that leave those tiles' GPU mostly idle: the K-splitting kernel
+    if (wave && wave_us < staged_us(g) && plan_wave(g, wave, wave_splits, &p)) return p;
+    return plan_staged(g);
+}
+
+// A route as SOKLYN_GEMM_ROUTE writes it; unset, or a name it does not know: as planned.
+void parse_route(const char *e, GemmRoute *r) {
+    *r = GemmRoute{};
+    if (!e) return;
+    if (!strcmp(e, "staged")) r->kind = Route::Staged;
+    if (!strcmp(e, "dma")) r->kind = Route::Dma;
+    if (!strcmp(e, "dma128")) r->kind = Route::Dma128;
+    if (!strcmp(e, "skinny")) r->kind = Route::Skinny;
+    unsigned t = 0, w = 0, sp = 0;
+    if (sscanf(e, "wave:%u:%u:%u", &t, &w, &sp) >= 1) *r = GemmRoute{Route::Wave, t, w, sp};
+}
+
+enum class GemmKind { Dma, Staged, Wave, SkinnyDw };
 
 // One GEMM launch; when skl_ctx_time_next_gemm armed a pair of events, the GEMM
 // kernel's own dispatch records them (no marker packets in the stream).
-hipError_t timed_gemm(skl_ctx *ctx, const GemmLaunch &g0, GemmKind kind) {
+hipError_t timed_gemm(skl_ctx *ctx, const GemmLaunch &g0, GemmKind kind, float *partials = nullptr) {
     GemmLaunch g = g0;
     g.time_start = ctx->gemm_start;
     g.time_stop = ctx->gemm_stop;
@@ -612,6 +711,7 @@ hipError_t timed_gemm(skl_ctx *ctx, const GemmLaunch &g0, GemmKind kind) {
     case GemmKind::Dma: return launch_gemm_dma(g, ctx->stream);
     case GemmKind::Staged: return launch_gemm(g, ctx->stream);
     case GemmKind::Wave: return launch_gemm_wave(g, ctx->stream);
+    case GemmKind::SkinnyDw: return launch_skinny_dw(g, partials, g.splits, ctx->stream);
     }
     return hipSuccess;
 }
@@ -627,11 +727,13 @@ enum : uint32_t { KEEP_A = 1, KEEP_B = 2 };
 int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool full_out = false,
                   const VecOptArgs *vec = nullptr, bool *vec_done = nullptr, uint32_t keep = 0) {
     if (vec_done) *vec_done = false;
+    SKL_CHECK(!p.refused, SKL_ERR_INVALID_CONFIGURATION);
     char *wa = ws, *wb = ws + p.a_bytes, *wpart = ws + p.a_bytes + p.b_bytes;
     const OptEpi oe = g.opt;
     const uint32_t M = g.M, N = g.N;
     if (p.wave) {
         g.tile = p.wave;
+        g.waves = p.waves;
         if (p.splits > 1) {
             g.op = Op::DwPartial;
             g.splits = p.splits;
@@ -647,6 +749,9 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
             if (vec_done) *vec_done = true;
         }
         SKL_TRY(timed_gemm(ctx, g, GemmKind::Wave));
+    } else if (p.skinny) {
+        g.splits = p.splits;
+        SKL_TRY(timed_gemm(ctx, g, GemmKind::SkinnyDw, reinterpret_cast<float *>(wpart)));
     } else if (p.dma) {
         // a d_prenorm_h padded by the GEMM before (or padded now into a kept slot),
         // else a padded copy in the workspace
@@ -744,15 +849,15 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
         g.tile = p.tile;
         SKL_TRY(timed_gemm(ctx, g, GemmKind::Staged));
     }
-    if (p.splits > 1) {
+    if (p.splits > 1 || p.skinny) {
         DwReduceArgs d{};
         d.dtype = g.dtype;
         d.rows = M;
         d.n = N;
         d.splits = p.splits;
         d.partials = reinterpret_cast<const float *>(wpart);
-        d.plane = p.dma ? (uint64_t)p.Mp * p.Np : p.wave ? g.st.split_stride : (uint64_t)M * N;
-        d.pld = p.dma ? p.Np : N;
+        d.plane = p.dma ? (uint64_t)p.Mp * p.Np : p.wave ? g.st.split_stride : (uint64_t)M * (p.skinny ? 16 : N);
+        d.pld = p.dma ? p.Np : p.skinny ? 16 : N;
         d.e = oe;
         if (vec) {
             d.with_vec = 1;
@@ -887,6 +992,7 @@ int32_t skl_ctx_create(int32_t ordinal, uint32_t tile_dim, skl_ctx **out) {
         const char *e = getenv("SOKLYN_PAD_KEEP");
         c->keep_pads = !(e && atoi(e) == 0);
     }
+    parse_route(getenv("SOKLYN_GEMM_ROUTE"), &c->route);
     {
         const int32_t sr = scratch_address(ordinal, &c->scratch);
         if (sr != SKL_OK) {
@@ -1064,7 +1170,7 @@ int32_t skl_dense_forward(skl_ctx *ctx, const skl_dense_desc *b, const void *in,
     if (g.fwd.fuse_act)
         in_place = in_place || overlaps(in, in_sz, b->predrop, o_sz) || overlaps(in, in_sz, b->out, o_sz) ||
                    (use_dropout && overlaps(in, in_sz, b->mask, o_sz));
-    const GemmPlan plan = plan_gemm(g, in_place);
+    const GemmPlan plan = plan_gemm(g, ctx->route, in_place);
     if ((r = ensure_ws(ctx, plan.bytes()))) return r;
     if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws)))) return r;
 
@@ -1222,7 +1328,7 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     g.B = next->w;
     g.splits = 1;
     g.op = Op::InputGrad;
-    const GemmPlan plan = plan_gemm(g);
+    const GemmPlan plan = plan_gemm(g, ctx->route);
 
     // A next layer of at most 16 outputs: its GEMM would pad k to 128, so the
     // error kernel forms s = next.d_prenorm . next.W^T itself, per element, from
@@ -1233,7 +1339,8 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     // beyond, its many short tiles are not: 4096 x 2048 27 -> 35, 12345 x 512 23 -> 29.
     const size_t esz = cur->dtype == SKL_F16 ? 2 : 4, cells = (size_t)batch * cur->outputs;
     const bool small = plan.wave && cur->outputs % 4 == 0 && cells <= (size_t(1) << 21);
-    if (next->outputs <= 16 && !small) {
+    const Route route = ctx->route.kind;
+    if (next->outputs <= 16 && (route == Route::Planned ? !small : route == Route::Skinny)) {
         uint32_t splits = 0;
         if ((r = ensure_cols(ctx, cur, batch, 2, &splits))) return r;
         const size_t a_bytes = ((size_t)batch * 16 * esz + 255) & ~(size_t)255;
@@ -1406,7 +1513,7 @@ static int32_t backward_impl(skl_ctx *ctx, const skl_dense_desc *b, const void *
     g.splits = 1;
     g.op = Op::DwOpt;
     g.opt = oe;
-    const GemmPlan plan = plan_gemm(g);
+    const GemmPlan plan = plan_gemm(g, ctx->route);
     const size_t gemm_bytes = (plan.bytes() + 255) & ~(size_t)255;
     const size_t col_bytes = cached ? 0 : (size_t)csplits * 3 * N * sizeof(float);
     if ((r = ensure_ws(ctx, gemm_bytes + col_bytes))) return r;
@@ -1576,7 +1683,7 @@ int32_t skl_dense_input_grad(skl_ctx *ctx, const skl_dense_desc *b, uint32_t bat
     const size_t esz = f16 ? 2 : 4, dx_sz = (size_t)batch * b->inputs * sizeof(float);
     const bool in_place = overlaps(dx, dx_sz, g.A, (size_t)batch * b->outputs * esz) ||
                           overlaps(dx, dx_sz, g.B, (size_t)b->inputs * b->outputs * esz);
-    const GemmPlan plan = plan_gemm(g, in_place);
+    const GemmPlan plan = plan_gemm(g, ctx->route, in_place);
     if ((r = ensure_ws(ctx, plan.bytes()))) return r;
     if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws), false, nullptr, nullptr, f16 ? KEEP_A : 0)))
         return r;
@@ -1596,6 +1703,34 @@ int32_t skl_dense_input_grad(skl_ctx *ctx, const skl_dense_desc *b, uint32_t bat
             c.call = ctx->calls;
     }
     return finish(ctx);
+}
+
+// For tests on a machine without a GPU (not part of soklyn_hip.h): the kernel that the planner
+// gives a forward (op 0), input gradient (1) or dW (2) whose output is M x N over K, rows
+// without padding and buffers aligned, in SOKLYN_GEMM_ROUTE's words.  The text is the thread's
+// own until its next call.
+const char *skl_diag_gemm_route(uint32_t dtype, uint32_t op, uint32_t M, uint32_t N, uint32_t K) {
+    static thread_local char text[64];
+    GemmLaunch g{};
+    g.dtype = dtype;
+    g.op = op == 0 ? Op::Fwd : op == 1 ? Op::InputGrad : Op::DwOpt;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.lda = op == 2 ? M : K;
+    g.ldb = op == 1 ? K : N;
+    g.a_kcontig = op != 2;
+    g.b_kcontig = op == 1;
+    g.A = g.B = reinterpret_cast<const void *>(uintptr_t(256));   // looked at for its alignment only
+    g.splits = 1;
+    g.fwd.ldc = g.st.ldc = g.opt.ldc = N;
+    const GemmPlan p = plan_gemm(g, GemmRoute{});
+    const char *kind = p.skinny ? "skinny" : p.wave ? "wave" : !p.dma ? "staged" : p.Kp == K && p.Mp == M && p.Np == N && p.tile == 128 && op != 2 ? "dma128" : "dma";
+    if (p.wave)
+        snprintf(text, sizeof(text), "wave:%u:%u:%u", p.wave, p.waves ? p.waves : gemm_wave_waves(g, p.wave), p.splits);
+    else
+        snprintf(text, sizeof(text), "%s:%u:%u", kind, p.dma ? p.tile : 0u, p.splits);
+    return text;
 }
 
 }  // extern "C"

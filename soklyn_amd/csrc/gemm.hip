@@ -334,6 +334,153 @@ uint32_t gemm_dma_splits(uint32_t K, uint32_t splits) {
     return (K + kps - 1) / kps;
 }
 
+// ---- dW of at most 16 columns ---------------------------------------------------------
+// A stream over X, whatever its size and pitch (64-bit offsets): 1024 workgroups of
+// 256 columns of X and a batch slice keep the GPU's loads in flight, and their short sums are
+// the more precise the longer the batch (f32 142860 x 1603 -> 10: 6.0e-7 against 64 bits, 1.07e-6 on the K-splitting
+// kernel).  The planner's skinny_us says where it is taken, with the times of both.
+constexpr uint32_t SKINNY_N = 16;
+
+// dW partial sums, thread per W row: thread k of workgroup (x, y) walks the batch rows
+// of slice y in order, acc[n] += X[b][k] * dP[b][n], with 64 rows of dP (fp32) at a
+// time in LDS (16-byte broadcast reads) and the X loads of 16 rows issued before
+// their FMAs; partials[y][k][0..15].
+__global__ void __launch_bounds__(256) skinny_dw_kernel(GemmShape sh, const float *__restrict__ X,
+                                                        const float *__restrict__ dp, float *__restrict__ partials,
+                                                        uint32_t per) {
+    __shared__ __attribute__((aligned(16))) float dps[64][SKINNY_N];
+    const uint32_t K = sh.M, N = sh.N;          // output [K x N]; reduction over sh.K batch rows
+    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t r0 = blockIdx.y * per;
+    const uint32_t r1 = min(sh.K, r0 + per);
+    float acc[SKINNY_N];
+#pragma unroll
+    for (int n = 0; n < (int)SKINNY_N; ++n) acc[n] = 0.0f;
+    for (uint32_t rb = r0; rb < r1; rb += 64) {
+        const uint32_t nrows = min(64u, r1 - rb);
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < 64 * SKINNY_N; i += 256) {
+            const uint32_t r = i / SKINNY_N, n = i % SKINNY_N;
+            dps[r][n] = (r < nrows && n < N) ? dp[(uint64_t)(rb + r) * sh.ldb + n] : 0.0f;
+        }
+        __syncthreads();
+        if (k < K) {
+            for (uint32_t r0b = 0; r0b < nrows; r0b += 16) {
+                float xv[16];
+#pragma unroll
+                for (uint32_t u = 0; u < 16; ++u)
+                    xv[u] = r0b + u < nrows ? X[(uint64_t)(rb + r0b + u) * sh.lda + k] : 0.0f;
+#pragma unroll
+                for (uint32_t u = 0; u < 16; ++u) {
+                    if (r0b + u >= nrows) break;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const floatx4 d = *reinterpret_cast<const floatx4 *>(&dps[r0b + u][4 * q]);
+                        acc[4 * q + 0] = fmaf(xv[u], d[0], acc[4 * q + 0]);
+                        acc[4 * q + 1] = fmaf(xv[u], d[1], acc[4 * q + 1]);
+                        acc[4 * q + 2] = fmaf(xv[u], d[2], acc[4 * q + 2]);
+                        acc[4 * q + 3] = fmaf(xv[u], d[3], acc[4 * q + 3]);
+                    }
+                }
+            }
+        }
+    }
+    if (k >= K) return;
+    float *p = partials + ((uint64_t)blockIdx.y * K + k) * SKINNY_N;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<floatx4 *>(p + 4 * q) = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+}
+
+// The same on MFMA (fp16; dP as its fp16 copy, the dW GEMMs' operand): thread t
+// of workgroup (x, y) loads column k = 256 x + t of X for 32 batch rows at a time
+// (coalesced 2-byte loads, all 32 issued before use) and writes them to LDS
+// transposed (xt[t][0..31], one 64-byte run); the 32 x 16 block of dP goes to
+// pt[n][0..31].  Wave w then runs v_mfma_f32_16x16x32_f16 on its 4 tiles of 16 W
+// rows: src0 lane l = xt[16 q + l % 16][8 (l / 16) ..] (X^T), src1 lane l =
+// pt[l % 16][8 (l / 16) ..] (dP); lane l ends with rows 4 (l / 16) .. + 3 of column
+// l % 16 of the tile.  LDS rows of 40 halves (80 bytes) keep the 16-byte reads of
+// 16 lanes in distinct banks.  partials[y][k][0..15] as in skinny_dw_kernel.
+__global__ void __launch_bounds__(256) skinny_dw_mfma_kernel(GemmShape sh, const half_t *__restrict__ X,
+                                                             const half_t *__restrict__ dp16,
+                                                             float *__restrict__ partials, uint32_t per) {
+    __shared__ __attribute__((aligned(16))) half_t xt[256][40];
+    __shared__ __attribute__((aligned(16))) half_t pt[SKINNY_N][40];
+    const uint32_t K = sh.M, N = sh.N;          // output [K x N]; reduction over sh.K batch rows
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t k0 = blockIdx.x * 256, k = k0 + tid;
+    const uint32_t r0 = blockIdx.y * per;
+    const uint32_t r1 = min(sh.K, r0 + per);
+    floatx4 acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t rb = r0; rb < r1; rb += 32) {
+        const uint32_t nrows = min(32u, r1 - rb);
+        half_t xv[32];
+#pragma unroll
+        for (uint32_t u = 0; u < 32; ++u)
+            xv[u] = (u < nrows && k < K) ? X[(uint64_t)(rb + u) * sh.lda + k] : (half_t)0;
+        half_t pv[2];
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+            const uint32_t i = tid + 256 * h, u = i >> 4, n = i & 15u;   // 32 rows x 16 columns
+            pv[h] = (u < nrows && n < N) ? dp16[(uint64_t)(rb + u) * sh.ldb + n] : (half_t)0;
+        }
+        __syncthreads();   // the previous block's fragments are read
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<halfx8 *>(&xt[tid][8 * q]) = *reinterpret_cast<const halfx8 *>(&xv[8 * q]);
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+            const uint32_t i = tid + 256 * h;
+            pt[i & 15u][i >> 4] = pv[h];
+        }
+        __syncthreads();
+        const halfx8 b = *reinterpret_cast<const halfx8 *>(&pt[lane & 15u][8 * (lane >> 4)]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const halfx8 a = *reinterpret_cast<const halfx8 *>(&xt[wave * 64 + 16 * q + (lane & 15u)][8 * (lane >> 4)]);
+            acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[q], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t ko = k0 + wave * 64 + 16 * q + 4 * (lane >> 4) + r;
+            if (ko < K) partials[((uint64_t)blockIdx.y * K + ko) * SKINNY_N + (lane & 15u)] = acc[q][r];
+        }
+    }
+}
+
+uint32_t skinny_dw_slices(uint32_t rows, uint32_t K) {
+    const uint32_t col_blocks = (K + 255) / 256;
+    uint32_t sl = (1024 + col_blocks - 1) / col_blocks;
+    const uint32_t cap = (rows + 63) / 64;
+    if (sl > cap) sl = cap;
+    return sl < 1 ? 1 : sl;
+}
+
+hipError_t launch_skinny_dw(const GemmLaunch &g, float *partials, uint32_t slices, hipStream_t s) {
+    if (g.N > SKINNY_N || !g.M || !g.K || !slices || g.a_kcontig || g.b_kcontig ||
+        (reinterpret_cast<uintptr_t>(partials) & 15u))
+        return hipErrorInvalidValue;
+    GemmShape sh{};
+    sh.M = g.M;          // W rows (inputs)
+    sh.N = g.N;          // W cols (outputs)
+    sh.K = g.K;          // batch rows
+    sh.lda = g.lda;      // X row pitch
+    sh.ldb = g.ldb;      // d_prenorm row pitch
+    const uint32_t per = (g.K + slices - 1) / slices;
+    const dim3 grid((g.M + 255) / 256, slices);
+    if (g.dtype == 1)
+        launch_timed(g, skinny_dw_mfma_kernel, grid, dim3(256), s, sh, reinterpret_cast<const half_t *>(g.A),
+                     reinterpret_cast<const half_t *>(g.B), partials, per);
+    else
+        launch_timed(g, skinny_dw_kernel, grid, dim3(256), s, sh, reinterpret_cast<const float *>(g.A),
+                     reinterpret_cast<const float *>(g.B), partials, per);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm(const GemmLaunch &g, hipStream_t s) {
     if (g.M == 0 || g.N == 0) return hipSuccess;
     if (gemm_direct_ok(g)) return launch_gemm_dma(g, s);

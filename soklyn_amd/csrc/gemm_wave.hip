@@ -78,37 +78,44 @@ static hipError_t run_wave_t(const GemmLaunch &g, const typename Epi::Params &p0
     return hipGetLastError();
 }
 
+// Waves per tile, on the planner's choice of 64x64 tiles and the one count of the others.
+uint32_t gemm_wave_waves(const GemmLaunch &g, uint32_t tile) {
+    if (tile == 16) return 16;
+    const bool reg = !wave_dword_rows(g);
+    if (tile == 32) return g.dtype == 0 || reg ? 8 : 4;
+    if (reg) return 4;
+    const uint32_t w = wave_share(g.dtype, tiles_of(g, 64));
+    return w == 1 && g.op == Op::DwOpt ? 4 : w;   // one wave: too few for the parameter update
+}
+
 template <typename T, class Epi, bool AK, bool BK>
 static hipError_t run_wave(const GemmLaunch &g, const typename Epi::Params &p, hipStream_t s) {
+    const uint32_t waves = g.waves ? g.waves : gemm_wave_waves(g, g.tile);
     if constexpr (sizeof(T) == 2) {
         if (!wave_dword_rows(g)) {
-            switch (g.tile) {
-            case 16: return run_wave_t<T, Epi, AK, BK, true, 1, 16, 1, 4>(g, p, s);
-            case 32: return run_wave_t<T, Epi, AK, BK, true, 2, 8, 1, 4>(g, p, s);
-            case 64: return run_wave_t<T, Epi, AK, BK, true, 4, 4, 1, 2>(g, p, s);
+            switch (g.tile * 32 + waves) {
+            case 16 * 32 + 16: return run_wave_t<T, Epi, AK, BK, true, 1, 16, 1, 4>(g, p, s);
+            case 32 * 32 + 8: return run_wave_t<T, Epi, AK, BK, true, 2, 8, 1, 4>(g, p, s);
+            case 64 * 32 + 4: return run_wave_t<T, Epi, AK, BK, true, 4, 4, 1, 2>(g, p, s);
             }
             return hipErrorInvalidValue;
         }
-        switch (g.tile) {
-        case 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
-        case 32: return run_wave_t<T, Epi, AK, BK, false, 2, 4, 2, 2>(g, p, s);
-        case 64:
-            return wave_share(1, tiles_of(g, 64)) == 2 ? run_wave_t<T, Epi, AK, BK, false, 4, 2, 1, 2>(g, p, s)
-                                                       : run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
+        switch (g.tile * 32 + waves) {
+        case 16 * 32 + 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
+        case 32 * 32 + 4: return run_wave_t<T, Epi, AK, BK, false, 2, 4, 2, 2>(g, p, s);
+        case 64 * 32 + 2: return run_wave_t<T, Epi, AK, BK, false, 4, 2, 1, 2>(g, p, s);
+        case 64 * 32 + 4: return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
         }
     } else {
-        switch (g.tile) {
-        case 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
-        case 32: return run_wave_t<T, Epi, AK, BK, false, 2, 8, 1, 4>(g, p, s);
-        case 64:
-            switch (wave_share(0, tiles_of(g, 64))) {
-            case 8: return run_wave_t<T, Epi, AK, BK, false, 4, 8, 1, 2>(g, p, s);
-            case 2: return run_wave_t<T, Epi, AK, BK, false, 4, 2, 1, 2>(g, p, s);
-            case 1:
-                if constexpr (!std::is_same<typename Epi::Params, OptEpi>::value)
-                    return run_wave_t<T, Epi, AK, BK, false, 4, 1, 1, 2>(g, p, s);
-            }
-            return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
+        switch (g.tile * 32 + waves) {
+        case 16 * 32 + 16: return run_wave_t<T, Epi, AK, BK, false, 1, 16, 2, 4>(g, p, s);
+        case 32 * 32 + 8: return run_wave_t<T, Epi, AK, BK, false, 2, 8, 1, 4>(g, p, s);
+        case 64 * 32 + 8: return run_wave_t<T, Epi, AK, BK, false, 4, 8, 1, 2>(g, p, s);
+        case 64 * 32 + 4: return run_wave_t<T, Epi, AK, BK, false, 4, 4, 1, 2>(g, p, s);
+        case 64 * 32 + 2: return run_wave_t<T, Epi, AK, BK, false, 4, 2, 1, 2>(g, p, s);
+        case 64 * 32 + 1:
+            if constexpr (!std::is_same<typename Epi::Params, OptEpi>::value)
+                return run_wave_t<T, Epi, AK, BK, false, 4, 1, 1, 2>(g, p, s);
         }
     }
     return hipErrorInvalidValue;

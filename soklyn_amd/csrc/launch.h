@@ -98,6 +98,7 @@ struct GemmLaunch {
     uint32_t splits;      // split-K factor (DwPartial only; 1 otherwise)
     uint32_t tile;        // direct-to-LDS kernel: 128 (4 waves, two workgroups per CU) or 256 (0 = 256);
                           // fp32 register-staged kernel: 128 asks for 128x128 tiles on any grid
+    uint32_t waves;       // K-splitting kernel: waves per tile (0: gemm_wave_waves)
     uint32_t mv, nv;      // real output extent when A / B are zero-padded copies (0 = M, N)
     // direct-to-LDS kernel: the launch covers output rows [m_begin, m_begin + m_rows)
     // only (0, 0: all M), m_begin a multiple of 256 and m_rows of the tile edge;
@@ -122,11 +123,16 @@ hipError_t launch_gemm_dma(const GemmLaunch &g, hipStream_t stream);
 bool gemm_dma_shape_ok(const GemmLaunch &g);
 // Its form for operands as stored (128x128 tiles; forward and input gradient).
 bool gemm_dma_rag_ok(const GemmLaunch &g);
+// dW of at most 16 columns, the batch in slices: partial sums of X^T . d_prenorm (fp32) into
+// partials [slices x M x 16]; skinny_dw_slices gives the slice count.
+uint32_t skinny_dw_slices(uint32_t rows, uint32_t K);
+hipError_t launch_skinny_dw(const GemmLaunch &g, float *partials, uint32_t slices, hipStream_t stream);
 // The K-splitting kernel (gemm_wave.h) on output tiles of edge g.tile (16, 32 or 64): any
 // M, N, K >= 1, operands as stored; DwPartial in g.splits slices of gemm_wave_slice k.
 // gemm_wave_tile picks the tile, and for a dW up to *splits slices, and estimates its time
 // (0: the kernel does not take the operands).
 hipError_t launch_gemm_wave(const GemmLaunch &g, hipStream_t stream);
+uint32_t gemm_wave_waves(const GemmLaunch &g, uint32_t tile);
 bool gemm_wave_ok(const GemmLaunch &g, uint32_t splits);
 bool wave_dword_rows(const GemmLaunch &g);
 uint32_t gemm_wave_slice(uint32_t K, uint32_t splits);
