@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/soklyn_hip.h"
+#include "gemm_cost.h"
 #include "launch.h"
 
 using namespace skl;
@@ -322,21 +323,23 @@ int32_t pad_keep(skl_ctx *ctx, const void *p, uint32_t rows, uint32_t cols, uint
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // ---- GEMM planning ------------------------------------------------------------------
-// Every DenseBlock GEMM runs on the fastest path its shapes allow:
+// Every DenseBlock GEMM runs on the path with the least estimated time (gemm_cost.h):
 //  * the 256x256 direct-to-LDS kernel (fp16).  Operands it cannot read as
 //    stored (M, N not whole 256 tiles, K not a multiple of 128, rows not
 //    16-byte aligned) are first copied into the workspace zero-padded to those
-//    multiples, and the epilogue stops at the real M x N.  Used when the padded
+//    multiples, and the epilogue stops at the real M x N.  Considered when the padded
 //    output wastes at most half of its grid and there are at least 192 tiles,
 //    counting the split-K slices a dW with fewer tiles than CUs is given (their
-//    fp32 partial sums, in the workspace, are reduced by the optimiser kernel).
-//  * the K-splitting kernel on small tiles (gemm_wave.h), for outputs that would leave
-//    those tiles' GPU mostly idle and for at most 16 columns: operands as stored, no
-//    workspace but the partial planes of a dW over a long batch;
+//    fp32 partial sums, in the workspace, are reduced by the optimiser kernel);
+//  * its form on 128x128 tiles over operands as stored (forward and input gradient);
+//  * the K-splitting kernel on small tiles (gemm_wave.h): operands as stored, no
+//    workspace but the partial planes of a dW over a long batch.  Outputs of at most 16
+//    columns take it whatever the estimate, as any larger tile is mostly padding;
 //  * the streaming kernel for a dW of at most 16 columns over a large X whose rows the
-//    K-splitting kernel reads slowly or not at all (skinny_us);
-//  * the register-staged kernels otherwise (large fp32; small fp16 with little k to
-//    reduce), with the same split-K for small dW grids.
+//    K-splitting kernel reads slowly or not at all;
+//  * the register-staged kernels (some large fp32; some fp16 with little k to reduce; an
+//    output over its own operand; operands past the others' 32-bit offsets), with split-K
+//    for small dW grids.
 struct GemmPlan {
     uint32_t wave;             // K-splitting kernel: its tile edge (0: another kernel)
     uint32_t waves;            // ... and its waves per tile (0: the launcher's choice)
@@ -350,6 +353,7 @@ struct GemmPlan {
     uint32_t Mp, Np, Kp;       // dims the kernel runs on
     uint32_t splits;           // split-K slices of a dW (then DwPartial + reduce)
     size_t a_bytes, b_bytes, part_bytes;
+    double us;                 // plan_gemm's estimate, for a hidden error of the whole call
     size_t bytes() const { return a_bytes + b_bytes + part_bytes; }
 };
 
@@ -414,18 +418,20 @@ uint32_t dw_dma_splits(uint32_t tiles, uint32_t Kp, uint64_t out_elems, uint32_t
 // 12544 x 1536 GEMMs (294 tiles) one 256x256 round plus a 128x128 launch ran
 // 3-4 us slower than 128x128 alone (a launch of fewer 128x128 workgroups than
 // CUs takes as long as a full round of them), hence two rounds at least.
-uint32_t dma_tile(Op op, uint32_t Mp, uint32_t Np, uint32_t splits, uint32_t *band) {
+// *rounds: the estimate, without the band where there is one.
+uint32_t dma_tile(Op op, uint32_t Mp, uint32_t Np, uint32_t splits, uint32_t *band, double *rounds,
+                  double *band_rounds) {
     *band = 0;
-    if (const uint32_t f = gemm_dma_tile_forced()) return f;
-    if (splits > 1) return 256;
     const uint32_t R = Mp / 256, Cn = Np / 256;   // 256x256 tile rows and columns
     const double f128 = op == Op::DwOpt ? 1.25 : 1.15;
     auto rounds256 = [](double tiles) { return std::ceil(tiles / 256.0); };
     auto rounds128 = [&](double tiles256) { return std::ceil(4.0 * tiles256 / 512.0) * 0.5 * f128; };
     const double r256 = rounds256((double)R * Cn), r128 = rounds128((double)R * Cn);
-    const uint32_t tile = r128 < 0.95 * r256 ? 128u : 256u;
-    if (op != Op::Fwd && op != Op::InputGrad) return tile;
-    double best = tile == 128 ? r128 : r256;
+    const uint32_t forced = gemm_dma_tile_forced();
+    const uint32_t tile = forced ? forced : splits <= 1 && r128 < 0.95 * r256 ? 128u : 256u;
+    *rounds = *band_rounds = tile == 128 ? r128 : r256;
+    if (forced || splits > 1 || (op != Op::Fwd && op != Op::InputGrad)) return tile;
+    double best = *rounds;
     uint32_t best_rows = 0;
     for (uint32_t k = 2; k < (uint32_t)r256; ++k) {
         uint32_t r1 = 256u * k / Cn;   // tile rows filling k rounds
@@ -439,40 +445,8 @@ uint32_t dma_tile(Op op, uint32_t Mp, uint32_t Np, uint32_t splits, uint32_t *ba
     }
     if (best_rows == 0) return tile;
     *band = best_rows * 256u;
+    *band_rounds = best;
     return 256u;
-}
-
-// Estimated time (us) of the register-staged kernels, from the measurements behind
-// gemm_wave_tile.  fp16: a 128x128 tile takes ~1 us per 64 k whatever the grid, 4 us when
-// its rows are not 16-byte aligned (gathered element by element), and a second tile per
-// CU hides part of it (4096 x 1024, K 1024: 25 us; 512 x 2048, K 2048: 36; 2000 x 1531,
-// K 777: 66).  fp32: grids of at least 192 tiles of 128x128 (160 for a dW) run them in
-// rounds of 256 (4096 x 1024, K 1024: dX 70 us, forward 82; 8192 rows 133 and 147);
-// smaller ones, and any fp16 dW (2048 x 2048 over 512 rows: 31 us, 25), are behind the
-// K-splitting kernel throughout.
-double staged_us(const GemmLaunch &g) {
-    const double tiles = (double)((g.M + 127) / 128) * ((g.N + 127) / 128);
-    const bool dw = g.op == Op::DwOpt;
-    if (g.dtype == SKL_F32) {
-        if (tiles < (dw ? 160 : 192)) return 1e30;
-        return std::ceil(tiles / 256.0) * (6.0 + (g.op == Op::InputGrad ? 1.95 : 2.1) * (double)((g.K + 31) / 32)) +
-               (dw ? (double)g.M * g.N * 16.0 / 7.0e6 : 0.0);
-    }
-    if (dw) return 1e30;
-    const uint32_t a_ext = g.a_kcontig ? g.K : g.M, b_ext = g.b_kcontig ? g.K : g.N;
-    const bool vec = g.lda % 8 == 0 && g.ldb % 8 == 0 && a_ext % 8 == 0 && b_ext % 8 == 0 && aligned16(g.A) &&
-                     aligned16(g.B);
-    const double kt = (double)((g.K + 63) / 64), u = tiles / 256.0;
-    return vec ? 10.0 + kt * (u > 1.25 ? 0.8 * u : 1.0) : 15.0 + kt * (u > 1.0 ? 4.0 * u : 4.0);
-}
-
-// The same for 128x128 direct-to-LDS tiles, whose operands are read in place (2048 x 2048,
-// K 2048: 29.4 us, 33 on the K-splitting kernel; 4096 x 2048: 42, 56; dX of 4096 x 1024,
-// K 1024: 14.6, 16.5).  Not the dW, whose fused optimiser is faster on small tiles (2048 x
-// 2048 over 512 rows: 31, 25).
-double dma128_us(const GemmLaunch &g) {
-    const double u = (double)((g.M + 127) / 128) * ((g.N + 127) / 128) / 256.0, kt = (double)((g.K + 63) / 64);
-    return (g.op == Op::InputGrad ? 4.5 : 8.5) + kt * (0.5 * u > 0.65 ? 0.5 * u : 0.65);
 }
 
 GemmPlan plan_as_stored(const GemmLaunch &g) {
@@ -486,10 +460,11 @@ GemmPlan plan_as_stored(const GemmLaunch &g) {
 }
 
 // The K-splitting kernel on tiles of edge `tile`, a dW in up to `splits` batch slices.
-bool plan_wave(const GemmLaunch &g, uint32_t tile, uint32_t splits, GemmPlan *out) {
+bool plan_wave(const GemmLaunch &g, uint32_t tile, uint32_t waves, uint32_t splits, GemmPlan *out) {
     if (!tile || !gemm_wave_ok(g, splits)) return false;
     GemmPlan p = plan_as_stored(g);
     p.wave = tile;
+    p.waves = waves;
     if (splits > 1) {
         const uint32_t slice = gemm_wave_slice(g.K, splits);
         p.splits = (g.K + slice - 1) / slice;
@@ -512,16 +487,17 @@ bool plan_skinny(const GemmLaunch &g, GemmPlan *out) {
 }
 
 // The direct-to-LDS kernel on operands padded to its tiles where they are not whole, for
-// grids that fill the GPU.  *us: its estimated time, the copies included.
-bool plan_dma(const GemmLaunch &g, GemmPlan *out, double *us) {
+// grids that fill the GPU.  *us: its estimated time, the copies included, for a hidden error
+// that of the whole call.
+bool plan_dma(const GemmLaunch &g, Work w, GemmPlan *out, double *us) {
     if (g.dtype != SKL_F16 || !gemm_dma_enabled() || !g.M || !g.N || !g.K) return false;
     const bool dw = g.op == Op::DwOpt;
     const uint32_t Mp = round_up(g.M, 256), Np = round_up(g.N, 256), Kp = round_up(g.K, 128);
     // in units of 256x256 tiles whatever the kernel's tile edge
     const uint32_t tiles = (Mp / 256) * (Np / 256);
     uint32_t dw_tile = 256;
-    *us = (tiles + 255) / 256 * (Kp / 128) * 3.4;
-    const uint32_t splits = dw && tiles < 160 ? dw_dma_splits(tiles, Kp, (uint64_t)Mp * Np, &dw_tile, us) : 1;
+    double loop_us = 0.0, rounds = 0.0, band_rounds = 0.0, pad_us = 0.0;
+    const uint32_t splits = dw && tiles < 160 ? dw_dma_splits(tiles, Kp, (uint64_t)Mp * Np, &dw_tile, &loop_us) : 1;
     const bool waste_ok = (uint64_t)Mp * Np <= (uint64_t)g.M * g.N * 3 / 2;
     // the kernel's operand offsets are 32-bit
     const uint64_t a_span = g.a_kcontig ? (uint64_t)Mp * (g.lda > Kp ? g.lda : Kp)
@@ -538,7 +514,7 @@ bool plan_dma(const GemmLaunch &g, GemmPlan *out, double *us) {
     p.Np = Np;
     p.Kp = Kp;
     p.splits = splits;
-    p.tile = dma_tile(g.op, Mp, Np, splits, &p.band);
+    p.tile = dma_tile(g.op, Mp, Np, splits, &p.band, &rounds, &band_rounds);
     if (dw && dw_tile == 128 && !gemm_dma_tile_forced()) p.tile = 128;
     // A: k-contiguous [M x K] or m-contiguous [K x M]; B likewise with N
     p.pad_a = g.a_kcontig ? !dma_operand_ok(g.A, g.M, g.K, g.lda, 256, 128)
@@ -549,6 +525,13 @@ bool plan_dma(const GemmLaunch &g, GemmPlan *out, double *us) {
     p.a_bytes = p.pad_a ? ((size_t)Mp * Kp * 2 + 255) & ~(size_t)255 : 0;
     p.b_bytes = p.pad_b ? ((size_t)Np * Kp * 2 + 255) & ~(size_t)255 : 0;
     p.part_bytes = splits > 1 ? (size_t)splits * Mp * Np * sizeof(float) : 0;
+    if (p.pad_a) pad_us += 2.0 + 1e-6 * g.M * g.K;
+    if (p.pad_b) pad_us += 2.0 + 1e-6 * g.N * g.K;
+    if (dw)
+        loop_us = tiles < 160 ? loop_us : rounds * (Kp / 128) * 3.4;
+    else
+        loop_us = (w == Work::Fwd || w == Work::Store ? band_rounds : rounds) * (Kp / 128);
+    *us = dma_us(g, w, loop_us, pad_us, splits);
     *out = p;
     return true;
 }
@@ -573,8 +556,9 @@ GemmPlan plan_staged(const GemmLaunch &g) {
     const uint32_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128), bk = gemm_bk(g.dtype);
     uint32_t tiles = gemm_tiles(g.dtype, g.M, g.N);
     // fp32: 128x128 tiles split over the batch rather than the 64x64 tiles a
-    // small grid would otherwise get (C2's 1024 x 1024 dW over 4096 rows: 4
-    // slices of 64 tiles, 103 -> 77 us, against 256 whole 64x64 tiles)
+    // small grid would otherwise get (1024 x 1024 over 4096 rows: 4 slices of 64
+    // tiles, 103 -> 77 us, against 256 whole 64x64 tiles; 70 on the K-splitting
+    // kernel, which falls behind over long batches: 65536 rows 1117, 1517 there)
     if (g.dtype == SKL_F32 && t128 < 160 && g.K >= 8 * 4 * bk) {
         tiles = t128;
         p.tile = 128;
@@ -592,98 +576,84 @@ GemmPlan plan_staged(const GemmLaunch &g) {
     return p;
 }
 
-// Time (us) of a dW of at most 16 columns, a stream over X, from 64 MB of it on (below, the
-// K-splitting kernel's one launch is ahead).  The streaming kernel: 4.3 TB/s
-// (fp16) and 4.8 (fp32) and the reduction's serial walk over its slices.  The K-splitting
-// kernel cannot be faster than ~5 TB/s, or 2.8 where rows are not 16-byte aligned or, in
-// fp16, the odd pitch of either operand takes it through registers.  Streaming kernel
-// against it: f16 4096 x 4096 -> 10 19 us, 16; 16384 x 2048 -> 10 26, 23; 9406 x 38336 -> 8 180, 144; 18807 x 29256 ->
-// 7 255, 408; f32 42395 x 4032 -> 5 141, 117; 93006 x 5038 -> 11 403, 918.  Above 2 GiB of X
-// only the streaming kernel takes it (the other's 32-bit offsets in a slice).
-double skinny_us(const GemmLaunch &g) {
-    const double bytes = (double)g.M * g.K * (g.dtype == SKL_F16 ? 2.0 : 4.0);
-    return 8.0 + bytes / (g.dtype == SKL_F16 ? 4.3e6 : 4.8e6) + 0.06 * skinny_dw_slices(g.K, g.M);
-}
-double narrow_wave_us(const GemmLaunch &g) {
-    const uint32_t esz = g.dtype == SKL_F16 ? 2 : 4;
-    const bool rows16 = (uint64_t)g.lda * esz % 16 == 0 && aligned16(g.A) && wave_dword_rows(g);
-    return 6.0 + (double)g.M * g.K * esz / (rows16 ? 5.0e6 : 2.8e6);
-}
+// What a GEMM's caller does with it beyond the op: the hidden error, whose routes differ in
+// whether the GEMM's epilogue may compute it.
+struct PlanCtx {
+    bool in_place;             // the output overlaps an operand
+    bool err, err_norm;        // hidden error, of a layer with a norm
+    bool err_dma, err_wave;    // ... in the epilogue of the direct-to-LDS / K-splitting kernel
+};
 
-GemmPlan plan_route(const GemmLaunch &g, const GemmRoute &route, bool in_place) {
+GemmPlan plan_route(const GemmLaunch &g, const GemmRoute &route, const PlanCtx &c) {
     GemmPlan p{};
     double us;
     bool ok = true;
     switch (route.kind) {
     case Route::Staged: p = plan_staged(g); break;
-    case Route::Dma: ok = plan_dma(g, &p, &us); break;
-    case Route::Dma128: ok = !in_place && plan_dma128(g, &p); break;
+    case Route::Dma: ok = plan_dma(g, Work::Store, &p, &us); break;
+    case Route::Dma128: ok = !c.in_place && plan_dma128(g, &p); break;
     case Route::Skinny: ok = plan_skinny(g, &p); break;
-    default: {
-        uint32_t splits = g.op == Op::DwOpt ? 16 : 1, tile = gemm_wave_tile(g, &splits, &us);
-        if (route.tile) {
-            tile = route.tile;
-            splits = g.op == Op::DwOpt && route.splits ? route.splits : 1;
-        }
-        ok = !in_place && plan_wave(g, tile, splits, &p);
-        p.waves = route.waves;
-    }
+    default:
+        ok = !c.in_place && plan_wave(g, route.tile, route.waves,
+                                      g.op == Op::DwOpt && route.splits ? route.splits : 1, &p);
     }
     p.refused = !ok;
     return p;
 }
 
-// in_place: the output overlaps an operand (a caller's dx over d_prenorm, a layer fed its own
-// output).  The K-splitting kernel's many small tiles would overwrite rows that others have
-// yet to read.
-GemmPlan plan_gemm(const GemmLaunch &g, const GemmRoute &route, bool in_place = false) {
-    if (route.kind != Route::Planned) return plan_route(g, route, in_place);
-    GemmPlan p{}, q{};
+// The earlier routes (direct-to-LDS where its grid fills the GPU, else register-staged; the
+// streaming dW) against 128x128 direct-to-LDS tiles and the K-splitting kernel, by
+// gemm_cost.h.  In place, the small tiles of the latter two would overwrite rows that others
+// have yet to read.
+GemmPlan plan_gemm(const GemmLaunch &g, const GemmRoute &route, const PlanCtx &c = PlanCtx{}) {
+    if (route.kind != Route::Planned) return plan_route(g, route, c);
     const bool dw = g.op == Op::DwOpt;
-    // a dW may go in batch slices (partial planes in the workspace) where the register-
-    // staged kernels would split it too: below 160 tiles of 128x128 and from 8 k-tiles on
+    const Work fused = c.err_norm ? Work::ErrNorm : Work::Err;
+    const Work w = dw ? Work::Dw : g.op == Op::Fwd ? Work::Fwd : Work::Store;
+    const double err = c.err ? err_us(g, c.err_norm) : 0.0;   // behind a stored sum
     const uint32_t t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128);
-    double wave_us = 0.0, dma_us = 0.0;
-    uint32_t wave_splits = dw && t128 < 160 && g.K >= 8 * gemm_bk(g.dtype) ? 16 : 1;
-    const uint32_t wave = in_place ? 0 : gemm_wave_tile(g, &wave_splits, &wave_us);
-    // outputs of at most 16 columns: any larger tile is >90% padding
-    if (dw && g.N <= 16) {
-        const bool w = plan_wave(g, wave, wave_splits, &p);
+    GemmPlan base{}, wave{}, skinny{}, dma128{};
+    double base_us = 0.0;
+    const bool dma = plan_dma(g, c.err_dma ? fused : w, &base, &base_us);
+    if (dma && gemm_dma_tile_forced()) return base;
+    if (dma) {
+        base_us += c.err_dma ? 0.0 : err;
+    } else {
+        const uint32_t a_ext = g.a_kcontig ? g.K : g.M, b_ext = g.b_kcontig ? g.K : g.N;
+        const uint32_t v = g.dtype == SKL_F16 ? 8 : 4;
+        const bool vec = g.lda % v == 0 && g.ldb % v == 0 && a_ext % v == 0 && b_ext % v == 0 && aligned16(g.A) &&
+                         aligned16(g.B);
+        base = plan_staged(g);
+        const bool small = g.dtype == SKL_F32 && base.tile != 128 && gemm_tiles(g.dtype, g.M, g.N) != t128;
+        base_us = staged_us(g, w, base.splits, small, vec) + err;
+    }
+    base.us = base_us;
+    if (c.in_place) return base;
+    // a dW may go in batch slices where the register-staged kernels would split it too
+    const bool wave_err = c.err && c.err_wave;
+    uint32_t splits = dw && t128 < 160 && g.K >= 8 * gemm_bk(g.dtype) ? 16 : 1;
+    double tile_us = 0.0;
+    const uint32_t tile = gemm_wave_tile(g, &splits, &tile_us);
+    const bool wave_ok = plan_wave(g, tile, 0, splits, &wave);
+    if (wave_ok) wave.us = wave_us(g, wave_err ? fused : w, tile, splits) + (wave_err ? 0.0 : err);
+    if (dw && g.N <= 16 && plan_skinny(g, &skinny)) {
+        // from 64 MB of X on (below, the K-splitting kernel's one launch is ahead), or where the
+        // K-splitting kernel's 32-bit offsets in a slice do not reach
         const bool large = (uint64_t)g.M * g.K * (g.dtype == SKL_F16 ? 2 : 4) >= (64ull << 20);
-        if (plan_skinny(g, &q) && (!w || (large && std::fmax(wave_us, narrow_wave_us(g)) > 0.9 * skinny_us(g))))
-            return q;
-        if (w) return p;
+        if (!wave_ok || (large && std::fmax(wave.us, narrow_wave_us(g)) > 0.9 * skinny_us(g))) return skinny;
     }
-    if (g.N <= 16 && plan_wave(g, wave, wave_splits, &p)) return p;
-    if (plan_dma(g, &p, &dma_us)) {
-        const uint32_t tiles = (p.Mp / 256) * (p.Np / 256);
-        // A dW of few tiles against the K-splitting kernel, with the copies of padded
-        // operands and the optimiser's bytes: 832 x 2368 over 1640 rows takes two
-        // copies, the GEMM and a reduction, 41 us, against 25 in one launch; 2048 x 2048
-        // over 16384 rows 163 against 220.
-        if (dw && wave && !gemm_dma_tile_forced()) {
-            const double elems = (double)g.M * g.N;
-            dma_us += elems * 26.0 / 7.0e6 + (p.splits > 1 ? 3.0 + elems * 4.0 * p.splits / 4.5e6 : 0.0);
-            if (p.pad_a) dma_us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
-            if (p.pad_b) dma_us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
-            if (wave_us < 0.9 * dma_us && plan_wave(g, wave, wave_splits, &q)) return q;
-        }
-        // padded copies against the operands as stored on 128x128 tiles
-        if (!dw && !in_place && (p.pad_a || p.pad_b) && gemm_dma_rag_ok(g) && !gemm_dma_tile_forced()) {
-            double us = 8.0 + std::ceil(tiles / 256.0) * (p.Kp / 128) * 3.2;
-            if (p.pad_a) us += 2.0 + 4.0 * g.M * g.K / 4.0e6;
-            if (p.pad_b) us += 2.0 + 4.0 * g.N * g.K / 4.0e6;
-            if (1.1 * dma128_us(g) < us && plan_dma128(g, &q)) return q;
-        }
-        return p;
+    // at most 16 columns: any larger tile is >90% padding; at most 16 k with the error in the
+    // epilogue: the caller weighs it against the error kernel's own sum
+    if (wave_ok && (g.N <= 16 || (g.K <= 16 && wave_err))) return wave;
+    const bool dma128_ok = plan_dma128(g, &dma128);
+    if (dma128_ok) {
+        const bool in_epilogue = c.err_dma && !dma128.rag;
+        dma128.us = dma128_us(g, in_epilogue ? fused : w, dma128.rag) + (in_epilogue ? 0.0 : err);
     }
-    if (!in_place && !gemm_dma_tile_forced() && plan_dma128(g, &p)) {
-        const double us = p.rag ? 1.1 * dma128_us(g) : dma128_us(g);
-        if ((!wave || us < wave_us) && us < staged_us(g)) return p;
-    }
-    // grids that leave those tiles' GPU mostly idle: the K-splitting kernel
-    if (wave && wave_us < staged_us(g) && plan_wave(g, wave, wave_splits, &p)) return p;
-    return plan_staged(g);
+    const bool use128 = dma128_ok && (!wave_ok || dma128.us < wave.us);
+    if (!use128 && !wave_ok) return base;
+    const GemmPlan &best = use128 ? dma128 : wave;
+    return best.us < (dw && dma ? DW_DMA_MARGIN : ROUTE_MARGIN) * base.us ? best : base;
 }
 
 // A route as SOKLYN_GEMM_ROUTE writes it; unset, or a name it does not know: as planned.
@@ -1170,7 +1140,9 @@ int32_t skl_dense_forward(skl_ctx *ctx, const skl_dense_desc *b, const void *in,
     if (g.fwd.fuse_act)
         in_place = in_place || overlaps(in, in_sz, b->predrop, o_sz) || overlaps(in, in_sz, b->out, o_sz) ||
                    (use_dropout && overlaps(in, in_sz, b->mask, o_sz));
-    const GemmPlan plan = plan_gemm(g, ctx->route, in_place);
+    PlanCtx how{};
+    how.in_place = in_place;
+    const GemmPlan plan = plan_gemm(g, ctx->route, how);
     if ((r = ensure_ws(ctx, plan.bytes()))) return r;
     if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws)))) return r;
 
@@ -1328,36 +1300,6 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     g.B = next->w;
     g.splits = 1;
     g.op = Op::InputGrad;
-    const GemmPlan plan = plan_gemm(g, ctx->route);
-
-    // A next layer of at most 16 outputs: its GEMM would pad k to 128, so the
-    // error kernel forms s = next.d_prenorm . next.W^T itself, per element, from
-    // copies of the two operands padded to 16 columns (same operands as the
-    // GEMM: f16(d_prenorm) and the working W for fp16 blocks).  Up to 2M elements
-    // the K-splitting kernel's epilogue is ahead, one launch for two: next of 10,
-    // 64 x 128 fp32 8.0 -> 5.4 us, 1024 x 512 fp16 8.4 -> 5.3, 4096 x 512 11.9 -> 9.5;
-    // beyond, its many short tiles are not: 4096 x 2048 27 -> 35, 12345 x 512 23 -> 29.
-    const size_t esz = cur->dtype == SKL_F16 ? 2 : 4, cells = (size_t)batch * cur->outputs;
-    const bool small = plan.wave && cur->outputs % 4 == 0 && cells <= (size_t(1) << 21);
-    const Route route = ctx->route.kind;
-    if (next->outputs <= 16 && (route == Route::Planned ? !small : route == Route::Skinny)) {
-        uint32_t splits = 0;
-        if ((r = ensure_cols(ctx, cur, batch, 2, &splits))) return r;
-        const size_t a_bytes = ((size_t)batch * 16 * esz + 255) & ~(size_t)255;
-        if ((r = ensure_ws(ctx, a_bytes + (size_t)cur->outputs * 16 * esz))) return r;
-        char *a16 = reinterpret_cast<char *>(ctx->ws), *w16 = a16 + a_bytes;
-        a.sk_a = a16;
-        a.sk_w = w16;
-        if (err_skinny_ok(a, ctx->cols)) {
-            SKL_TRY(launch_skinny_operands(cur->dtype, next_dp, batch, next->w, cur->outputs, next->outputs, a16, w16,
-                                           ctx->stream));
-            SKL_TRY(launch_error_skinny(a, ctx->cols, splits, ctx->stream));
-            record_cols(ctx, cur, batch, splits);
-            return SKL_OK;
-        }
-        a.sk_a = a.sk_w = nullptr;
-    }
-
     ErrEpi &e = g.err;
     // an operand act' does not read aliases the mask (loaded anyway: cache hits)
     e.predrop = act_uses_output(cur->act) ? cur->predrop : cur->mask;
@@ -1381,6 +1323,7 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
     e.inv_m = 1.0f / (float)batch;
     // Layers that share their backward buffers: an epilogue that writes cur's error would
     // overwrite rows of next's that other tiles have yet to read; the sum goes first then.
+    const size_t esz = cur->dtype == SKL_F16 ? 2 : 4, cells = (size_t)batch * cur->outputs;
     auto over_next = [&](const void *p, size_t sz) {
         return overlaps(p, cells * sz, next_dp, (size_t)batch * next->outputs * esz) ||
                overlaps(p, cells * sz, next->w, (size_t)cur->outputs * next->outputs * esz);
@@ -1389,7 +1332,41 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
                         (cur->dtype == SKL_F16 && over_next(cur->d_prenorm_h, 2)) ||
                         (cur->norm != SKL_NORM_DISABLED &&
                          (over_next(cur->d_norm_w, 4) || over_next(cur->d_norm_b, 4)));
-    if (!shared && plan.dma && !plan.rag && hidden_err_fusable(e, batch, cur->outputs)) {
+    PlanCtx how{};
+    how.err = true;
+    how.err_norm = cur->norm != SKL_NORM_DISABLED;
+    how.err_dma = !shared && hidden_err_fusable(e, batch, cur->outputs);
+    how.err_wave = !shared && hidden_err_wave_ok(e, cur->outputs);
+    const GemmPlan plan = plan_gemm(g, ctx->route, how);
+
+    // A next layer of at most 16 outputs: the error kernel forms s = next.d_prenorm .
+    // next.W^T itself, per element, from copies of the two operands padded to 16 columns
+    // (same operands as the GEMM: f16(d_prenorm) and the working W for fp16 blocks), where
+    // the K-splitting kernel's epilogue is not ahead (up to 512K elements it always is, one
+    // launch for two): next of 10, 64 x 128 fp32 8.0 us, 5.4 there; 1024 x 512 fp16 8.4, 5.3;
+    // 44376 x 64 55, 18; but 2648 x 576 fp16 below 6 11.2, 12.5.
+    const Route route = ctx->route.kind;
+    const bool in_epilogue = how.err_wave && plan.wave &&
+                             (cells <= (size_t(1) << 19) || plan.us < ROUTE_MARGIN * err_skinny_us(g, how.err_norm));
+    if (next->outputs <= 16 && (route == Route::Planned ? !in_epilogue : route == Route::Skinny)) {
+        uint32_t splits = 0;
+        if ((r = ensure_cols(ctx, cur, batch, 2, &splits))) return r;
+        const size_t a_bytes = ((size_t)batch * 16 * esz + 255) & ~(size_t)255;
+        if ((r = ensure_ws(ctx, a_bytes + (size_t)cur->outputs * 16 * esz))) return r;
+        char *a16 = reinterpret_cast<char *>(ctx->ws), *w16 = a16 + a_bytes;
+        a.sk_a = a16;
+        a.sk_w = w16;
+        if (err_skinny_ok(a, ctx->cols)) {
+            SKL_TRY(launch_skinny_operands(cur->dtype, next_dp, batch, next->w, cur->outputs, next->outputs, a16, w16,
+                                           ctx->stream));
+            SKL_TRY(launch_error_skinny(a, ctx->cols, splits, ctx->stream));
+            record_cols(ctx, cur, batch, splits);
+            return SKL_OK;
+        }
+        a.sk_a = a.sk_w = nullptr;
+    }
+
+    if (how.err_dma && plan.dma && !plan.rag) {
         // One kernel, as the reference has it (backward.cu:59-102): the 256x256
         // GEMM's epilogue computes the error from the sum in its accumulators
         // and leaves the column sums of each 256-row tile for cur's backward.
@@ -1402,7 +1379,7 @@ static int32_t hidden_error_impl(skl_ctx *ctx, const skl_dense_desc *cur, const 
         record_cols(ctx, cur, batch, tiles_m);
         return SKL_OK;
     }
-    if (!shared && plan.wave && hidden_err_wave_ok(e, cur->outputs)) {
+    if (how.err_wave && plan.wave) {
         // the same on the K-splitting kernel's tiles
         const uint32_t tiles_m = (batch + plan.wave - 1) / plan.wave;
         if ((r = ensure_cols_splits(ctx, tiles_m, cur->outputs))) return r;
@@ -1683,7 +1660,9 @@ int32_t skl_dense_input_grad(skl_ctx *ctx, const skl_dense_desc *b, uint32_t bat
     const size_t esz = f16 ? 2 : 4, dx_sz = (size_t)batch * b->inputs * sizeof(float);
     const bool in_place = overlaps(dx, dx_sz, g.A, (size_t)batch * b->outputs * esz) ||
                           overlaps(dx, dx_sz, g.B, (size_t)b->inputs * b->outputs * esz);
-    const GemmPlan plan = plan_gemm(g, ctx->route, in_place);
+    PlanCtx how{};
+    how.in_place = in_place;
+    const GemmPlan plan = plan_gemm(g, ctx->route, how);
     if ((r = ensure_ws(ctx, plan.bytes()))) return r;
     if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws), false, nullptr, nullptr, f16 ? KEEP_A : 0)))
         return r;
@@ -1706,26 +1685,33 @@ int32_t skl_dense_input_grad(skl_ctx *ctx, const skl_dense_desc *b, uint32_t bat
 }
 
 // For tests on a machine without a GPU (not part of soklyn_hip.h): the kernel that the planner
-// gives a forward (op 0), input gradient (1) or dW (2) whose output is M x N over K, rows
-// without padding and buffers aligned, in SOKLYN_GEMM_ROUTE's words.  The text is the thread's
+// gives a forward (op 0), input gradient (1), dW (2) or hidden error of a layer without a norm
+// (3) whose output is M x N over K, rows without padding and buffers aligned, in
+// SOKLYN_GEMM_ROUTE's words.  The text is the thread's
 // own until its next call.
 const char *skl_diag_gemm_route(uint32_t dtype, uint32_t op, uint32_t M, uint32_t N, uint32_t K) {
     static thread_local char text[64];
     GemmLaunch g{};
     g.dtype = dtype;
-    g.op = op == 0 ? Op::Fwd : op == 1 ? Op::InputGrad : Op::DwOpt;
+    g.op = op == 0 ? Op::Fwd : op == 2 ? Op::DwOpt : Op::InputGrad;
     g.M = M;
     g.N = N;
     g.K = K;
     g.lda = op == 2 ? M : K;
-    g.ldb = op == 1 ? K : N;
+    g.ldb = op == 1 || op == 3 ? K : N;
     g.a_kcontig = op != 2;
-    g.b_kcontig = op == 1;
+    g.b_kcontig = op == 1 || op == 3;
     g.A = g.B = reinterpret_cast<const void *>(uintptr_t(256));   // looked at for its alignment only
     g.splits = 1;
     g.fwd.ldc = g.st.ldc = g.opt.ldc = N;
-    const GemmPlan p = plan_gemm(g, GemmRoute{});
-    const char *kind = p.skinny ? "skinny" : p.wave ? "wave" : !p.dma ? "staged" : p.Kp == K && p.Mp == M && p.Np == N && p.tile == 128 && op != 2 ? "dma128" : "dma";
+    g.fwd.fuse_act = 1;
+    PlanCtx how{};
+    how.err = op == 3;
+    how.err_dma = op == 3 && M % 256 == 0 && N % 256 == 0;
+    how.err_wave = op == 3 && N % 4 == 0;
+    const GemmPlan p = plan_gemm(g, GemmRoute{}, how);
+    const bool whole = p.Mp == M && p.Np == N && p.Kp == K;
+    const char *kind = p.skinny ? "skinny" : !p.dma ? "staged" : op != 2 && p.tile == 128 && whole ? "dma128" : "dma";
     if (p.wave)
         snprintf(text, sizeof(text), "wave:%u:%u:%u", p.wave, p.waves ? p.waves : gemm_wave_waves(g, p.wave), p.splits);
     else

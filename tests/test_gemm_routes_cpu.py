@@ -9,7 +9,7 @@ import pytest
 from soklyn_amd import abi
 
 F32, F16 = 0, 1
-FWD, DX, DW = 0, 1, 2
+FWD, DX, DW, HID = 0, 1, 2, 3
 
 
 @pytest.fixture(scope="module")
@@ -41,3 +41,22 @@ def test_narrow_dw_streams_large_inputs_of_odd_pitch(route, dtype, inputs, outpu
 @pytest.mark.parametrize("inputs,outputs,batch", [(2048, 10, 16384), (784, 10, 64), (512, 16, 1024), (1, 1, 1)])
 def test_narrow_dw_of_ordinary_sizes_takes_one_launch_or_few_slices(route, dtype, inputs, outputs, batch):
     assert route(dtype, DW, inputs, outputs, batch).startswith("wave")
+
+
+# calls that routes newer than direct-to-LDS tiles (padded copies) and register-staged ones run
+# slower, measured with each kernel forced (1.2-1.6x): output M x N over K
+@pytest.mark.parametrize("dtype,op,M,N,K,kernel", [
+    (F16, DW, 2304, 1984, 6741, "dma"), (F16, DW, 2560, 528, 13216, "dma"), (F16, DW, 3008, 3408, 6202, "staged"),
+    (F32, DW, 1024, 1024, 65536, "staged"), (F32, FWD, 936, 2496, 44, "staged"), (F32, DX, 3153, 512, 192, "staged"),
+    (F16, HID, 65536, 1024, 1000, "dma"), (F16, HID, 16384, 1024, 1000, "dma"), (F16, HID, 16469, 272, 55, "staged")])
+def test_calls_that_the_newer_routes_slow_down_keep_theirs(route, dtype, op, M, N, K, kernel):
+    assert route(dtype, op, M, N, K).split(":")[0] == kernel
+
+
+# ... and that they are ahead of by 1.5x and more
+@pytest.mark.parametrize("dtype,op,M,N,K,kernel", [
+    (F16, FWD, 16, 4096, 4096, "wave"), (F16, FWD, 512, 2048, 2048, "wave"), (F32, FWD, 500, 1531, 777, "wave"),
+    (F16, DW, 2048, 2048, 512, "wave"), (F16, DX, 2048, 1024, 1024, "wave"), (F16, HID, 512, 2048, 2048, "wave"),
+    (F16, FWD, 35940, 3072, 256, "dma128")])
+def test_calls_that_the_newer_routes_speed_up_take_them(route, dtype, op, M, N, K, kernel):
+    assert route(dtype, op, M, N, K).split(":")[0] == kernel
