@@ -66,14 +66,16 @@ struct GemmRoute {
     uint32_t tile, waves, splits;
 };
 
-// Scratch of kernels that hand partial results to the launch after them (a BatchNorm's
-// column statistics), one piece per stream the context has run on: forwards on two
-// streams of one context share nothing else, so they may overlap.
-constexpr int kStreamSlots = 8;
-constexpr size_t STREAM_SCRATCH_BYTES = size_t(4) << 20;
-struct StreamScratch {
-    hipStream_t stream;
+// Scratch of a BatchNorm's column statistics between its two launches, one piece per context,
+// made at the first call that wants it.  `done` is recorded by the launch that reads it; the
+// next call waits for it on its own stream, whichever that is, so a context whose stream is
+// changed between forwards, or destroyed after one, needs no other order between them.  (Only
+// this scratch is so ordered: other workspaces of a context belong to one call at a time.)
+constexpr size_t NORM_SCRATCH_BYTES = size_t(8) << 20;
+struct NormScratch {
     void *buf;
+    hipEvent_t done;
+    bool used;           // done has been recorded
 };
 
 struct skl_ctx {
@@ -93,7 +95,7 @@ struct skl_ctx {
     GemmRoute route;     // SOKLYN_GEMM_ROUTE at skl_ctx_create: the kernel every GEMM must take
     hipEvent_t gemm_start, gemm_stop;   // skl_ctx_time_next_gemm
     void *scratch;       // device address of this device's copy of `scratch` (below)
-    StreamScratch streams[kStreamSlots];
+    NormScratch norm;
 };
 
 // Scratch of the allocation-free entry point (skl_dense_error_from_sum_noalloc):
@@ -154,26 +156,32 @@ int32_t ensure_buf(skl_ctx *ctx, void **buf, size_t *have, size_t bytes) {
 
 int32_t ensure_ws(skl_ctx *ctx, size_t bytes) { return ensure_buf(ctx, &ctx->ws, &ctx->ws_bytes, bytes); }
 
-// The stream's scratch, or null where the caller has to do without: more bytes than a
-// piece holds, a ninth stream, no memory, or a stream under capture (a replayed graph may
-// overlap eager calls on its stream's context, so captured kernels use none).
-void *stream_scratch(skl_ctx *ctx, size_t bytes) {
-    if (bytes == 0 || bytes > STREAM_SCRATCH_BYTES) return nullptr;
+// The context's BatchNorm scratch, safe to write on its stream, or null where the caller has to
+// do without: more bytes than it holds, no memory, or a stream under capture (a replay may
+// overlap eager calls, and other replays, so captured kernels use none).
+float *norm_scratch(skl_ctx *ctx, size_t bytes) {
+    NormScratch &n = ctx->norm;
+    if (bytes == 0 || bytes > NORM_SCRATCH_BYTES) return nullptr;
+    auto without = [] {
+        (void)hipGetLastError();   // the caller goes on without
+        return nullptr;
+    };
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
-    for (StreamScratch &s : ctx->streams) {
-        if (s.buf && s.stream == ctx->stream) return s.buf;
-        if (!s.buf) {
-            if (hipMalloc(&s.buf, STREAM_SCRATCH_BYTES) != hipSuccess) {
-                (void)hipGetLastError();   // the caller goes on without
-                s.buf = nullptr;
-                return nullptr;
-            }
-            s.stream = ctx->stream;
-            return s.buf;
-        }
+    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess) return without();
+    if (cs != hipStreamCaptureStatusNone) return nullptr;
+    if (!n.buf) {
+        // another thread's capture in the global mode forbids this one's allocations
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return without();
+        hipError_t e = n.done ? hipSuccess : hipEventCreateWithFlags(&n.done, hipEventDisableTiming | hipEventDisableSystemFence);
+        if (e == hipSuccess) e = hipMalloc(&n.buf, NORM_SCRATCH_BYTES);
+        const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) n.buf = nullptr;
+        if (e != hipSuccess || back != hipSuccess) return without();
     }
-    return nullptr;
+    if (n.used && hipStreamWaitEvent(ctx->stream, n.done, 0) != hipSuccess) return without();
+    n.used = true;
+    return reinterpret_cast<float *>(n.buf);
 }
 
 // Device address of `scratch` on device `dev` (current), looked up once per device.
@@ -994,8 +1002,9 @@ int32_t skl_ctx_destroy(skl_ctx *ctx) {
     if (ctx->cols) note(hipFree(ctx->cols));
     for (PadCopy &c : ctx->pads)
         if (c.buf) note(hipFree(c.buf));
-    for (StreamScratch &s : ctx->streams)
-        if (s.buf) note(hipFree(s.buf));
+    if (ctx->norm.used) note(hipEventSynchronize(ctx->norm.done));   // on whichever stream it was
+    if (ctx->norm.buf) note(hipFree(ctx->norm.buf));
+    if (ctx->norm.done) note(hipEventDestroy(ctx->norm.done));
     note(hipStreamDestroy(ctx->own_stream));
     delete ctx;
     return first == hipSuccess ? SKL_OK : hip_status(first);
@@ -1166,10 +1175,8 @@ int32_t skl_dense_forward(skl_ctx *ctx, const skl_dense_desc *b, const void *in,
         a.out = b->out;
         a.mask = b->mask;
         a.norm_rstd = b->norm_rstd;
-        float *stats = nullptr;
-        if (a.norm == SKL_NORM_BATCH)
-            stats = reinterpret_cast<float *>(stream_scratch(ctx, norm_cols_scratch(a.m, a.n)));
-        SKL_TRY(launch_norm_act(a, stats, ctx->stream));
+        float *stats = a.norm == SKL_NORM_BATCH ? norm_scratch(ctx, norm_cols_scratch(a.m, a.n)) : nullptr;
+        SKL_TRY(launch_norm_act(a, stats, ctx->norm.done, ctx->stream));
     }
     return finish(ctx);
 }

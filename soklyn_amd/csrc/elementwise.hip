@@ -2,6 +2,8 @@
 // (gfx950, wave64): fill / cast, norm + activation + dropout, softmax, output
 // error, hidden error from a given sum, column reductions + vector optimiser,
 // split-K dW reduction + optimiser.
+#include <hip/hip_ext.h>
+
 #include "launch.h"
 #include "vec_opt.h"
 
@@ -512,23 +514,71 @@ template <typename T, int PER> __global__ void __launch_bounds__(256) norm_rows_
     }
 }
 
-// BatchNorm (forward.cu:74-126 with norm == 3), then act + dropout, in one launch: a
-// workgroup of 1024 threads per 16 columns, all batch rows.  LPR = 16 / VW lanes share a
-// row (4 elements each with VEC, one otherwise), so the workgroup takes RPW = 1024 / LPR
-// rows per step and thread t the rows t / LPR, + RPW, ...  HELD: the thread's (at most
-// PER) rows stay in registers, so prenorm is read once for the mean, the variance about
-// it and the outputs; longer batches read it again for each (from L2).  Each sum runs
-// over a thread's rows, then the wave's lanes of a column (butterfly), then the 16 waves
-// in order.  Bound: a row is one piece of a line in each of five tensors, ~4 clocks apiece
-// in the CU's address path whatever the piece's width (2048 x 1024 fp16: 20 us with 4, 8
-// or 16 columns per workgroup; 1565 us with one thread walking a column).  Taken for
-// short batches and where the two-launch form below has no scratch.
-template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024) norm_cols_kernel(RowNormArgs a) {
-    constexpr uint32_t CT = 16, VW = VEC ? 4 : 1, LPR = CT / VW, RPW = 1024 / LPR;
+// The outputs of VW elements of one BatchNorm row (forward.cu:74-126 with norm == 3, then act +
+// dropout), stored by put(tensor, index, values).
+template <typename T, uint32_t VW, class Put>
+__device__ __forceinline__ void norm_cols_row(const RowNormArgs &a, uint32_t r, uint32_t c0, const T (&v)[VW],
+                                              const float (&mean)[VW], const float (&rstd)[VW], const float (&g)[VW],
+                                              const float (&bias)[VW], float scale, Put put) {
+    T cen[VW], pre[VW], pd[VW], mk[VW], ot[VW];
+    const uint32_t rk = dropout_rowkey(r, a.seed + r * 7u);
+#pragma unroll
+    for (uint32_t e = 0; e < VW; ++e) {
+        const float d = to_f32(v[e]) - mean[e];
+        cen[e] = from_f32<T>(d);
+        pre[e] = from_f32<T>(fmaf(d * rstd[e], g[e], bias[e]));
+        const float act = activation<T>(a.act, to_f32(pre[e]), a.leaky);
+        pd[e] = ot[e] = from_f32<T>(act);
+        if (a.use_dropout) {
+            const bool keep = (uint64_t)dropout_bits((c0 + e) * kDropColMul, rk) >= a.keep_min;
+            mk[e] = keep ? from_f32<T>(scale) : (T)0;
+            ot[e] = keep ? from_f32<T>(act * scale) : (T)0;
+        }
+    }
+    const uint64_t idx = (uint64_t)r * a.n + c0;
+    put(a.centered, idx, cen);
+    put(a.preact, idx, pre);
+    put(a.predrop, idx, pd);
+    put(a.out, idx, ot);
+    if (a.use_dropout) put(a.mask, idx, mk);
+}
+
+// Loads and stores of a row's VW elements (4 with VEC, one otherwise).
+template <typename T, bool VEC> struct ColVec {
+    static constexpr uint32_t VW = VEC ? 4 : 1;
     typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
     typedef typename std::conditional<sizeof(T) == 2, u32x2_t, u32x4_t>::type G;   // 4 elements
-    constexpr bool HELD = PER > 0;
-    constexpr int UNR = HELD ? PER : 4;   // rows loaded before any is used
+    __device__ __forceinline__ static void load(const void *p, uint64_t i, T (&v)[VW]) {
+        if constexpr (VEC)
+            *reinterpret_cast<G *>(v) = *reinterpret_cast<const G *>(reinterpret_cast<const T *>(p) + i);
+        else
+            v[0] = ldv<T>(p, i);
+    }
+    __device__ __forceinline__ static void put(void *p, uint64_t i, const T (&v)[VW]) {
+        if constexpr (VEC)
+            *reinterpret_cast<G *>(reinterpret_cast<T *>(p) + i) = *reinterpret_cast<const G *>(v);
+        else
+            stv<T>(p, i, v[0]);
+    }
+    __device__ __forceinline__ static void put_nt(void *p, uint64_t i, const T (&v)[VW]) {
+        if constexpr (VEC)
+            __builtin_nontemporal_store(*reinterpret_cast<const G *>(v),
+                                        reinterpret_cast<G *>(reinterpret_cast<T *>(p) + i));
+        else
+            stv<T>(p, i, v[0]);
+    }
+};
+
+// BatchNorm of at most 512 rows, in one launch: a workgroup of 1024 threads per 16 columns,
+// the batch in registers.  LPR = 16 / VW lanes share a row, so the workgroup takes RPW =
+// 1024 / LPR rows per step and thread t the rows t / LPR, + RPW, ...  Each sum runs over a
+// thread's rows, then the wave's lanes of a column (butterfly), then the 16 waves in order.
+// Bound: a row is one piece of a line in each of five tensors, ~4 clocks apiece in the CU's
+// address path whatever the piece's width (~4 us + 8 ns per row; one thread walking a column
+// took 0.75 us per row).
+template <typename T, bool VEC> __global__ void __launch_bounds__(1024) norm_cols_kernel(RowNormArgs a) {
+    typedef ColVec<T, VEC> C;
+    constexpr uint32_t CT = 16, VW = C::VW, LPR = CT / VW, RPW = 1024 / LPR, PER = 512 / RPW;
     __shared__ float red[16][CT];
     // workgroup w runs on XCD w % 8: consecutive tiles go to one XCD
     uint32_t tile = blockIdx.x;
@@ -538,37 +588,15 @@ template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024)
     const uint32_t c0 = tile * CT + lr * VW;
     const bool cin = c0 < n;              // VEC: n % VW == 0, so whole groups
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    T zr[UNR][VW];
-
-    auto load = [&](uint32_t r, T (&v)[VW]) {
-        if constexpr (VEC)
-            *reinterpret_cast<G *>(v) =
-                *reinterpret_cast<const G *>(reinterpret_cast<const T *>(a.prenorm) + (uint64_t)r * n + c0);
-        else
-            v[0] = ldv<T>(a.prenorm, (uint64_t)r * n + c0);
-    };
+    T zr[PER][VW];
+#pragma unroll
+    for (uint32_t i = 0; i < PER; ++i)
+        if (cin && r0 + i * RPW < m) C::load(a.prenorm, (uint64_t)(r0 + i * RPW) * n + c0, zr[i]);
     // f(row, its VW elements) over the thread's rows
-    auto rows = [&](bool first, auto f) {
-        if constexpr (HELD) {
-            if (first) {
+    auto rows = [&](auto f) {
 #pragma unroll
-                for (int i = 0; i < UNR; ++i)
-                    if (cin && r0 + i * RPW < m) load(r0 + i * RPW, zr[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < UNR; ++i)
-                if (cin && r0 + i * RPW < m) f(r0 + i * RPW, zr[i]);
-        } else {
-            if (!cin) return;
-            for (uint32_t rb = r0; rb < m; rb += UNR * RPW) {
-#pragma unroll
-                for (int i = 0; i < UNR; ++i)
-                    if (rb + i * RPW < m) load(rb + i * RPW, zr[i]);
-#pragma unroll
-                for (int i = 0; i < UNR; ++i)
-                    if (rb + i * RPW < m) f(rb + i * RPW, zr[i]);
-            }
-        }
+        for (uint32_t i = 0; i < PER; ++i)
+            if (cin && r0 + i * RPW < m) f(r0 + i * RPW, zr[i]);
     };
     // sum of s over the column's threads; s becomes it in every one of them
     auto column_sum = [&](float (&s)[VW]) {
@@ -592,14 +620,14 @@ template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024)
     };
 
     float mean[VW] = {}, rstd[VW] = {};
-    rows(true, [&](uint32_t, const T (&v)[VW]) {
+    rows([&](uint32_t, const T (&v)[VW]) {
 #pragma unroll
         for (uint32_t e = 0; e < VW; ++e) mean[e] += to_f32(v[e]);
     });
     column_sum(mean);
 #pragma unroll
     for (uint32_t e = 0; e < VW; ++e) mean[e] /= (float)m;
-    rows(false, [&](uint32_t, const T (&v)[VW]) {
+    rows([&](uint32_t, const T (&v)[VW]) {
 #pragma unroll
         for (uint32_t e = 0; e < VW; ++e) {
             const float d = to_f32(v[e]) - mean[e];
@@ -617,35 +645,8 @@ template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024)
         bias[e] = to_f32(ldv<T>(a.norm_b, c0 + e));
     }
     const float scale = a.use_dropout ? 1.0f / (1.0f - a.p) : 1.0f;
-    rows(false, [&](uint32_t r, const T (&v)[VW]) {
-        T cen[VW], pre[VW], pd[VW], mk[VW], ot[VW];
-        const uint32_t rk = dropout_rowkey(r, a.seed + r * 7u);
-#pragma unroll
-        for (uint32_t e = 0; e < VW; ++e) {
-            const float d = to_f32(v[e]) - mean[e];
-            cen[e] = from_f32<T>(d);
-            pre[e] = from_f32<T>(fmaf(d * rstd[e], g[e], bias[e]));
-            const float act = activation<T>(a.act, to_f32(pre[e]), a.leaky);
-            pd[e] = ot[e] = from_f32<T>(act);
-            if (a.use_dropout) {
-                const bool keep = (uint64_t)dropout_bits((c0 + e) * kDropColMul, rk) >= a.keep_min;
-                mk[e] = keep ? from_f32<T>(scale) : (T)0;
-                ot[e] = keep ? from_f32<T>(act * scale) : (T)0;
-            }
-        }
-        const uint64_t idx = (uint64_t)r * n + c0;
-        auto put = [&](void *p, const T (&x)[VW]) {
-            if constexpr (VEC)
-                *reinterpret_cast<G *>(reinterpret_cast<T *>(p) + idx) = *reinterpret_cast<const G *>(x);
-            else
-                stv<T>(p, idx, x[0]);
-        };
-        put(a.centered, cen);
-        put(a.preact, pre);
-        put(a.predrop, pd);
-        put(a.out, ot);
-        if (a.use_dropout) put(a.mask, mk);
-    });
+    auto put = [](void *p, uint64_t at, const T (&v)[VW]) { C::put(p, at, v); };
+    rows([&](uint32_t r, const T (&v)[VW]) { norm_cols_row<T, VW>(a, r, c0, v, mean, rstd, g, bias, scale, put); });
 }
 
 // BatchNorm in two launches, for batches of more than a few hundred rows: rows are split
@@ -657,23 +658,14 @@ template <typename T, bool VEC, int PER> __global__ void __launch_bounds__(1024)
 //    64 rows.
 // 256 threads: LPR = 64 / VW lanes per row, RPS = 256 / LPR rows per step.
 // 2048 x 1024 fp16: 4.0 + 8.0 us, against 20 us in one launch.
-template <typename T, bool VEC> struct ColRows {
-    static constexpr uint32_t VW = VEC ? 4 : 1, LPR = 64 / VW, RPS = 256 / LPR;
-    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-    typedef typename std::conditional<sizeof(T) == 2, u32x2_t, u32x4_t>::type G;   // 4 elements
-    __device__ __forceinline__ static void load(const void *p, uint64_t i, T (&v)[VW]) {
-        if constexpr (VEC)
-            *reinterpret_cast<G *>(v) = *reinterpret_cast<const G *>(reinterpret_cast<const T *>(p) + i);
-        else
-            v[0] = ldv<T>(p, i);
-    }
-    __device__ __forceinline__ static void put(void *p, uint64_t i, const T (&v)[VW]) {
-        if constexpr (VEC)
-            __builtin_nontemporal_store(*reinterpret_cast<const G *>(v),
-                                        reinterpret_cast<G *>(reinterpret_cast<T *>(p) + i));
-        else
-            stv<T>(p, i, v[0]);
-    }
+// The row block of a (column tiles, row blocks) grid: y, and z beyond 65535 of them.
+constexpr uint32_t GRID_Y = 65535;
+__device__ __forceinline__ uint32_t rows_block() { return blockIdx.y + blockIdx.z * GRID_Y; }
+static dim3 rows_grid(uint32_t x, uint32_t blocks) {
+    return dim3(x, std::min(blocks, GRID_Y), (blocks + GRID_Y - 1) / GRID_Y);
+}
+template <typename T, bool VEC> struct ColRows : ColVec<T, VEC> {
+    static constexpr uint32_t LPR = 64 / ColVec<T, VEC>::VW, RPS = 256 / LPR;
 };
 
 template <typename T, bool VEC, int PER>
@@ -682,8 +674,10 @@ __global__ void __launch_bounds__(256) norm_cols_stats_kernel(RowNormArgs a, flo
     constexpr uint32_t VW = C::VW, LPR = C::LPR, RPS = C::RPS;
     __shared__ float red[RPS][64];
     const uint32_t n = a.n, lr = threadIdx.x % LPR, rr = threadIdx.x / LPR;
-    const uint32_t c0 = blockIdx.x * 64 + lr * VW;
-    const uint32_t r0 = blockIdx.y * (PER * RPS), cnt = min(a.m - r0, PER * RPS);
+    const uint32_t slice = rows_block(), c0 = blockIdx.x * 64 + lr * VW;
+    const uint32_t r0 = slice * (PER * RPS);
+    if (r0 >= a.m) return;
+    const uint32_t cnt = min(a.m - r0, PER * RPS);
     const bool cin = c0 < n;
     T z[PER][VW];
 #pragma unroll
@@ -723,7 +717,7 @@ __global__ void __launch_bounds__(256) norm_cols_stats_kernel(RowNormArgs a, flo
         }
     column_sum(m2);
     if (rr != 0 || !cin) return;
-    float *p = stats + (uint64_t)blockIdx.y * 2 * n + c0;
+    float *p = stats + (uint64_t)slice * 2 * n + c0;
 #pragma unroll
     for (uint32_t e = 0; e < VW; ++e) {
         p[e] = mean[e];
@@ -738,7 +732,8 @@ __global__ void __launch_bounds__(256) norm_cols_apply_kernel(RowNormArgs a, con
     constexpr uint32_t VW = C::VW, LPR = C::LPR, RPS = C::RPS;
     __shared__ float red[4][64], fin[2][64];
     const uint32_t n = a.n, m = a.m, lr = threadIdx.x % LPR, rr = threadIdx.x / LPR;
-    const uint32_t c0 = blockIdx.x * 64 + lr * VW, r0 = blockIdx.y * 64;
+    const uint32_t block = rows_block(), c0 = blockIdx.x * 64 + lr * VW, r0 = block * 64;
+    if (r0 >= m) return;
     const bool cin = c0 < n;
     constexpr int PER = 64 / RPS;
     T z[PER][VW];
@@ -785,7 +780,7 @@ __global__ void __launch_bounds__(256) norm_cols_apply_kernel(RowNormArgs a, con
             const float var = ((red[0][t] + red[1][t]) + (red[2][t] + red[3][t])) / (float)m + 1e-6f;
             fin[0][t] = mean;
             fin[1][t] = 1.0f / sqrtf(var);
-            if (in && blockIdx.y == 0) stv<T>(a.norm_rstd, c, from_f32<T>(fin[1][t]));
+            if (in && block == 0) stv<T>(a.norm_rstd, c, from_f32<T>(fin[1][t]));
         }
         __syncthreads();
     }
@@ -803,27 +798,8 @@ __global__ void __launch_bounds__(256) norm_cols_apply_kernel(RowNormArgs a, con
     for (int i = 0; i < PER; ++i) {
         const uint32_t r = r0 + rr + i * RPS;
         if (r >= m) break;
-        T cen[VW], pre[VW], pd[VW], mk[VW], ot[VW];
-        const uint32_t rk = dropout_rowkey(r, a.seed + r * 7u);
-#pragma unroll
-        for (uint32_t e = 0; e < VW; ++e) {
-            const float d = to_f32(z[i][e]) - mean[e];
-            cen[e] = from_f32<T>(d);
-            pre[e] = from_f32<T>(fmaf(d * rstd[e], g[e], bias[e]));
-            const float act = activation<T>(a.act, to_f32(pre[e]), a.leaky);
-            pd[e] = ot[e] = from_f32<T>(act);
-            if (a.use_dropout) {
-                const bool keep = (uint64_t)dropout_bits((c0 + e) * kDropColMul, rk) >= a.keep_min;
-                mk[e] = keep ? from_f32<T>(scale) : (T)0;
-                ot[e] = keep ? from_f32<T>(act * scale) : (T)0;
-            }
-        }
-        const uint64_t idx = (uint64_t)r * n + c0;
-        C::put(a.centered, idx, cen);
-        C::put(a.preact, idx, pre);
-        C::put(a.predrop, idx, pd);
-        C::put(a.out, idx, ot);
-        if (a.use_dropout) C::put(a.mask, idx, mk);
+        norm_cols_row<T, VW>(a, r, c0, z[i], mean, rstd, g, bias, scale,
+                             [](void *p, uint64_t at, const T (&v)[VW]) { C::put_nt(p, at, v); });
     }
 }
 
@@ -832,6 +808,141 @@ static bool a16p(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) 
 // Rows up to 256 x 16 elements run with the row in registers (16-byte chunks when
 // rows are 16-byte aligned, aligned 4-element groups when only the buffers are);
 // longer rows take the looping kernel.
+// The same in one launch without scratch, for calls that have none (a stream under capture,
+// more slices than the scratch holds): a workgroup per 16 columns, a wave per slice, 16
+// slices at a time.  Every sum is added in the order of the two launches, so the results are
+// theirs bit for bit.  A layer's forward with it, captured, over K 64: fp16 2048 x 1024 29 us
+// (17 eagerly), 16384 x 4096 440 (184); fp32 2048 x 1024 34 (22).
+template <typename T, bool VEC, int PER>
+__global__ void __launch_bounds__(1024) norm_cols_one_kernel(RowNormArgs a, uint32_t slices) {
+    typedef ColVec<T, VEC> C;
+    constexpr uint32_t CT = 16, VW = C::VW, LPR = CT / VW, RPS = 64 / LPR, SLICE = PER * RPS, KEPT = 512;
+    static_assert(RPS == ColRows<T, VEC>::RPS, "the rows of a step as in norm_cols_stats_kernel");
+    __shared__ float red[16][RPS][CT];             // a wave's column sums, by row of its step
+    __shared__ float st[2][KEPT][CT];              // mean and squares about it of the last KEPT slices
+    __shared__ float part[4][CT], fin[2][CT];
+    uint32_t tile = blockIdx.x;
+    if ((gridDim.x & 7u) == 0) tile = (tile & 7u) * (gridDim.x >> 3) + (tile >> 3);
+    const uint32_t n = a.n, m = a.m, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t lr = lane % LPR, rr = lane / LPR, c0 = tile * CT + lr * VW;
+    const bool cin = c0 < n;
+    auto column_sum = [&](float (&s)[VW]) {
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) red[wave][rr][lr * VW + e] = s[e];
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) {
+            float t = 0.0f;
+#pragma unroll
+            for (uint32_t w = 0; w < RPS; ++w) t += red[wave][w][lr * VW + e];
+            s[e] = t;
+        }
+    };
+    // st of slices k .. k + 15, slice k + wave by this wave (norm_cols_stats_kernel's sums; rows
+    // that 1024 threads cannot hold are read again for the squares, from cache)
+    auto sixteen = [&](uint32_t k) {
+        const uint32_t slice = k + wave, r0 = slice * SLICE, cnt = slice < slices ? min(m - r0, SLICE) : 0u;
+        constexpr int LD = PER < 8 ? PER : 8;   // loads in flight
+        T z[LD][VW];
+        // f(elements) over the slice's rows rr, rr + RPS, ... of this lane
+        auto rows = [&](bool first, auto f) {
+#pragma unroll 1
+            for (int i0 = 0; i0 < PER; i0 += LD) {
+                if (first || PER > LD) {
+#pragma unroll
+                    for (int i = 0; i < LD; ++i)
+                        if (cin && rr + (i0 + i) * RPS < cnt)
+                            C::load(a.prenorm, (uint64_t)(r0 + rr + (i0 + i) * RPS) * n + c0, z[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < LD; ++i)
+                    if (cin && rr + (i0 + i) * RPS < cnt) f(z[i]);
+            }
+        };
+        float mean[VW] = {}, m2[VW] = {};
+        rows(true, [&](const T (&v)[VW]) {
+#pragma unroll
+            for (uint32_t e = 0; e < VW; ++e) mean[e] += to_f32(v[e]);
+        });
+        column_sum(mean);
+#pragma unroll
+        for (uint32_t e = 0; e < VW; ++e) mean[e] /= (float)cnt;
+        rows(false, [&](const T (&v)[VW]) {
+#pragma unroll
+            for (uint32_t e = 0; e < VW; ++e) {
+                const float d = to_f32(v[e]) - mean[e];
+                m2[e] = fmaf(d, d, m2[e]);
+            }
+        });
+        column_sum(m2);
+        if (rr == 0) {
+#pragma unroll
+            for (uint32_t e = 0; e < VW; ++e) {
+                st[0][slice % KEPT][lr * VW + e] = mean[e];
+                st[1][slice % KEPT][lr * VW + e] = m2[e];
+            }
+        }
+        __syncthreads();
+    };
+    // thread (q, column) of the first wave merges slices q, q + 4, ... (norm_cols_apply_kernel's order)
+    const uint32_t q = threadIdx.x / CT, c = threadIdx.x % CT;
+    const bool merge = threadIdx.x < 4 * CT;
+    auto rows_of = [&](uint32_t s) { return (float)min(SLICE, m - s * SLICE); };
+    float s1 = 0.0f, s2 = 0.0f;
+    for (uint32_t k = 0; k < slices; k += 16) {
+        sixteen(k);
+        for (uint32_t s = k + q; merge && s < min(slices, k + 16); s += 4)
+            s1 = fmaf(rows_of(s), st[0][s % KEPT][c], s1);
+    }
+    if (merge) part[q][c] = s1;
+    __syncthreads();
+    const float total_mean = ((part[0][c] + part[1][c]) + (part[2][c] + part[3][c])) / (float)m;
+    auto square = [&](uint32_t s) {
+        const float d = st[0][s % KEPT][c] - total_mean;
+        s2 += fmaf(rows_of(s) * d, d, st[1][s % KEPT][c]);
+    };
+    if (slices <= KEPT) {
+        for (uint32_t s = q; merge && s < slices; s += 4) square(s);
+    } else {   // too many to keep: once more
+        for (uint32_t k = 0; k < slices; k += 16) {
+            sixteen(k);
+            for (uint32_t s = k + q; merge && s < min(slices, k + 16); s += 4) square(s);
+        }
+    }
+    __syncthreads();
+    if (merge) part[q][c] = s2;
+    __syncthreads();
+    if (threadIdx.x < CT) {
+        const float var = ((part[0][c] + part[1][c]) + (part[2][c] + part[3][c])) / (float)m + 1e-6f;
+        fin[0][c] = total_mean;
+        fin[1][c] = 1.0f / sqrtf(var);
+        if (tile * CT + c < n) stv<T>(a.norm_rstd, tile * CT + c, from_f32<T>(fin[1][c]));
+    }
+    __syncthreads();
+    if (!cin) return;
+    float mean[VW], rstd[VW], g[VW], bias[VW];
+#pragma unroll
+    for (uint32_t e = 0; e < VW; ++e) {
+        mean[e] = fin[0][lr * VW + e];
+        rstd[e] = fin[1][lr * VW + e];
+        g[e] = to_f32(ldv<T>(a.norm_w, c0 + e));
+        bias[e] = to_f32(ldv<T>(a.norm_b, c0 + e));
+    }
+    const float scale = a.use_dropout ? 1.0f / (1.0f - a.p) : 1.0f;
+    auto put = [](void *p, uint64_t at, const T (&v)[VW]) { C::put(p, at, v); };
+    constexpr uint32_t STEP = 16 * RPS, UNR = 4;   // rows of the workgroup's step; loads in flight
+    for (uint32_t rb = wave * RPS + rr; rb < m; rb += UNR * STEP) {
+        T z[UNR][VW];
+#pragma unroll
+        for (uint32_t i = 0; i < UNR; ++i)
+            if (rb + i * STEP < m) C::load(a.prenorm, (uint64_t)(rb + i * STEP) * n + c0, z[i]);
+#pragma unroll
+        for (uint32_t i = 0; i < UNR; ++i)
+            if (rb + i * STEP < m) norm_cols_row<T, VW>(a, rb + i * STEP, c0, z[i], mean, rstd, g, bias, scale, put);
+    }
+}
+
 template <typename T> static void launch_norm_rows(const RowNormArgs &a, hipStream_t s) {
     constexpr uint32_t VW = 16 / sizeof(T);
     const bool vec = a.n % VW == 0 && a16p(a.prenorm) && a16p(a.norm_w) && (a.norm != 2 || a16p(a.norm_b)) &&
@@ -869,9 +980,8 @@ template <typename T> static void launch_norm_rows(const RowNormArgs &a, hipStre
 }
 
 // BatchNorm.  4-element groups where every row of every tensor starts on one.  Batches
-// of more than 384 rows in two launches when there is scratch for their slices (the one
-// launch takes ~4 us + 8 ns per row, the two ~7 us and the bytes); otherwise in one, the
-// batch in registers where it fits.
+// of more than 384 rows by row slices, in two launches when there is scratch for them (one
+// launch takes ~4 us + 8 ns per row, the two ~7 us and the bytes), else in one.
 constexpr uint32_t COLS_TWO_MIN = 384;
 // Rows per slice: 64, or 256 where that would be more than 64 slices.
 static uint32_t norm_cols_per(uint32_t m) { return m <= 64 * 64 ? 64 : 256; }
@@ -881,52 +991,52 @@ size_t norm_cols_scratch(uint32_t m, uint32_t n) {
     return (size_t)cdiv(m, norm_cols_per(m)) * 2 * n * sizeof(float);
 }
 
-template <typename T> static void launch_norm_cols(const RowNormArgs &a, float *stats, hipStream_t s) {
-    constexpr uint32_t RPW_V = 256, RPW_1 = 64;   // rows per step
+template <typename T, bool VEC, int PER>
+static void launch_norm_slices(const RowNormArgs &a, float *stats, hipEvent_t done, hipStream_t s) {
+    const uint32_t per = norm_cols_per(a.m), slices = cdiv(a.m, per), gx = cdiv(a.n, 64);
+    if (!stats) {
+        hipLaunchKernelGGL((norm_cols_one_kernel<T, VEC, PER>), dim3(cdiv(a.n, 16)), dim3(1024), 0, s, a, slices);
+        return;
+    }
+    hipLaunchKernelGGL((norm_cols_stats_kernel<T, VEC, PER>), rows_grid(gx, slices), dim3(256), 0, s, a, stats);
+    // the event comes with the dispatch: no packet of its own between the kernels
+    hipExtLaunchKernelGGL((norm_cols_apply_kernel<T, VEC>), rows_grid(gx, cdiv(a.m, 64)), dim3(256), 0, s, nullptr, done,
+                          0, a, stats, slices, per);
+}
+
+template <typename T> static void launch_norm_cols(const RowNormArgs &a, float *stats, hipEvent_t done, hipStream_t s) {
     constexpr uintptr_t GB = 4 * sizeof(T) - 1;
     auto ga = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & GB) == 0; };
     const bool vec = a.n % 4 == 0 && ga(a.prenorm) && ga(a.centered) && ga(a.preact) && ga(a.predrop) && ga(a.out) &&
                      (!a.use_dropout || ga(a.mask));
-    if (stats && a.m > COLS_TWO_MIN) {
-        const uint32_t per = norm_cols_per(a.m), slices = cdiv(a.m, per);
-        const dim3 gs(cdiv(a.n, 64), slices), ga2(cdiv(a.n, 64), cdiv(a.m, 64)), b(256);
-        if (vec) {
-            if (per == 64)
-                hipLaunchKernelGGL((norm_cols_stats_kernel<T, true, 4>), gs, b, 0, s, a, stats);
-            else
-                hipLaunchKernelGGL((norm_cols_stats_kernel<T, true, 16>), gs, b, 0, s, a, stats);
-            hipLaunchKernelGGL((norm_cols_apply_kernel<T, true>), ga2, b, 0, s, a, stats, slices, per);
-        } else {
-            if (per == 64)
-                hipLaunchKernelGGL((norm_cols_stats_kernel<T, false, 16>), gs, b, 0, s, a, stats);
-            else
-                hipLaunchKernelGGL((norm_cols_stats_kernel<T, false, 64>), gs, b, 0, s, a, stats);
-            hipLaunchKernelGGL((norm_cols_apply_kernel<T, false>), ga2, b, 0, s, a, stats, slices, per);
-        }
-        return;
-    }
     const dim3 g(cdiv(a.n, 16)), b(1024);
-    if (vec && a.m <= 2 * RPW_V)
-        hipLaunchKernelGGL((norm_cols_kernel<T, true, 2>), g, b, 0, s, a);
-    else if (vec && a.m <= 8 * RPW_V)
-        hipLaunchKernelGGL((norm_cols_kernel<T, true, 8>), g, b, 0, s, a);
-    else if (vec)
-        hipLaunchKernelGGL((norm_cols_kernel<T, true, 0>), g, b, 0, s, a);
-    else if (a.m <= 8 * RPW_1)
-        hipLaunchKernelGGL((norm_cols_kernel<T, false, 8>), g, b, 0, s, a);
-    else
-        hipLaunchKernelGGL((norm_cols_kernel<T, false, 0>), g, b, 0, s, a);
+    if (a.m <= COLS_TWO_MIN) {
+        if (vec)
+            hipLaunchKernelGGL((norm_cols_kernel<T, true>), g, b, 0, s, a);
+        else
+            hipLaunchKernelGGL((norm_cols_kernel<T, false>), g, b, 0, s, a);
+    } else if (norm_cols_per(a.m) == 64) {
+        if (vec)
+            launch_norm_slices<T, true, 4>(a, stats, done, s);
+        else
+            launch_norm_slices<T, false, 16>(a, stats, done, s);
+    } else {
+        if (vec)
+            launch_norm_slices<T, true, 16>(a, stats, done, s);
+        else
+            launch_norm_slices<T, false, 64>(a, stats, done, s);
+    }
 }
 
-hipError_t launch_norm_act(const RowNormArgs &a0, float *stats, hipStream_t s) {
+hipError_t launch_norm_act(const RowNormArgs &a0, float *stats, hipEvent_t done, hipStream_t s) {
     if (a0.m == 0 || a0.n == 0) return hipSuccess;
     RowNormArgs a = a0;
     a.keep_min = dropout_keep_min(a.p);
     if (a.norm == 3) {
         if (a.dtype == 1)
-            launch_norm_cols<half_t>(a, stats, s);
+            launch_norm_cols<half_t>(a, stats, done, s);
         else
-            launch_norm_cols<float>(a, stats, s);
+            launch_norm_cols<float>(a, stats, done, s);
     } else if (a.dtype == 1) {
         launch_norm_rows<half_t>(a, s);
     } else {

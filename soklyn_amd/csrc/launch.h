@@ -164,9 +164,9 @@ struct RowNormArgs {
     uint64_t keep_min;   // set by launch_norm_act: dropout_keep_min(p)
 };
 // fwd1 + fwd2 fused (RMS / LN per row; BN per column then act).  stats: scratch of
-// norm_cols_scratch(m, n) bytes for a BatchNorm over a long batch, or null (then one,
-// slower launch needs none).
-hipError_t launch_norm_act(const RowNormArgs &a, float *stats, hipStream_t s);
+// norm_cols_scratch(m, n) bytes for a BatchNorm over a long batch, whose last reader records
+// `done`, or null (then one, slower launch with the same results needs none).
+hipError_t launch_norm_act(const RowNormArgs &a, float *stats, hipEvent_t done, hipStream_t s);
 size_t norm_cols_scratch(uint32_t m, uint32_t n);
 
 hipError_t launch_softmax(uint32_t dtype, void *out, uint32_t rows, uint32_t n, hipStream_t s);
