@@ -345,9 +345,8 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //    columns take it whatever the estimate, as any larger tile is mostly padding;
 //  * the streaming kernel for a dW of at most 16 columns over a large X whose rows the
 //    K-splitting kernel reads slowly or not at all;
-//  * the register-staged kernels (some large fp32; some fp16 with little k to reduce; an
-//    output over its own operand; operands past the others' 32-bit offsets), with split-K
-//    for small dW grids.
+//  * the register-staged kernels (some large fp32; some fp16 with little k to reduce;
+//    operands past the others' 32-bit offsets), with split-K for small dW grids.
 struct GemmPlan {
     uint32_t wave;             // K-splitting kernel: its tile edge (0: another kernel)
     uint32_t waves;            // ... and its waves per tile (0: the launcher's choice)
@@ -587,23 +586,21 @@ GemmPlan plan_staged(const GemmLaunch &g) {
 // What a GEMM's caller does with it beyond the op: the hidden error, whose routes differ in
 // whether the GEMM's epilogue may compute it.
 struct PlanCtx {
-    bool in_place;             // the output overlaps an operand
     bool err, err_norm;        // hidden error, of a layer with a norm
     bool err_dma, err_wave;    // ... in the epilogue of the direct-to-LDS / K-splitting kernel
 };
 
-GemmPlan plan_route(const GemmLaunch &g, const GemmRoute &route, const PlanCtx &c) {
+GemmPlan plan_route(const GemmLaunch &g, const GemmRoute &route) {
     GemmPlan p{};
     double us;
     bool ok = true;
     switch (route.kind) {
     case Route::Staged: p = plan_staged(g); break;
     case Route::Dma: ok = plan_dma(g, Work::Store, &p, &us); break;
-    case Route::Dma128: ok = !c.in_place && plan_dma128(g, &p); break;
+    case Route::Dma128: ok = plan_dma128(g, &p); break;
     case Route::Skinny: ok = plan_skinny(g, &p); break;
     default:
-        ok = !c.in_place && plan_wave(g, route.tile, route.waves,
-                                      g.op == Op::DwOpt && route.splits ? route.splits : 1, &p);
+        ok = plan_wave(g, route.tile, route.waves, g.op == Op::DwOpt && route.splits ? route.splits : 1, &p);
     }
     p.refused = !ok;
     return p;
@@ -611,10 +608,9 @@ GemmPlan plan_route(const GemmLaunch &g, const GemmRoute &route, const PlanCtx &
 
 // The earlier routes (direct-to-LDS where its grid fills the GPU, else register-staged; the
 // streaming dW) against 128x128 direct-to-LDS tiles and the K-splitting kernel, by
-// gemm_cost.h.  In place, the small tiles of the latter two would overwrite rows that others
-// have yet to read.
+// gemm_cost.h.
 GemmPlan plan_gemm(const GemmLaunch &g, const GemmRoute &route, const PlanCtx &c = PlanCtx{}) {
-    if (route.kind != Route::Planned) return plan_route(g, route, c);
+    if (route.kind != Route::Planned) return plan_route(g, route);
     const bool dw = g.op == Op::DwOpt;
     const Work fused = c.err_norm ? Work::ErrNorm : Work::Err;
     const Work w = dw ? Work::Dw : g.op == Op::Fwd ? Work::Fwd : Work::Store;
@@ -636,7 +632,6 @@ GemmPlan plan_gemm(const GemmLaunch &g, const GemmRoute &route, const PlanCtx &c
         base_us = staged_us(g, w, base.splits, small, vec) + err;
     }
     base.us = base_us;
-    if (c.in_place) return base;
     // a dW may go in batch slices where the register-staged kernels would split it too
     const bool wave_err = c.err && c.err_wave;
     uint32_t splits = dw && t128 < 160 && g.K >= 8 * gemm_bk(g.dtype) ? 16 : 1;
@@ -845,6 +840,35 @@ int32_t exec_gemm(skl_ctx *ctx, GemmLaunch g, const GemmPlan &p, char *ws, bool 
         if (vec_done) *vec_done = vec != nullptr;
     }
     return SKL_OK;
+}
+
+// An operand that the output overlaps (a caller's dx over d_prenorm, a layer fed its own output)
+// is read from a copy in the workspace: every tile writes columns of rows that the other
+// tiles of the row still read.
+struct OperandCopies {
+    size_t a, b;   // bytes, 0: read in place
+    size_t bytes() const { return a_at() + ((b + 255) & ~size_t(255)); }
+    size_t a_at() const { return (a + 255) & ~size_t(255); }
+};
+
+int32_t plan_and_exec(skl_ctx *ctx, GemmLaunch g, const OperandCopies &c, uint32_t keep) {
+    const void *A = g.A, *B = g.B;
+    // for the plan, the alignment of the workspace
+    if (c.a) g.A = reinterpret_cast<const void *>(uintptr_t(256));
+    if (c.b) g.B = reinterpret_cast<const void *>(uintptr_t(256));
+    const GemmPlan plan = plan_gemm(g, ctx->route);
+    int32_t r;
+    if ((r = ensure_ws(ctx, c.bytes() + plan.bytes()))) return r;
+    char *ws = reinterpret_cast<char *>(ctx->ws);
+    if (c.a) {
+        SKL_TRY(hipMemcpyAsync(ws, A, c.a, hipMemcpyDeviceToDevice, ctx->stream));
+        g.A = ws;
+    }
+    if (c.b) {
+        SKL_TRY(hipMemcpyAsync(ws + c.a_at(), B, c.b, hipMemcpyDeviceToDevice, ctx->stream));
+        g.B = ws + c.a_at();
+    }
+    return exec_gemm(ctx, g, plan, ws + c.bytes(), false, nullptr, nullptr, c.a ? keep & ~KEEP_A : keep);
 }
 
 // Common configuration checks of a block descriptor.
@@ -1141,19 +1165,13 @@ int32_t skl_dense_forward(skl_ctx *ctx, const skl_dense_desc *b, const void *in,
     g.fwd.leaky = b->act == SKL_ACT_LEAKY_RELU ? b->leaky : 0.0f;       // ffn_device.rs:32-35
     g.fwd.p = b->mask_coeff;
     g.fwd.ldc = b->outputs;
-    // the layer's own output as its input (up to one tile wide): a tile then reads its rows
-    // whole before it writes them, which the smaller tiles do not
     const size_t esz = b->dtype == SKL_F16 ? 2 : 4, in_sz = (size_t)batch * in_cols * esz;
     const size_t o_sz = (size_t)batch * b->outputs * esz;
-    bool in_place = overlaps(in, in_sz, g.fwd.z_out, o_sz);
+    bool over = overlaps(in, in_sz, g.fwd.z_out, o_sz);
     if (g.fwd.fuse_act)
-        in_place = in_place || overlaps(in, in_sz, b->predrop, o_sz) || overlaps(in, in_sz, b->out, o_sz) ||
-                   (use_dropout && overlaps(in, in_sz, b->mask, o_sz));
-    PlanCtx how{};
-    how.in_place = in_place;
-    const GemmPlan plan = plan_gemm(g, ctx->route, how);
-    if ((r = ensure_ws(ctx, plan.bytes()))) return r;
-    if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws)))) return r;
+        over = over || overlaps(in, in_sz, b->predrop, o_sz) || overlaps(in, in_sz, b->out, o_sz) ||
+               (use_dropout && overlaps(in, in_sz, b->mask, o_sz));
+    if ((r = plan_and_exec(ctx, g, OperandCopies{over ? in_sz : 0, 0}, 0))) return r;
 
     if (b->norm != SKL_NORM_DISABLED) {
         RowNormArgs a{};
@@ -1665,14 +1683,9 @@ int32_t skl_dense_input_grad(skl_ctx *ctx, const skl_dense_desc *b, uint32_t bat
     g.st.split_stride = 0;
     g.st.ldc = b->inputs;
     const size_t esz = f16 ? 2 : 4, dx_sz = (size_t)batch * b->inputs * sizeof(float);
-    const bool in_place = overlaps(dx, dx_sz, g.A, (size_t)batch * b->outputs * esz) ||
-                          overlaps(dx, dx_sz, g.B, (size_t)b->inputs * b->outputs * esz);
-    PlanCtx how{};
-    how.in_place = in_place;
-    const GemmPlan plan = plan_gemm(g, ctx->route, how);
-    if ((r = ensure_ws(ctx, plan.bytes()))) return r;
-    if ((r = exec_gemm(ctx, g, plan, reinterpret_cast<char *>(ctx->ws), false, nullptr, nullptr, f16 ? KEEP_A : 0)))
-        return r;
+    const size_t a_sz = (size_t)batch * b->outputs * esz, b_sz = (size_t)b->inputs * b->outputs * esz;
+    const OperandCopies copies{overlaps(dx, dx_sz, g.A, a_sz) ? a_sz : 0, overlaps(dx, dx_sz, g.B, b_sz) ? b_sz : 0};
+    if ((r = plan_and_exec(ctx, g, copies, f16 ? KEEP_A : 0))) return r;
     // dX reads d_prenorm (or its fp16 copy) and W and writes dx only: column sums
     // that the error call just before left stay valid for the backward after
     // this call (a single block's dX before its optimiser step), unless dx

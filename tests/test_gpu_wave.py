@@ -186,3 +186,37 @@ def test_forward_of_its_own_output(ctx, half, M, N):
     db.forward(db.out, M)
     torch.cuda.synchronize()
     check("out", db.get("out"), ob.out, FP16_TOL if half else FP32_TOL)
+
+
+# ... and of any width and number of rounds of tiles: a copy of the operand is read
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N", [(300, 520), (2100, 1030), (4096, 1024)])
+def test_forward_of_its_own_wide_output(ctx, half, M, N):
+    _, db = make_pair(ctx, N, N, M, seed=N, half=half, act=abi.ACT_SILU)
+    x = dev(inputs(114, M, N, half), half)
+    db.forward(x, M)
+    torch.cuda.synchronize()
+    want = db.out.clone()
+    db.out.copy_(x)
+    db.forward(db.out, M)
+    torch.cuda.synchronize()
+    check("out", db.get("out"), want.float().cpu().numpy(), FP16_TOL if half else FP32_TOL)
+
+
+# the input gradient over the fp32 operand it is computed from, and over half of it; over the fp16
+# copy that an fp16 block's reads
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,K,N", [(320, 200, 200), (300, 520, 520), (1000, 777, 1560), (4096, 1024, 1024)])
+def test_input_grad_over_its_operand(ctx, half, M, K, N):
+    _, db = make_pair(ctx, K, N, M, seed=K + N, half=half, act=abi.ACT_IDENTITY)
+    d = torch.from_numpy((rng(115).standard_normal((M, N)) * 512).astype(np.float32)).cuda()
+    db.d_prenorm.copy_(d)
+    name = "d_prenorm"
+    if half:
+        name = "d_prenorm_h"   # room for the fp32 output behind its rows
+        db.d_prenorm_h = torch.empty(2 * M * max(K, N), device="cuda", dtype=torch.float16)[:M * N].view(M, N)
+        db.d_prenorm_h.copy_(d)
+    want = db.input_grad(M).cpu().numpy()
+    out = torch.as_strided(getattr(db, name).view(torch.float32) if half else db.d_prenorm, (M, K), (K, 1))
+    got = db.input_grad(M, out=out).cpu().numpy()
+    check("dx", got, want, FP32_TOL)
