@@ -27,7 +27,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,K,N,norm,act,p", [
     (3001, 777, 4001, 0, abi.ACT_SILU, 0.2),      # padded A and B, fused act + dropout epilogue
     (3001, 777, 4001, 2, abi.ACT_LEAKY, 0.0),     # padded, prenorm epilogue then LayerNorm
-    (4096, 1000, 3072, 1, abi.ACT_MISH, 0.1),     # only A padded (K % 128), whole output tiles
+    (4096, 1000, 3072, 1, abi.ACT_MISH, 0.1),     # K not whole 128s: 128x128 tiles over A as stored
 ])
 def test_forward_padded(ctx, M, K, N, norm, act, p):
     print(f"forward padded {M}x{K}x{N} norm {norm}", flush=True)
@@ -122,7 +122,7 @@ def test_input_grad_row_band(ctx):
 
 @pytest.mark.parametrize("M,K,N,norm", [
     (6000, 1000, 1531, 2),   # 24 padded tiles: split-K over the batch, partial planes reduced
-    (2048, 2048, 2048, 0),   # 64 whole tiles, operands read in place: split-K only
+    (2048, 2048, 2048, 0),   # 64 whole tiles: the K-splitting kernel (split-K: tests/test_gpu_routes.py)
     (300, 4000, 3001, 1),    # 192 padded tiles, no split: Adam in the element-wise epilogue
     # split-K grids whose (tile, slice) count is not a multiple of 8 keep the tile order
     # (the others are remapped onto the XCDs): 49 tiles x 5 slices on 256x256 ...
@@ -152,7 +152,7 @@ def test_backward_padded_and_split(ctx, M, K, N, norm):
 @pytest.mark.parametrize("M,K,N", [(2048, 1024, 1024), (333, 200, 150)])
 def test_gemm_timing_hook(ctx, M, K, N):
     """skl_ctx_time_next_gemm: the next GEMM kernel's dispatch records the two events
-    (the 256x256 kernel, then the register-staged one); the call's results are unchanged."""
+    (tiles of 64x64, then of 16x16); the call's results are unchanged."""
     print(f"timing hook {M}x{K}x{N}", flush=True)
     ob, db = make_pair(ctx, K, N, M, seed=5, half=True, act=abi.ACT_SILU)
     x = inputs(6, M, K, True)

@@ -5,8 +5,9 @@ rounds d_prenorm to fp16 only for its dX (backward_wmma.cu:44) and sums its dW
 in fp32 from the fp32 d_prenorm (backward.cu:181-186), so where |d_prenorm| >
 65504 its dW stays finite while an fp16 copy of those values is infinite.  The
 device sums such elements again in fp32 from d_prenorm (in the optimiser
-epilogue of every dW path: the fused direct-to-LDS and register-staged kernels,
-the padded element-wise epilogue, the split-K reduction), so W, its master and
+epilogue of every dW path: the fused direct-to-LDS and K-splitting kernels, the
+padded element-wise epilogue, the split-K reduction; tests/test_gpu_routes.py runs
+the register-staged kernels and each K-splitting tile so), so W, its master and
 both moments must come out finite and match the oracle, whose dW is the
 reference's fp32 sum.  The dX of such a block is infinite on both sides (the
 reference rounds dX's operand to fp16 as well).
@@ -29,8 +30,8 @@ pytestmark = pytest.mark.gpu
     (512, 4096, 3072, "direct-to-LDS dW + Adam, whole tiles, no split-K"),
     (6000, 1000, 1531, "direct-to-LDS split-K partials on zero-padded operands + reduction"),
     (300, 4000, 3001, "zero-padded operands: element-wise Adam epilogue"),
-    (256, 128, 160, "register-staged dW + Adam"),
-    (4096, 512, 512, "register-staged split-K partials + reduction"),
+    (256, 128, 160, "K-splitting dW + Adam"),
+    (4096, 512, 512, "K-splitting partials in batch slices + reduction"),
 ])
 def test_dw_finite_where_d_prenorm_saturates_fp16(ctx, M, K, N, what):
     print(f"[case] {what}: M={M} K={K} N={N}", flush=True)

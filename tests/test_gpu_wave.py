@@ -1,8 +1,10 @@
-"""The K-splitting GEMM (16x16, 32x32 and 64x64 tiles, each wave its own k-tiles) through a
-layer's step, against the oracle: sizes around the edges of its tiles and k-tiles, fewer
-k-tiles than waves, widths that are odd (fp16 rows through registers), even but not whole
-16-byte chunks (the last chunk of a row masked), and large enough for each tile; outputs and
-inputs off a 16-byte boundary.  Gates as everywhere (tests/helpers.py)."""
+"""A layer's step at sizes whose GEMMs the planner gives mostly to the K-splitting kernel (16x16,
+32x32 and 64x64 tiles, each wave its own k-tiles), against the oracle: sizes around the edges
+of its tiles and k-tiles, fewer k-tiles than waves, widths that are odd (fp16 rows through
+registers), even but not whole 16-byte chunks (the last chunk of a row masked); outputs and
+inputs off a 16-byte boundary.  Which tile, or which other kernel, a size takes is the
+planner's choice; tests/test_gpu_routes.py runs each by name.  Gates as everywhere
+(tests/helpers.py)."""
 from __future__ import annotations
 
 import numpy as np
@@ -21,9 +23,9 @@ pytestmark = pytest.mark.gpu
 SHAPES = [  # batch, inputs, outputs
     (1, 1, 1), (2, 3, 5), (16, 64, 16), (17, 65, 33), (15, 63, 31), (64, 128, 64), (33, 130, 66), (5, 1000, 24),
     (70, 77, 200), (130, 36, 12), (20, 4100, 10), (257, 520, 136),
-    (700, 72, 900), (515, 330, 902), (701, 129, 835),      # 64x64 tiles
-    (1700, 40, 2000), (2500, 33, 2560), (2000, 1700, 40),  # fewer waves per tile
-    (3001, 200, 96), (4100, 61, 35), (5000, 130, 10), (2053, 40, 3),   # dW in batch slices
+    (700, 72, 900), (515, 330, 902), (701, 129, 835),      # several hundred tiles
+    (1700, 40, 2000), (2500, 33, 2560), (2000, 1700, 40),  # more than one round of them
+    (3001, 200, 96), (4100, 61, 35), (5000, 130, 10), (2053, 40, 3),   # long batches under few tiles of dW
 ]
 
 
@@ -139,8 +141,8 @@ def test_hidden_error(ctx, half, M, N0, N1, norm, act, p):
         check(name, d0.get(name), getattr(o0, name), tol)
 
 
-# the layer above of at most 16 outputs: in the epilogue up to 2M elements, in the error kernel
-# beyond and for widths that are not whole 4-column groups
+# the layer above of at most 16 outputs: in the epilogue of small layers, in the error kernel
+# of larger ones and for widths that are not whole 4-column groups
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("M,N0,N1,norm", [(1, 4, 1, abi.NORM_DISABLED), (64, 128, 10, abi.NORM_DISABLED),
                                           (300, 260, 3, abi.NORM_RMS), (1024, 512, 16, abi.NORM_LAYER),
