@@ -422,23 +422,7 @@ template <typename T> struct EpiErrK {
         // its rows; slot wave RPS + lane / CPL of the NW RPS partials per column
         constexpr uint32_t CPL = BN / 4, RPS = 64 / CPL, SLOTS = NW * RPS;
         const uint32_t lane = tid & 63u, wave = tid >> 6;
-        const uint32_t slot = wave * RPS + lane / CPL;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t c = 4u * (lane % CPL) + j;
-            lds[(slot * 3 + 0) * BN + c] = acc.dp[j];
-            lds[(slot * 3 + 1) * BN + c] = acc.nw[j];
-            lds[(slot * 3 + 2) * BN + c] = acc.nb[j];
-        }
-        __syncthreads();
-        for (uint32_t t = tid; t < 3 * BN; t += 64 * NW) {
-            const uint32_t k = t / BN, c = t % BN;
-            if ((k > 0 && !e.norm) || n0 + c >= e.ncols) continue;
-            float s = 0.0f;
-#pragma unroll
-            for (uint32_t w = 0; w < SLOTS; ++w) s += lds[(w * 3 + k) * BN + c];
-            e.partials[((uint64_t)tm * 3 + k) * e.ncols + n0 + c] = s;
-        }
+        flush_slots<SLOTS, BN, 64 * NW>(e, acc, lds, tid, wave * RPS + lane / CPL, lane % CPL, tm, n0);
     }
 };
 

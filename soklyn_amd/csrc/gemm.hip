@@ -112,8 +112,8 @@ uint32_t gemm_tiles(uint32_t dtype, uint32_t M, uint32_t N) {
 
 uint32_t gemm_bk(uint32_t dtype) { return dtype == 1 ? 64 : 32; }
 
-// The direct-to-LDS 256x256 kernel (gemm_dma.h).  SOKLYN_GEMM_DMA=0 selects
-// the register-staged kernels instead (A/B comparisons).
+// The direct-to-LDS kernel (gemm_dma.h).  SOKLYN_GEMM_DMA=0 leaves it out of the
+// planner's choice (A/B comparisons).
 bool gemm_dma_enabled() {
     static bool on = [] {
         const char *e = getenv("SOKLYN_GEMM_DMA");
