@@ -805,11 +805,8 @@ __global__ void __launch_bounds__(256) norm_cols_apply_kernel(RowNormArgs a, con
 
 static bool a16p(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Rows up to 256 x 16 elements run with the row in registers (16-byte chunks when
-// rows are 16-byte aligned, aligned 4-element groups when only the buffers are);
-// longer rows take the looping kernel.
-// The same in one launch without scratch, for calls that have none (a stream under capture,
-// more slices than the scratch holds): a workgroup per 16 columns, a wave per slice, 16
+// The statistics by slices and the outputs in one launch without scratch, for calls that have
+// none (a stream under capture, more slices than the scratch holds): a workgroup per 16 columns, a wave per slice, 16
 // slices at a time.  Every sum is added in the order of the two launches, so the results are
 // theirs bit for bit.  A layer's forward with it, captured, over K 64: fp16 2048 x 1024 29 us
 // (17 eagerly), 16384 x 4096 440 (184); fp32 2048 x 1024 34 (22).
@@ -943,6 +940,9 @@ __global__ void __launch_bounds__(1024) norm_cols_one_kernel(RowNormArgs a, uint
     }
 }
 
+// Rows up to 256 x 16 elements run with the row in registers (16-byte chunks when
+// rows are 16-byte aligned, aligned 4-element groups when only the buffers are);
+// longer rows take the looping kernel.
 template <typename T> static void launch_norm_rows(const RowNormArgs &a, hipStream_t s) {
     constexpr uint32_t VW = 16 / sizeof(T);
     const bool vec = a.n % VW == 0 && a16p(a.prenorm) && a16p(a.norm_w) && (a.norm != 2 || a16p(a.norm_b)) &&

@@ -158,7 +158,8 @@ bool gemm_wave_ok(const GemmLaunch &g, uint32_t splits) {
     return layout && span(g.a_kcontig, g.lda) < (1ull << 31) && span(g.b_kcontig, g.ldb) < (1ull << 31);
 }
 
-// Estimated time (us) of the three tiles, the larger of two lines fitted to measurements of
+// The choice among the three tiles (gemm_cost.h weighs the chosen one against other kernels):
+// the least of their estimated times (us), the larger of two lines fitted to measurements of
 // 100 shapes between 16 x 16 x 64 and 16384 x 4096 x 4096 (each within ~20%): what one
 // workgroup takes (the latency of its k-tiles, kt of 128 bytes), and the GPU's rate over
 // units of 256 workgroups (one per CU; a CU with one more of the first few than others
